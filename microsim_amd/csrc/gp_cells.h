@@ -7,12 +7,14 @@
  * it reads is Mpure[b], and its update is the pure-phase arithmetic of phase b. Every other interior cell is an
  * interface cell.
  *
- * k_cbulk updates the bulk cells of a tile (60-cell y-strip x seg_len x-rows, one wavefront, as the march tiles):
- * it streams the mu rows with a deep prefetch and forms, per lane, the same operations in the same order as the
- * pure-phase step and k_bulk, so the results are bit-identical. A tile whose staged codes are all one phase takes
- * that phase as a scalar and skips the per-cell classification. phi of a bulk cell is e_b; when the output buffer
- * already holds e_b there (the cell was purely b two states back) it is not rewritten.
- * k_cbulk also lists the interface cells of its tile (LDS, then one atomic per wavefront into a global list);
+ * k_cbulk updates the bulk cells of a tile (124-cell y-strip x SEG x-rows, one wavefront, two adjacent cells per
+ * lane): it streams the mu rows through a ring of registers and forms, per cell, the same operations in the same order
+ * as the pure-phase step and k_bulk, so the results are bit-identical. A tile whose staged codes are all one phase
+ * takes that phase as a scalar. The other tiles classify their cells with one bit per row in each lane and run
+ * the row loop once per phase that has bulk cells. phi of a bulk cell is e_b; when the output buffer already holds e_b
+ * there (the cell was purely b two states back) it is not rewritten.
+ * k_cbulk also appends the interface cells and the delta-phi candidates of its tile to two global lists (one atomic
+ * per mixed tile);
  * k_ilist runs the general per-cell update (gp_model.h: jat_x, jat_y, mu_update -- bit-identical to the
  * reference by construction) on the listed cells in a grid-stride loop, so that every lane of every wavefront
  * works on an interface cell (a march row has about one in five) and no wavefront holds more than its share.
@@ -25,228 +27,87 @@
 
 namespace gpk {
 
-#ifndef GP_CELL_SEG_MAX
-#define GP_CELL_SEG_MAX 16
-#endif
-constexpr int kCellSegMax = GP_CELL_SEG_MAX;   /* longest x-segment the kernels stage (LDS sized for it) */
-constexpr int kCellRows = kCellSegMax + 4;     /* staged code rows per tile */
-
-/* b when the radius-2 diamond of lane l at staged row r is purely phase b, else -1 (l in 2..61) */
-__device__ __forceinline__ int bulk_of(const int8_t *cs, int r, int l) {
-  const int b = cs[r * 64 + l];
-  if (b < 0) return -1;
-  const bool ok = cs[(r - 1) * 64 + l] == b && cs[(r + 1) * 64 + l] == b && cs[(r - 2) * 64 + l] == b &&
-                  cs[(r + 2) * 64 + l] == b && cs[r * 64 + l - 1] == b && cs[r * 64 + l + 1] == b &&
-                  cs[r * 64 + l - 2] == b && cs[r * 64 + l + 2] == b && cs[(r - 1) * 64 + l - 1] == b &&
-                  cs[(r - 1) * 64 + l + 1] == b && cs[(r + 1) * 64 + l - 1] == b && cs[(r + 1) * 64 + l + 1] == b;
-  return ok ? b : -1;
-}
-
-/* per-wavefront tile geometry, shared by the two kernels */
-struct CellTile {
-  int64_t y, yl, xa, xb;
-  bool out_lane;
-  __device__ CellTile(int w, int lane, int64_t mx, int64_t my, int seg_len, int nstrips) {
-    const int strip = w % nstrips, seg = w / nstrips;
-    const int64_t ry = my + 6;
-    y = 3 + (int64_t)strip * kMarchOut - 2 + lane;
-    yl = y < ry - 1 ? y : ry - 1;
-    xa = 3 + (int64_t)seg * seg_len;
-    xb = (xa + seg_len - 1 < mx + 2) ? xa + seg_len - 1 : mx + 2;
-    out_lane = lane >= 2 && lane <= 61 && y <= my + 2;
-  }
-};
+constexpr int kCellOut = 124;  /* output cells of a k_cbulk strip: 64 lanes x 2 cells less two on either side */
+constexpr int kCellSegMax = 16; /* longest x-segment of k_cbulk (instantiated for 16 and kCellSegMin rows) */
+constexpr int kCellSegMin = 4;
+/* Tiles from which k_cbulk takes the long segments: about one wavefront per SIMD. Below it the rows of a tile in turn are
+ * the step's critical path (1024^2 FP64, 576 long tiles: 39 us long, 28 us short); above it the short segments' doubled
+ * prologue costs more than it hides (2047 x 1801 FP32, 1920 long tiles: 33 us long, 45 us short). */
+constexpr int kCellFill = 1024;
+constexpr int kPadOut = 60, kPadSeg = 16; /* tiles of the statistics' padding rows (pad_stats) */
 
 /* a wave-uniform value read as a scalar: a per-lane choice among such values then stays a register select */
 __device__ __forceinline__ float scalar_val(float v) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __forceinline__ double scalar_val(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffll));
-  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 /* FP32 bulk cells take the closed form through Model::Kbulk; FP64 keeps the reference's operations (bit-exact) */
 template <typename R>
 constexpr bool kLeanBulk = sizeof(R) < sizeof(double);
 
-/* the bulk update of one cell in phase b. UNIFORM: b is the same on every lane (a scalar); every lane computes,
- * only lanes with `store` write, the mu statistics take every lane (the caller resets the lanes without a cell
- * once per tile) and the phi extrema (e_b on every cell) are left to the caller, once per tile. Otherwise the
- * caller calls it on the bulk lanes only, and it folds the full statistics. */
-template <int N, int NC, typename R, bool P2, bool STATS, bool UNIFORM, int NSA, bool C = false>
-__device__ __forceinline__ void cbulk_cell(const Model<R> &m, int b, int64_t c, const R *m0,
-                                           const R *m1, const R *m2, const R *mud, const R *muu, R divjat0,
-                                           R *__restrict__ phi_o, R *__restrict__ mu_o,
-                                           int8_t *__restrict__ codes_out, int64_t fs, bool kept, bool store,
-                                           bool live, R (&st)[NSA], unsigned &seen,
-                                           const int8_t *q1 = nullptr, float *__restrict__ plo_o = nullptr,
-                                           int8_t *__restrict__ mlo_o = nullptr) {
-  using Vw = View<R, P2, false, kFastOf<R>>;
-  R pe[N];
+/* The pure-phase update of one cell from mu of the cell, m1, and of its neighbours m0 (x-1), m2 (x+1), muu (y-1) and
+ * mud (y+1): the new mu and its increment.
+ * FP32: the closed form dmu = K . lap(mu), K = Kbulk of the cell's phase (equal in exact arithmetic to the flux
+ * divergence through Mpure followed by Mu_lin; the anti-trapping divergence is a signed zero). The second differences
+ * are formed from first differences, so their rounding is relative to the increment, as in the flux form. */
+template <int NC>
+__device__ __forceinline__ void bulk_update_lean(const Model<float> &m, const float (*K)[NC], const float *m0,
+                                                 const float *m1, const float *m2, const float *mud, const float *muu,
+                                                 float *munew, float *deltamu) {
+  float lap[NC];
 #pragma unroll
-  for (int a = 0; a < N; a++) pe[a] = a == b ? R(1.0) : R(0.0);
-  R deltamu[NC], munew[NC];
-  if constexpr (kLeanBulk<R>) {
-    /* FP32: the pure-phase update in closed form, dmu = Kbulk[b] . lap(mu) (equal in exact arithmetic to the
-     * flux divergence through Mpure[b] followed by Mu_lin; divjat0 is a signed zero). The second differences
-     * are formed from first differences, so their rounding is relative to the increment, as in the flux form. */
-    R lap[NC];
-#pragma unroll
-    for (int l = 0; l < NC; l++) {
-      const R gx = (m2[l] - m1[l]) - (m1[l] - m0[l]);
-      const R gy = (mud[l] - m1[l]) - (m1[l] - muu[l]);
-      lap[l] = __builtin_fmaf(gx, m.lap_x, gy * m.lap_y);
-    }
-#pragma unroll
-    for (int k = 0; k < NC; k++) {
-      R s = R(0.0);
-#pragma unroll
-      for (int l = 0; l < NC; l++) {
-        R kk;
-        if (UNIFORM) {
-          kk = m.Kbulk[b][k][l];
-        } else {
-          /* per-lane phase: pick among the phases' scalar values (kept scalar, so that the choice is a register
-           * select and not a per-lane load issued just before its use) */
-          kk = scalar_val(m.Kbulk[0][k][l]);
-#pragma unroll
-          for (int a = 1; a < N; a++)
-            if (b == a) kk = scalar_val(m.Kbulk[a][k][l]);
-        }
-        s = l == 0 ? kk * lap[0] : __builtin_fmaf(kk, lap[l], s);
-      }
-      deltamu[k] = s;
-      munew[k] = m1[k] + s;
-    }
-  } else {
-  R Mb[NC][NC];
-#pragma unroll
-  for (int k = 0; k < NC; k++)
-#pragma unroll
-    for (int l = 0; l < NC; l++) {
-      if (UNIFORM) {
-        Mb[k][l] = m.Mpure[b][k][l];
-      } else {
-        Mb[k][l] = scalar_val(m.Mpure[0][k][l]);
-#pragma unroll
-        for (int a = 1; a < N; a++)
-          if (b == a) Mb[k][l] = scalar_val(m.Mpure[a][k][l]);
-      }
-    }
-  R divflux[NC];
+  for (int l = 0; l < NC; l++) {
+    const float gx = (m2[l] - m1[l]) - (m1[l] - m0[l]);
+    const float gy = (mud[l] - m1[l]) - (m1[l] - muu[l]);
+    lap[l] = __builtin_fmaf(gx, m.lap_x, gy * m.lap_y);
+  }
 #pragma unroll
   for (int k = 0; k < NC; k++) {
-    divflux[k] = R(0.0);
+    float s = K[k][0] * lap[0];
+#pragma unroll
+    for (int l = 1; l < NC; l++) s = __builtin_fmaf(K[k][l], lap[l], s);
+    deltamu[k] = s;
+    munew[k] = m1[k] + s;
+  }
+}
+/* FP64: the reference's operations, phase b wave-uniform (its coefficients are scalars) */
+template <int N, int NC, typename R, bool P2>
+__device__ __forceinline__ void bulk_update_ref(const Model<R> &m, int b, const R *m0, const R *m1, const R *m2,
+                                                const R *mud, const R *muu, R divjat0, R *munew, R *deltamu) {
+  using Vw = View<R, P2, false, kFastOf<R>>;
+  R c_new[NC];
+#pragma unroll
+  for (int k = 0; k < NC; k++) {
+    R divflux = R(0.0);
 #pragma unroll
     for (int l = 0; l < NC; l++) {
-      const R Fb = Mb[k][l] * divx<Vw>(m, (m1[l] - m0[l]));
-      const R Ff = Mb[k][l] * divx<Vw>(m, (m2[l] - m1[l]));
-      const R Fy = Mb[k][l] * divy<Vw>(m, (mud[l] - m1[l]));
-      const R Fyl = Mb[k][l] * divy<Vw>(m, (m1[l] - muu[l])); /* = Fy of the lane below, bit for bit */
-      divflux[k] += divx<Vw>(m, (Ff - Fb));
-      divflux[k] += divy<Vw>(m, (Fy - Fyl));
+      const R Mb = m.Mpure[b][k][l];
+      const R Fb = Mb * divx<Vw>(m, (m1[l] - m0[l]));
+      const R Ff = Mb * divx<Vw>(m, (m2[l] - m1[l]));
+      const R Fy = Mb * divy<Vw>(m, (mud[l] - m1[l]));
+      const R Fyl = Mb * divy<Vw>(m, (m1[l] - muu[l])); /* = Fy of the cell below, bit for bit */
+      divflux += divx<Vw>(m, (Ff - Fb));
+      divflux += divy<Vw>(m, (Fy - Fyl));
     }
+    c_new[k] = c_mu<NC>(m, m1, b, k) + m.dt * (divflux)-divjat0;
   }
-  if (kDirectBulkMu<R>) {
-    R dc[NC];
 #pragma unroll
-    for (int k = 0; k < NC; k++) dc[k] = m.dt * (divflux[k]) - divjat0;
-#pragma unroll
-    for (int k = 0; k < NC; k++) {
-      R s = R(0);
-      if (UNIFORM) {
-        s = Mu_lin<NC>(m, dc, b, k);
-      } else {
-#pragma unroll
-        for (int a = 0; a < N; a++)
-          if (a == b) s = Mu_lin<NC>(m, dc, a, k);
-      }
-      deltamu[k] = s;
-      munew[k] = m1[k] + deltamu[k];
-    }
-  } else {
-    R c_new[NC];
-#pragma unroll
-    for (int k = 0; k < NC; k++) {
-      R s = R(0);
-      if (UNIFORM) {
-        s = c_mu<NC>(m, m1, b, k);
-      } else {
-#pragma unroll
-        for (int a = 0; a < N; a++)
-          if (a == b) s = c_mu<NC>(m, m1, a, k);
-      }
-      c_new[k] = s + m.dt * (divflux[k]) - divjat0;
-    }
-#pragma unroll
-    for (int k = 0; k < NC; k++) {
-      R s = R(0);
-      if (UNIFORM) {
-        s = Mu<NC>(m, c_new, b, k);
-      } else {
-#pragma unroll
-        for (int a = 0; a < N; a++)
-          if (a == b) s = Mu<NC>(m, c_new, a, k);
-      }
-      munew[k] = s;
-      deltamu[k] = munew[k] - m1[k];
-    }
+  for (int k = 0; k < NC; k++) {
+    munew[k] = Mu<NC>(m, c_new, b, k);
+    deltamu[k] = munew[k] - m1[k];
   }
-  }
-  int8_t qn[NC];
-  if constexpr (C) {
-    /* compensated mode: the increment is added to the decoded value (hi plus its extension) and the sum is
-     * re-encoded, so the bits of the increment below the FP32 part are kept */
+}
+
+/* the mu statistics of one bulk cell: delta-phi is 0 and phi = e_b, so the squared increments of phi add +0 to sums
+ * that start at +0 and e_b is finite; the extrema of phi follow from the phases seen (bulk_seen_fold) */
+template <int N, int NC, typename R, int NSA>
+__device__ __forceinline__ void bulk_stats(R (&st)[NSA], const R *munew, const R *deltamu) {
 #pragma unroll
-    for (int k = 0; k < NC; k++) {
-      float hn;
-      c32_encode(c32_decode((float)m1[k], q1[k]) + (double)deltamu[k], hn, qn[k]);
-      munew[k] = (R)hn;
-    }
-  }
-  if (store) {
-    const int8_t code = (int8_t)b;
-    /* kept: the output buffers hold the state before the current one and its codes; a cell that was purely
-     * phase b there already holds phi = e_b, so only mu is written */
-    if (!kept) {
-#pragma unroll
-      for (int a = 0; a < N; a++) phi_o[a * fs + c] = pe[a];
-      if constexpr (C) {
-#pragma unroll
-        for (int a = 0; a < N; a++) plo_o[a * fs + c] = 0.0f;
-      }
-      codes_out[c] = code;
-    }
-#pragma unroll
-    for (int k = 0; k < NC; k++) mu_o[k * fs + c] = munew[k];
-    if constexpr (C) {
-#pragma unroll
-      for (int k = 0; k < NC; k++) mlo_o[k * fs + c] = qn[k];
-    }
-  }
-  if (STATS && UNIFORM && live) {
-#pragma unroll
-    for (int k = 0; k < NC; k++) {
-      st[2 * N + k] = fmax(st[2 * N + k], munew[k]);
-      st[2 * N + NC + k] = fmin(st[2 * N + NC + k], munew[k]);
-      st[3 * N + 2 * NC + k] += deltamu[k] * deltamu[k];
-      if (!isfinite(munew[k])) st[NSA - 1] += R(1.0);
-    }
-  } else if (STATS) {
-    /* stats_add with delta-phi = 0 and phi = e_b: the squared increments of phi add +0 to sums that start at +0
-     * and e_b is finite, so only the extrema of phi and the mu terms remain; the extrema of phi over cells that are
-     * each some e_b follow from the set of phases seen (folded once, bulk_seen_fold) */
-    seen |= 1u << b;
-#pragma unroll
-    for (int k = 0; k < NC; k++) {
-      st[2 * N + k] = fmax(st[2 * N + k], munew[k]);
-      st[2 * N + NC + k] = fmin(st[2 * N + NC + k], munew[k]);
-      st[3 * N + 2 * NC + k] += deltamu[k] * deltamu[k];
-      if (!isfinite(munew[k])) st[NSA - 1] += R(1.0);
-    }
+  for (int k = 0; k < NC; k++) {
+    st[2 * N + k] = fmax(st[2 * N + k], munew[k]);
+    st[2 * N + NC + k] = fmin(st[2 * N + NC + k], munew[k]);
+    st[3 * N + 2 * NC + k] += deltamu[k] * deltamu[k];
+    if (!isfinite(munew[k])) st[NSA - 1] += R(1.0);
   }
 }
 
@@ -264,262 +125,475 @@ __device__ __forceinline__ void bulk_seen_fold(R (&st)[NSA], unsigned seen) {
   }
 }
 
-/* mu rows in flight ahead of the row after the current one, per precision (register budget: FP64 rows take twice
- * the registers); kCellRing = depth + 2 register slots hold rows x-1, x, x+1 and those in flight, and divides the
- * tile's 16 rows */
-#ifndef GP_CELL_DEPTH_F32
-#define GP_CELL_DEPTH_F32 2
-#endif
-#ifndef GP_CELL_DEPTH_F64
-#define GP_CELL_DEPTH_F64 2
-#endif
-template <typename R>
-constexpr int kCellBulkDepth = sizeof(R) == 8 ? GP_CELL_DEPTH_F64 : GP_CELL_DEPTH_F32;
-template <typename R>
-constexpr int kCellRing = kCellBulkDepth<R> + 2;
+/* mu rows in flight ahead of the row after the current one; kCellRing = depth + 2 register slots hold rows x-1, x,
+ * x+1 and those in flight, and divides the tile's rows */
+constexpr int kCellDepth = 2;
+constexpr int kCellRing = kCellDepth + 2;
+static_assert(kCellSegMin % kCellRing == 0 && kCellSegMax % kCellRing == 0 && kCellSegMax + 4 <= 32,
+              "a tile is whole turns of the ring, and its staged rows fit one 32-bit mask");
 
 /* k_cbulk keeps its row offsets in 32 bits. The largest it forms is the refill offset of the last tile: row
  * x + D + 1 for a row x <= xb + RG - 1 of the unrolled ring (rows past xb run on clamped rows), i.e. below
  * (xb + RG + D + 1) ps with xb <= mesh_x + 2, before it is clamped to row xb + 1; the in-row offset adds less than
  * ps. A grid takes the cells path only when all of these fit: (rows_x + kCellSlack) * ps <= INT32_MAX. */
 constexpr int kCellSlack = 32;
-static_assert(kCellRing<float> + kCellBulkDepth<float> + 1 <= kCellSlack - 4 &&
-                  kCellRing<double> + kCellBulkDepth<double> + 1 <= kCellSlack - 4,
-              "the cells path's 32-bit offset bound needs a larger slack");
+static_assert(kCellRing + kCellDepth + 1 <= kCellSlack - 4, "the cells path's 32-bit offset bound needs a larger slack");
 __host__ __device__ constexpr bool cells_fit(int64_t rows_x, int64_t ps) {
   return (rows_x + kCellSlack) * ps <= (int64_t)0x7fffffff;
+}
+
+/* Append to the two lists of a step: counts holds their lengths (interface cells, delta-phi candidates) as one 64-bit
+ * word, so that a wavefront reserves its entries in both with one atomic. */
+__device__ __forceinline__ uint64_t list_reserve(int *counts, int ni, int nc) {
+  return atomicAdd((unsigned long long *)counts, (unsigned long long)ni | ((unsigned long long)nc << 32));
 }
 
 /* Delta-phi candidates on the ring x or y in {2, mesh+3} around the interior (k_cbulk's tiles list the interior
  * ones): ring cell i (one per thread of k_cbulk's extra blocks), appended to the same list. */
 __device__ __forceinline__ void dring_cell(int64_t i, const int8_t *__restrict__ codes, int32_t *__restrict__ clist,
-                                           int *ccount, int64_t ps, int64_t mx, int64_t my) {
+                                           int *counts, int64_t ps, int64_t mx, int64_t my) {
   const int lane = threadIdx.x & 63;
   const int64_t nxr = my + 2, nyr = mx; /* rows x = 2, mx+3 over y in [2, my+3]; columns y = 2, my+3 over x in [3, mx+2] */
   int64_t x = -1, y = -1;
   if (i < 2 * nxr) {
     x = (i < nxr) ? 2 : mx + 3;
-    y = 2 + (i % nxr);
+    y = 2 + (i < nxr ? i : i - nxr);
   } else if (i < 2 * nxr + 2 * nyr) {
     const int64_t k = i - 2 * nxr;
     y = (k < nyr) ? 2 : my + 3;
-    x = 3 + (k % nyr);
+    x = 3 + (k < nyr ? k : k - nyr);
   }
   bool cand = false;
   const int64_t c = x * ps + y + kYOff;
   if (x >= 0) {
-    const int8_t k0 = codes[c];
-    cand = k0 < 0 || codes[c - ps] != k0 || codes[c + ps] != k0 || codes[c - 1] != k0 || codes[c + 1] != k0;
+    const int8_t k0 = codes[c], k1 = codes[c - ps], k2 = codes[c + ps], k3 = codes[c - 1], k4 = codes[c + 1];
+    cand = (k0 < 0) | (k1 != k0) | (k2 != k0) | (k3 != k0) | (k4 != k0);
   }
   const uint64_t mask = __ballot(cand);
   if (!mask) return;
   const int leader = __ffsll((long long)mask) - 1;
   int base = 0;
-  if (lane == leader) base = atomicAdd(ccount, __popcll(mask));
+  if (lane == leader) base = (int)(list_reserve(counts, 0, __popcll(mask)) >> 32);
   base = __shfl(base, leader);
   if (cand) clist[base + __popcll(mask & ((1ull << lane) - 1ull))] = (int32_t)c;
 }
 
-/* a floor of waves per SIMD for k_cbulk's register allocation: the FP32 kernels of up to two mu fields fit seven
- * (the LDS bound) with at most one spilled register; the others keep their natural allocation */
-template <typename R, int NC>
-constexpr int kCbulkWaves = (sizeof(R) == 4 && NC <= 2) ? 7 : 1;
+/* Element i of a row at the wave-uniform address p: a scalar base plus an unsigned 32-bit byte offset per lane, the
+ * addressing mode of the global instructions. The base goes through an empty asm so that the compiler keeps that form: left
+ * to itself it adds the lane's offset first and holds a 64-bit vector address per plane. */
+template <typename T, typename E>
+__device__ __forceinline__ T row_ld(const E *p, unsigned i) {
+#if defined(__AMDGCN__)
+  uint64_t b = (uint64_t)p;
+  asm("" : "+s"(b));
+  return *(const __attribute__((address_space(1))) T *)(b + (uint64_t)(i * (unsigned)sizeof(E)));
+#else
+  return *(const T *)(p + i);
+#endif
+}
+template <typename T, typename E>
+__device__ __forceinline__ void row_st(E *p, unsigned i, T v) {
+#if defined(__AMDGCN__)
+  uint64_t b = (uint64_t)p;
+  asm("" : "+s"(b));
+  *(__attribute__((address_space(1))) T *)(b + (uint64_t)(i * (unsigned)sizeof(E))) = v;
+#else
+  *(T *)(p + i) = v;
+#endif
+}
 
-template <int N, int NC, typename R, bool P2, bool STATS, bool C = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCbulkWaves<R, NC>)))
-void k_cbulk(const Model<R> *__restrict__ mp, const R *__restrict__ mu,
-                                               const int8_t *__restrict__ codes_in, R *__restrict__ phi_o,
-                                               R *__restrict__ mu_o, int8_t *__restrict__ codes_out,
-                                               double *__restrict__ partials, int64_t pstride, int64_t fs, int64_t ps,
-                                               int64_t mx, int64_t my, int seg_len, int nstrips, int nwaves,
-                                               int keep, int32_t *__restrict__ ilist, int32_t *__restrict__ clist,
-                                               int *counts, int *counts_next, int tile_blocks,
-                                               const int8_t *__restrict__ mlo, float *__restrict__ plo_o,
-                                               int8_t *__restrict__ mlo_o) {
+/* two adjacent cells of a row, the first (x) at an even element offset */
+template <typename R>
+struct PairOf;
+template <>
+struct PairOf<float> {
+  typedef float type __attribute__((ext_vector_type(2)));
+};
+template <>
+struct PairOf<double> {
+  typedef double type __attribute__((ext_vector_type(2)));
+};
+template <typename R>
+using Pair = typename PairOf<R>::type;
+/* their phase codes, zero-extended: the first in the low byte, the second in the high one */
+__device__ __forceinline__ unsigned code_pair(const int8_t *row, unsigned i) { return row_ld<uint16_t>(row, i); }
+
+/* Row classes of a lane's two columns over the staged rows, one bit per row (bit r: staged row r): bulk cells of every
+ * phase, and cells whose five-point codes are uniform (no delta-phi candidate). Vertical neighbours are shifts of
+ * the column's mask, horizontal ones the other column of the lane or a DPP move of the neighbour lane's masks: about
+ * 25 VALU instructions per phase for all rows of the tile, where the code-by-code test reads 13 codes per cell. */
+template <int N>
+struct TileMasks {
+  uint32_t be[N], bo[N]; /* bulk cells of phase b in the first / second column */
+  uint32_t ue, uo;       /* cells with uniform five-point codes */
+};
+template <int N, int ROWS>
+__device__ __forceinline__ TileMasks<N> tile_masks(const unsigned (&cv)[ROWS]) {
+  TileMasks<N> t;
+  t.ue = t.uo = 0u;
+#pragma unroll
+  for (int b = 0; b < N; b++) {
+    uint32_t e = 0u, o = 0u;
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+      e |= ((cv[r] & 0xffu) == (unsigned)b ? 1u : 0u) << r;
+      o |= ((cv[r] >> 8) == (unsigned)b ? 1u : 0u) << r;
+    }
+    const uint32_t el = (uint32_t)lane_up((int)e), er = (uint32_t)lane_dn((int)e);
+    const uint32_t ol = (uint32_t)lane_up((int)o), or_ = (uint32_t)lane_dn((int)o);
+    auto v1 = [](uint32_t c) { return c & (c << 1) & (c >> 1); };
+    const uint32_t e1 = v1(e), o1 = v1(o);
+    t.be[b] = e1 & (e << 2) & (e >> 2) & o1 & v1(ol) & el & er;
+    t.bo[b] = o1 & (o << 2) & (o >> 2) & e1 & v1(er) & ol & or_;
+    t.ue |= e1 & o & ol;
+    t.uo |= o1 & e & er;
+  }
+  return t;
+}
+
+/* The statistics of the padding rows. The reported extrema and sums of squared increments of mu include, on a grid whose
+ * rows are not a multiple of four, up to three rows past mesh+2 for the tiles of kPadOut cells by kPadSeg rows at the
+ * grid's end whose cells and neighbours are all of one phase: the updates of row mesh+3 with itself as the row above
+ * (and, after the first, below). These terms belong to no cell; they are kept so that the reported figures stay what
+ * they were. One wavefront per strip s; returns its partials through st. */
+template <int N, int NC, typename R, bool P2, bool C, int NSA>
+__device__ __forceinline__ void pad_stats(const Model<R> &m, const R *__restrict__ mu, const int8_t *__restrict__ mlo,
+                                          const int8_t *__restrict__ codes, int s, int64_t fs, int64_t ps, int64_t mx,
+                                          int64_t my, R divjat0, R (&st)[NSA]) {
+  const int lane = threadIdx.x & 63;
+  const int64_t y = 3 + (int64_t)s * kPadOut - 2 + lane, ry = my + 6, c0 = (y < ry - 1 ? y : ry - 1) + kYOff;
+  const int64_t xb = mx + 2, xa = 3 + (mx - 1) / kPadSeg * kPadSeg;
+  const int b = codes[(xa - 2) * ps + c0];
+  bool same = b >= 0;
+  for (int64_t x = xa - 1; x <= xb + 2; x++) same = same & (codes[x * ps + c0] == b);
+  const int b0 = __builtin_amdgcn_readfirstlane(b);
+  if (!__all(same && b == b0)) return;
+  R m0[NC], m1[NC], up[NC], dn[NC], mn[NC], dm[NC];
+#pragma unroll
+  for (int k = 0; k < NC; k++) {
+    m0[k] = mu[k * fs + xb * ps + c0];
+    m1[k] = mu[k * fs + (xb + 1) * ps + c0];
+    up[k] = lane_up(m1[k]);
+    dn[k] = lane_dn(m1[k]);
+  }
+  const bool out = lane >= 2 && lane <= 61 && y <= my + 2;
+  for (int64_t i = mx % 4; i < 4; i++) {
+    if constexpr (kLeanBulk<R>) {
+      R K[NC][NC];
+#pragma unroll
+      for (int k = 0; k < NC; k++)
+#pragma unroll
+        for (int l = 0; l < NC; l++) K[k][l] = m.Kbulk[b0][k][l];
+      bulk_update_lean<NC>(m, K, m0, m1, m1, dn, up, mn, dm);
+    } else {
+      bulk_update_ref<N, NC, R, P2>(m, b0, m0, m1, m1, dn, up, divjat0, mn, dm);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+      if constexpr (C) {
+        float hn;
+        int8_t qn;
+        c32_encode(c32_decode((float)m1[k], mlo[k * fs + (xb + 1) * ps + c0]) + (double)dm[k], hn, qn);
+        mn[k] = (R)hn;
+      }
+      m0[k] = m1[k];
+    }
+    if (out) bulk_stats<N, NC>(st, mn, dm);
+  }
+}
+
+/* Two cells per lane and no LDS: a wavefront has 512 B (FP32) or 1 KiB (FP64) per load in flight, neighbouring lanes meet by
+ * one DPP move per two cells, and a strip re-reads 4 of 128 columns where one cell per lane re-reads 4 of 64. Bound by
+ * VALU issue and memory together: 4096^2 compensated, 1.2% of the cells at interfaces, 122 us (137 with one cell
+ * per lane, codes in LDS) for 411 MB of traffic; FP32 2047 x 1801 33 us (45). On small grids it is one tile's latency:
+ * 48 x 40 ternary FP64 13 us with 4-row segments (39 with 16-row ones and the cell-by-cell test), 200^2 binary 12 (30). */
+template <int N, int NC, typename R, bool P2, bool STATS, int SEG, bool C = false>
+__global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, const R *__restrict__ mu, const int8_t *__restrict__ codes_in,
+             R *__restrict__ phi_o, R *__restrict__ mu_o, int8_t *__restrict__ codes_out,
+             double *__restrict__ partials, int64_t pstride, int64_t fs, int64_t ps, int64_t mx, int64_t my,
+             int nstrips, int nwaves, int keep, const int8_t *__restrict__ tin, int8_t *__restrict__ tout,
+             int32_t *__restrict__ ilist, int32_t *__restrict__ clist, int *counts, int *counts_next, int tile_blocks,
+             int ring_blocks, const int8_t *__restrict__ mlo, float *__restrict__ plo_o, int8_t *__restrict__ mlo_o) {
   using Vw = View<R, P2, false, kFastOf<R>>;
   constexpr int NS = 3 * N + 3 * NC + 1;
   constexpr int NSA = STATS ? NS : 1;
-  if ((int)blockIdx.x >= tile_blocks) {
-    /* the blocks past the tiles list the delta-phi candidates of the ring x or y in {2, mesh+3} around the
-     * interior (one thread per ring cell; the tiles list the interior ones) */
-    dring_cell((int64_t)(blockIdx.x - tile_blocks) * blockDim.x + threadIdx.x, codes_in, clist, counts + 1, ps, mx,
-               my);
-    return;
-  }
-  __shared__ int8_t cs_all[4][kCellRows * 64];
-  __shared__ uint16_t il_all[4][kCellSegMax * 64], cl_all[4][kCellSegMax * 64];
-  __shared__ int wcnt[2][4], wbase[2][4];
-  uint16_t *il = il_all[threadIdx.x >> 6], *cl = cl_all[threadIdx.x >> 6];
-  int icnt = 0, ccnt = 0;
+  constexpr int RG = kCellRing, D = kCellDepth, ROWS = SEG + 4;
   const Model<R> &m = *mp;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int w = blockIdx.x * 4 + wv; /* wave-uniform: the tile's rows and the row loop are scalar */
-  int8_t *cs = cs_all[wv];
-  R st[NSA];
-  if (STATS) stats_init<N, NC>(st);
-  unsigned seen = 0u; /* phases of the lane's bulk cells in mixed tiles (their phi extrema, folded at the end) */
-  const CellTile t(w, lane, mx, my, seg_len, nstrips);
-  const int64_t c0 = t.yl + kYOff;
+  const R zj = R(0.0) * m.jat_fac; /* (j - j_prev) * jat_fac with both currents +0 */
+  R divjat0 = divx<Vw>(m, zj);
+  divjat0 += divy<Vw>(m, zj);
+  if ((int)blockIdx.x >= tile_blocks) {
+    /* the blocks past the tiles list the delta-phi candidates of the ring x or y in {2, mesh+3} around the
+     * interior (one thread per ring cell; the tiles list the interior ones), then fold the padding rows */
+    const int q = (int)blockIdx.x - tile_blocks;
+    if (q < ring_blocks) {
+      dring_cell((int64_t)q * 256 + threadIdx.x, codes_in, clist, counts, ps, mx, my);
+    } else if constexpr (STATS) {
+      const int s = (q - ring_blocks) * 4 + wv, npad = (int)((my + kPadOut - 1) / kPadOut);
+      if (s >= npad) return;
+      R st[NSA];
+      stats_init<N, NC>(st);
+      pad_stats<N, NC, R, P2, C>(m, mu, mlo, codes_in, s, fs, ps, mx, my, divjat0, st);
+      stats_partials<N, NC, true>(st, partials, pstride, nwaves + s, nwaves + npad, lane);
+    }
+    return;
+  }
   /* the next step's list lengths start at zero (the kernels that read them last ran before this one) */
   if (blockIdx.x == 0 && threadIdx.x < 2) counts_next[threadIdx.x] = 0;
+  /* blocks go round the eight XCDs in turn: each XCD takes a contiguous run of tiles, so that the lines and rows two
+   * neighbouring tiles share meet in one L2 */
+  const int chunk = tile_blocks >> 3, bid = (int)blockIdx.x;
+  const int tblk = bid < 8 * chunk ? (bid & 7) * chunk + (bid >> 3) : bid;
+  const int w = tblk * 4 + wv; /* wave-uniform: the tile's rows and the row loop are scalar */
+  if (w >= nwaves) return;
+  const int strip = w % nstrips, seg = w / nstrips;
+  const int xa = 3 + seg * SEG, nrow = min(SEG, (int)mx + 3 - xa), xb = xa + nrow - 1;
+  /* the lane's cells y (an even element offset) and y + 1; lanes past the grid read its last pair */
+  const int y = 1 + strip * kCellOut + 2 * lane, ry = (int)my + 6;
+  const int yl = min(y, (ry - 3) | 1);
+  const bool inner = lane >= 1 && lane <= 62;
+  const bool oe = inner && y <= (int)my + 2, oo = inner && y + 1 <= (int)my + 2;
+  /* addresses: a scalar row offset and an unsigned in-row offset per lane, so that a plane costs no vector registers */
+  const int pso = (int)ps, xlast = (xb + 1) * pso;
+  const unsigned c0i = (unsigned)(yl + kYOff), cyi = (unsigned)(y + kYOff);
+
+  R st[NSA];
+  if (STATS) stats_init<N, NC>(st);
+  unsigned seen = 0u; /* phases of the lane's bulk cells (their phi extrema, folded at the end) */
+
   /* mu rows in a ring of kCellRing register slots, row r in slot (r - xa) mod kCellRing, so that no slot is
    * ever copied: the row being updated reads rows x-1, x, x+1 where they were loaded, and the slot of x-1 then
-   * takes row x + kCellBulkDepth + 1. The phase codes of the output buffers (for `kept`) ride the same ring,
-   * kCellBulkDepth rows ahead. A loaded value is first read kCellBulkDepth rows after its load, and no wait
-   * in between covers a newer load (the counter of outstanding memory operations is in order). */
-  constexpr int RG = kCellRing<R>, D = kCellBulkDepth<R>;
-  R ring[RG][NC];
-  int8_t qring[RG][NC]; /* compensated mode: the mu extensions of the ring's rows */
-  uint8_t kc[RG]; /* output codes as bytes (zero-extending loads, no sign extension after the load) */
-  const uint8_t *codes_ou = (const uint8_t *)codes_out;
-  if (w < nwaves) {
-    /* the tile's loads all issue before the first wait: its phase codes (rows xa-2 .. xa+kCellRows-3, clamped
-     * to xb+2), the first mu rows and output codes of the ring (every load is issued on every path; rows past the
-     * tile's end are clamped to its last row + 1, which is inside the halo) */
-    int8_t cv[kCellRows];
+   * takes row x + kCellDepth + 1. The phase codes of the output buffers (which tell whether phi is already e_b
+   * there) ride the same ring in the mixed tiles. A loaded value is first read kCellDepth rows after its load, and
+   * no wait in between covers a newer load (the counter of outstanding memory operations is in order). */
+  Pair<R> ring[RG][NC];
+  uint16_t qring[RG][NC]; /* compensated mode: the mu extensions of the ring's rows */
+  unsigned kc[RG];
+  auto load_row = [&](int slot, int off) {
 #pragma unroll
-    for (int r = 0; r < kCellRows; r++) {
-      const int64_t xr = t.xa - 2 + r <= t.xb + 2 ? t.xa - 2 + r : t.xb + 2;
-      cv[r] = codes_in[xr * ps + c0];
+    for (int k = 0; k < NC; k++) ring[slot][k] = row_ld<Pair<R>>(mu + (k * fs + off), c0i);
+    if constexpr (C) {
+#pragma unroll
+      for (int k = 0; k < NC; k++) qring[slot][k] = row_ld<uint16_t>(mlo + (k * fs + off), c0i);
     }
+  };
+  /* the tile's first loads all issue before the first wait: its phase codes (rows xa-2 .. xa+SEG+1, clamped to xb+2)
+   * and the first mu rows of the ring (rows past the tile's end are clamped to its last row + 1) */
+  unsigned cv[ROWS];
 #pragma unroll
-    for (int d = -1; d <= D; d++) {
-      const int64_t xr = t.xa + d <= t.xb + 1 ? t.xa + d : t.xb + 1;
+  for (int r = 0; r < ROWS; r++) cv[r] = code_pair(codes_in + (int64_t)(min(xa - 2 + r, xb + 2) * pso), c0i);
 #pragma unroll
-      for (int k = 0; k < NC; k++) ring[(d + RG) % RG][k] = mu[k * fs + xr * ps + c0];
-      if constexpr (C) {
+  for (int d = -1; d <= D; d++) load_row((d + RG) % RG, min((xa + d) * pso, xlast));
+  /* a full tile whose staged codes are all one phase tb has only bulk cells of that phase */
+  int tb = -1;
+  if (nrow == SEG && (strip + 1) * kCellOut <= (int)my) {
+    unsigned diff = 0u;
 #pragma unroll
-        for (int k = 0; k < NC; k++) qring[(d + RG) % RG][k] = mlo[k * fs + xr * ps + c0];
+    for (int r = 1; r < ROWS; r++) diff |= cv[r] ^ cv[0];
+    const unsigned u0 = __builtin_amdgcn_readfirstlane(cv[0]);
+    if (__all(diff == 0u && cv[0] == u0) && (u0 >> 8) == (u0 & 0xffu) && !(u0 & 0x80u)) tb = (int)(u0 & 0xffu);
+  }
+  /* tile flags: the phase of a uniform tile of the current state for the next step, whose output buffers hold this
+   * state; the previous step's flag says the same of this step's output buffers */
+  const bool kept_tile = keep && tb >= 0 && tin[w] == tb;
+  if (lane == 0) tout[w] = (int8_t)tb;
+
+  /* The rows of the tile, instantiated twice so that the uniform form is a loop of its own: every lane of it computes
+   * and folds the mu statistics, only the inner ones write. t: the mixed form's bulk cells, bit r + 2 for row xa + r.
+   * In FP32 a mixed row is one pass with each cell's coefficients selected by its phase; in FP64, whose update takes
+   * seven times the coefficients, it is one pass per phase that has bulk cells in the row. */
+  auto rows = [&](auto uniform, const TileMasks<N> &t) {
+    constexpr bool UNI = decltype(uniform)::value;
+    int xoff = xa * pso;
+    for (int x0 = 0; x0 < nrow; x0 += RG) {
+#pragma unroll
+      for (int j = 0; j < RG; j++) {
+        const int64_t xo = xoff;
+        R e0[NC], e1[NC], e2[NC], o0[NC], o1[NC], o2[NC], ol[NC], er[NC];
+#pragma unroll
+        for (int k = 0; k < NC; k++) {
+          const Pair<R> q0 = ring[(j + RG - 1) % RG][k], q1 = ring[j][k], q2 = ring[(j + 1) % RG][k];
+          e0[k] = q0.x;
+          o0[k] = q0.y;
+          e1[k] = q1.x;
+          o1[k] = q1.y;
+          e2[k] = q2.x;
+          o2[k] = q2.y;
+          ol[k] = lane_up(o1[k]);
+          er[k] = lane_dn(e1[k]);
+        }
+        /* the cells' new mu (and extensions), phi = e_b where the output buffer does not hold it already, statistics */
+        auto finish = [&](bool se, bool so, int be, int bo, R *ne, R *de, R *no, R *dn) {
+          uint16_t qn[NC];
+          if constexpr (C) {
+            /* compensated mode: the increment is added to the decoded value (hi plus its extension) and the sum is
+             * re-encoded, so the bits of the increment below the FP32 part are kept */
+#pragma unroll
+            for (int k = 0; k < NC; k++) {
+              const unsigned q = qring[j][k];
+              float he, ho;
+              int8_t ne8, no8;
+              c32_encode(c32_decode((float)e1[k], (int8_t)(q & 0xffu)) + (double)de[k], he, ne8);
+              c32_encode(c32_decode((float)o1[k], (int8_t)(q >> 8)) + (double)dn[k], ho, no8);
+              ne[k] = (R)he;
+              no[k] = (R)ho;
+              qn[k] = (uint16_t)((unsigned)(uint8_t)ne8 | ((unsigned)(uint8_t)no8 << 8));
+            }
+          }
+          if (se && so) {
+#pragma unroll
+            for (int k = 0; k < NC; k++) row_st<Pair<R>>(mu_o + (k * fs + xo), cyi, Pair<R>{ne[k], no[k]});
+            if constexpr (C) {
+#pragma unroll
+              for (int k = 0; k < NC; k++) row_st<uint16_t>(mlo_o + (k * fs + xo), cyi, qn[k]);
+            }
+          } else if (!UNI && (se || so)) {
+            const unsigned c1 = se ? cyi : cyi + 1u;
+#pragma unroll
+            for (int k = 0; k < NC; k++) row_st<R>(mu_o + (k * fs + xo), c1, se ? ne[k] : no[k]);
+            if constexpr (C) {
+#pragma unroll
+              for (int k = 0; k < NC; k++)
+                row_st<int8_t>(mlo_o + (k * fs + xo), c1, (int8_t)(se ? qn[k] & 0xffu : qn[k] >> 8));
+            }
+          }
+          if (UNI) {
+            if (!kept_tile && inner) {
+#pragma unroll
+              for (int a = 0; a < N; a++) {
+                const R p = a == be ? R(1.0) : R(0.0);
+                row_st<Pair<R>>(phi_o + (a * fs + xo), cyi, Pair<R>{p, p});
+                if constexpr (C) row_st<Pair<float>>(plo_o + (a * fs + xo), cyi, Pair<float>{0.0f, 0.0f});
+              }
+              row_st<uint16_t>(codes_out + xo, cyi, (uint16_t)(be * 0x101));
+            }
+          } else {
+            if (se && !(keep && (kc[j] & 0xffu) == (unsigned)be)) {
+#pragma unroll
+              for (int a = 0; a < N; a++) {
+                row_st<R>(phi_o + (a * fs + xo), cyi, a == be ? R(1.0) : R(0.0));
+                if constexpr (C) row_st<float>(plo_o + (a * fs + xo), cyi, 0.0f);
+              }
+              row_st<int8_t>(codes_out + xo, cyi, (int8_t)be);
+            }
+            if (so && !(keep && (kc[j] >> 8) == (unsigned)bo)) {
+#pragma unroll
+              for (int a = 0; a < N; a++) {
+                row_st<R>(phi_o + (a * fs + xo), cyi + 1u, a == bo ? R(1.0) : R(0.0));
+                if constexpr (C) row_st<float>(plo_o + (a * fs + xo), cyi + 1u, 0.0f);
+              }
+              row_st<int8_t>(codes_out + xo, cyi + 1u, (int8_t)bo);
+            }
+          }
+          if (STATS) {
+            if (UNI || se) bulk_stats<N, NC>(st, ne, de);
+            if (UNI || so) bulk_stats<N, NC>(st, no, dn);
+          }
+        };
+        R ne[NC], no[NC], de[NC], dn[NC];
+        if constexpr (kLeanBulk<R>) {
+          R Ke[NC][NC], Ko[NC][NC];
+          bool se = UNI && inner, so = se;
+          int be = UNI ? tb : 0, bo = be;
+#pragma unroll
+          for (int a = 0; a < N; a++) {
+            const bool ea = (t.be[a] >> (x0 + j + 2)) & 1u, oa = (t.bo[a] >> (x0 + j + 2)) & 1u;
+            if (!UNI) {
+              se = se || ea;
+              so = so || oa;
+              be = ea ? a : be;
+              bo = oa ? a : bo;
+            }
+#pragma unroll
+            for (int k = 0; k < NC; k++)
+#pragma unroll
+              for (int l = 0; l < NC; l++) {
+                const R kk = UNI ? m.Kbulk[tb][k][l] : scalar_val(m.Kbulk[a][k][l]);
+                Ke[k][l] = UNI || a == 0 || ea ? kk : Ke[k][l];
+                Ko[k][l] = UNI || a == 0 || oa ? kk : Ko[k][l];
+              }
+            if (UNI) break;
+          }
+          if (UNI || __any(se || so)) {
+            bulk_update_lean<NC>(m, Ke, e0, e1, e2, o1, ol, ne, de);
+            bulk_update_lean<NC>(m, Ko, o0, o1, o2, er, e1, no, dn);
+            finish(se, so, be, bo, ne, de, no, dn);
+          }
+        } else {
+#pragma unroll
+          for (int a = 0; a < (UNI ? 1 : N); a++) {
+            const bool se = UNI ? inner : (t.be[a] >> (x0 + j + 2)) & 1u;
+            const bool so = UNI ? inner : (t.bo[a] >> (x0 + j + 2)) & 1u;
+            if (UNI || __any(se || so)) {
+              const int b = UNI ? tb : a;
+              bulk_update_ref<N, NC, R, P2>(m, b, e0, e1, e2, o1, ol, divjat0, ne, de);
+              bulk_update_ref<N, NC, R, P2>(m, b, o0, o1, o2, er, e1, divjat0, no, dn);
+              finish(se, so, b, b, ne, de, no, dn);
+            }
+          }
+        }
+        /* refill: row x + D + 1 into the slot of row x - 1, the output codes of row x + D */
+        const int xn = min(xoff + (D + 1) * pso, xlast);
+        load_row((j + RG - 1) % RG, xn);
+        if (!UNI) kc[(j + D) % RG] = code_pair(codes_out + (xn - pso), c0i);
+        xoff += pso;
+        /* the rows stay apart: interleaved, the four rows of a turn would take twice the registers */
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-#pragma unroll
-    for (int d = 0; d < D; d++) kc[d] = codes_ou[(t.xa + d <= t.xb ? t.xa + d : t.xb) * ps + c0];
-#pragma unroll
-    for (int r = 0; r < kCellRows; r++) cs[r * 64 + lane] = cv[r];
+  };
+
+  if (tb >= 0) {
     /* the prologue's loads complete here, once per tile: the loop's first row then waits on nothing, and the
      * wait counts inside the loop follow from the loop body alone (vmcnt 0, expcnt and lgkmcnt unconstrained) */
     __builtin_amdgcn_s_waitcnt(0x0f70);
-  }
-  __syncthreads();
-  if (w < nwaves) {
-    /* a tile whose staged codes are all one phase b has only bulk cells of phase b: no per-cell test */
-    int tb = -1;
-    {
-      const int u = cs[lane];
-      bool same = u >= 0;
-      const int nr = (int)(t.xb - t.xa) + 5;
-      for (int r = 1; r < nr; r++) same = same && cs[r * 64 + lane] == u;
-      const int u0 = __builtin_amdgcn_readfirstlane(u);
-      if (__all(same && u == u0)) tb = u0;
+    rows(std::true_type{}, TileMasks<N>{});
+    if (STATS) {
+      if (!inner) stats_init<N, NC>(st);
+      else seen = 1u << tb;
     }
-    const R zj = R(0.0) * m.jat_fac; /* (j - j_prev) * jat_fac with both currents +0 */
-    R divjat0 = divx<Vw>(m, zj);
-    divjat0 += divy<Vw>(m, zj);
-    /* the row loop, instantiated twice so that the tile-uniform form is a loop of its own (no per-row test) */
-    /* row offsets in 32 bits (the cells path runs on grids of fewer than 2^31 cells), kept incrementally */
-    const int pso = (int)ps, c0i = (int)c0, cyi = (int)(t.y + kYOff);
-    const int xa = (int)t.xa, xb = (int)t.xb, mxi = (int)mx;
-    const int xlast = (xb + 1) * pso;
-    auto rows = [&](auto uniform) {
-      constexpr bool UNI = decltype(uniform)::value;
-      int xoff = xa * pso;
-      for (int x0 = xa; x0 <= xb; x0 += RG) {
+  } else {
 #pragma unroll
-        for (int j = 0; j < RG; j++) {
-          /* rows past the tile's last one (at the grid's end) run on clamped rows and write nothing: the loop
-           * has one exit and every path through its body issues every load */
-          const int x = x0 + j;
-          const bool live = x <= xb;
-          const int64_t c = (int64_t)xoff + cyi;
-          const R *m0 = ring[(j + RG - 1) % RG], *m1 = ring[j], *m2 = ring[(j + 1) % RG];
-          R mud[NC], muu[NC];
+    for (int d = 0; d < D; d++) kc[d] = code_pair(codes_out + min((xa + d) * pso, xlast - pso), c0i);
+    TileMasks<N> t = tile_masks<N>(cv);
+    const uint32_t live = ((1u << nrow) - 1u) << 2;
+    const uint32_t le = oe ? live : 0u, lo = oo ? live : 0u;
+    uint32_t ie = le, io = lo;
 #pragma unroll
-          for (int k = 0; k < NC; k++) {
-            mud[k] = lane_dn(m1[k]);
-            muu[k] = lane_up(m1[k]);
-          }
-          if (UNI) {
-            cbulk_cell<N, NC, R, P2, STATS, true, NSA, C>(m, tb, c, m0, m1, m2, mud, muu, divjat0, phi_o, mu_o,
-                                                          codes_out, fs, keep && kc[j] == (uint8_t)tb,
-                                                          live && t.out_lane, live, st, seen, qring[j], plo_o, mlo_o);
-          } else if (live) {
-            const int bl = t.out_lane ? bulk_of(cs, x - xa + 2, lane) : -1;
-            {
-              /* the row's interface cells (for k_ilist) and delta-phi candidates (for k_dlist) */
-              const int r = x - xa + 2;
-              const int8_t k0 = cs[r * 64 + lane];
-              const bool cand = t.out_lane && (k0 < 0 || cs[(r - 1) * 64 + lane] != k0 ||
-                                               cs[(r + 1) * 64 + lane] != k0 || cs[r * 64 + lane - 1] != k0 ||
-                                               cs[r * 64 + lane + 1] != k0);
-              const bool iface = t.out_lane && bl < 0;
-              const uint16_t e = (uint16_t)((x - xa) * 64 + lane);
-              const uint64_t lt = (1ull << lane) - 1ull;
-              const uint64_t mi = __ballot(iface), mc = __ballot(cand);
-              if (iface) il[icnt + __popcll(mi & lt)] = e;
-              if (cand) cl[ccnt + __popcll(mc & lt)] = e;
-              icnt += __popcll(mi);
-              ccnt += __popcll(mc);
-            }
-            if (bl >= 0)
-              cbulk_cell<N, NC, R, P2, STATS, false, NSA, C>(m, bl, c, m0, m1, m2, mud, muu, divjat0, phi_o, mu_o,
-                                                             codes_out, fs, keep && kc[j] == (uint8_t)bl, true, true,
-                                                             st, seen, qring[j], plo_o, mlo_o);
-          }
-          /* refill: row x + D + 1 into the slot of row x - 1, the output codes of row x + D */
-          const int xn = min(xoff + (D + 1) * pso, xlast);
-#pragma unroll
-          for (int k = 0; k < NC; k++) ring[(j + RG - 1) % RG][k] = mu[k * fs + (int64_t)(xn + c0i)];
-          if constexpr (C) {
-#pragma unroll
-            for (int k = 0; k < NC; k++) qring[(j + RG - 1) % RG][k] = mlo[k * fs + (int64_t)(xn + c0i)];
-          }
-          kc[(j + D) % RG] = codes_ou[(int64_t)(xn - pso + c0i)];
-          xoff += pso;
-        }
-      }
-    };
-    if (tb >= 0)
-      rows(std::true_type{});
-    else
-      rows(std::false_type{});
-    if (STATS && tb >= 0) {
-      /* the tile-uniform rows folded the mu statistics of every lane: keep those of the tile's cells, and add
-       * the phi extrema of its cells (e_tb on each) once */
-      if (!t.out_lane) {
-        stats_init<N, NC>(st);
-      } else {
-#pragma unroll
-        for (int a = 0; a < N; a++) {
-          st[a] = fmax(st[a], a == tb ? R(1.0) : R(0.0));
-          st[N + a] = fmin(st[N + a], a == tb ? R(1.0) : R(0.0));
-        }
+    for (int b = 0; b < N; b++) {
+      t.be[b] &= le;
+      t.bo[b] &= lo;
+      ie &= ~t.be[b];
+      io &= ~t.bo[b];
+      if (t.be[b] | t.bo[b]) seen |= 1u << b;
+    }
+    const uint32_t ce = le & ~t.ue, co = lo & ~t.uo;
+    /* reserve the tile's list entries (the atomic's latency passes under the row loop) */
+    const int cnt = wave_sum((int)((__popc(ie) + __popc(io)) | ((__popc(ce) + __popc(co)) << 16)));
+    uint64_t base = 0;
+    if (cnt && lane == 0) base = list_reserve(counts, cnt & 0xffff, cnt >> 16);
+    rows(std::false_type{}, t);
+    /* the lists, row by row: a wavefront of the list kernels then gathers neighbouring cells of a row */
+    if (cnt) {
+      int bi = __builtin_amdgcn_readfirstlane((int)(base & 0xffffffffull));
+      int bc = __builtin_amdgcn_readfirstlane((int)(base >> 32));
+      int cell = xa * pso + (int)cyi;
+      auto emit = [&](int32_t *list, int &at, uint32_t e, uint32_t o, int r) {
+        const bool pe = (e >> r) & 1u, po = (o >> r) & 1u;
+        const uint64_t be = __ballot(pe), bo = __ballot(po);
+        if (!(be | bo)) return;
+        const uint64_t lt = (1ull << lane) - 1ull;
+        const int pos = at + __popcll(be & lt) + __popcll(bo & lt);
+        if (pe) list[pos] = cell;
+        if (po) list[pos + (pe ? 1 : 0)] = cell + 1;
+        at += __popcll(be) + __popcll(bo);
+      };
+      for (int r = 2; r < nrow + 2; r++, cell += pso) {
+        emit(ilist, bi, ie, io, r);
+        emit(clist, bc, ce, co, r);
       }
     }
-  }
-  /* one atomic per block and list: reserve the block's interface cells and candidates in the global lists */
-  if (lane == 0) {
-    wcnt[0][wv] = icnt;
-    wcnt[1][wv] = ccnt;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0)
-    for (int l = 0; l < 2; l++) {
-      int tot = 0;
-      for (int v = 0; v < 4; v++) {
-        wbase[l][v] = tot;
-        tot += wcnt[l][v];
-      }
-      const int b = tot > 0 ? atomicAdd(&counts[l], tot) : 0;
-      for (int v = 0; v < 4; v++) wbase[l][v] += b;
-    }
-  __syncthreads();
-  for (int i = lane; i < icnt; i += 64) {
-    const int e = il[i];
-    ilist[wbase[0][wv] + i] = (int32_t)((t.xa + (e >> 6)) * ps + (t.y - lane + (e & 63)) + kYOff);
-  }
-  for (int i = lane; i < ccnt; i += 64) {
-    const int e = cl[i];
-    clist[wbase[1][wv] + i] = (int32_t)((t.xa + (e >> 6)) * ps + (t.y - lane + (e & 63)) + kYOff);
   }
   if (!STATS) return;
   bulk_seen_fold<N>(st, seen);

@@ -64,6 +64,11 @@ __device__ __forceinline__ float mov(float v, float identity) {
 __device__ __forceinline__ float lane63(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ int mov(int v, int identity) {
+  return __builtin_amdgcn_update_dpp(identity, v, CTRL, ROWMASK, 0xf, false);
+}
+__device__ __forceinline__ int lane63(int v) { return __builtin_amdgcn_readlane(v, 63); }
 template <class T, class Op>
 __device__ __forceinline__ T reduce(T v, T identity, Op op) {
   v = op(v, mov<kQuad1032, 0xf>(v, identity));
@@ -84,6 +89,9 @@ __device__ __forceinline__ double wave_min(double v) {
 }
 __device__ __forceinline__ double wave_sum(double v) {
   return dpp::reduce<double>(v, 0.0, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ int wave_sum(int v) {
+  return dpp::reduce<int>(v, 0, [](int a, int b) { return a + b; });
 }
 /* extrema are exact in any precision: FP32 values take the single-register form */
 __device__ __forceinline__ float wave_max(float v) {

@@ -90,16 +90,16 @@ static void march_plan(gp_handle *h) {
   h->march_nstrips = (int)nstrips;
   h->march_nsegs = (int)((mx + seg - 1) / seg);
   h->march_nwaves = nstrips * h->march_nsegs;
-  /* the cell-classified kernels have almost no per-tile warm-up: 16-row segments (more, smaller tiles) even out
-   * the interface work between wavefronts; GP_CELL_SEG overrides (at most kCellSegMax) */
-  int64_t cseg = 16;
+  /* k_cbulk: a tile costs one memory latency plus its rows in turn, so segments are long only when that still gives
+   * kCellFill tiles; GP_CELL_SEG overrides (a value below kCellSegMax selects the short segments) */
+  const int64_t cstrips = (my + kCellOut - 1) / kCellOut;
+  int64_t cseg = cstrips * ((mx + kCellSegMax - 1) / kCellSegMax) >= kCellFill ? kCellSegMax : kCellSegMin;
   const char *ce = getenv("GP_CELL_SEG");
-  if (ce && atoi(ce) > 0) cseg = atoi(ce);
-  if (cseg > kCellSegMax) cseg = kCellSegMax;
-  if (cseg > mx) cseg = mx;
+  if (ce && atoi(ce) > 0) cseg = atoi(ce) >= kCellSegMax ? kCellSegMax : kCellSegMin;
   h->cell_seg = (int)cseg;
-  h->cell_nsegs = (int)((mx + cseg - 1) / cseg);
-  h->cell_nwaves = nstrips * h->cell_nsegs;
+  h->cell_nstrips = (int)cstrips;
+  h->cell_nwaves = cstrips * ((mx + cseg - 1) / cseg);
+  h->cell_npad = mx % 4 ? (int)((my + kPadOut - 1) / kPadOut) : 0;
 }
 
 /* ------------------------------------------------------------------------------------------------ helpers */
@@ -452,7 +452,7 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
   }
   h->nblocks_mu = ((params->mesh_y + kBX - 1) / kBX) * ((params->mesh_x + kBY - 1) / kBY);
   march_plan(h);
-  h->nparts_max = std::max(h->nblocks_mu, std::max(2 * h->march_nwaves, h->cell_nwaves + 4 * (int64_t)kListBlocks));
+  h->nparts_max = std::max(h->nblocks_mu, std::max(2 * h->march_nwaves, h->cell_nwaves + h->cell_npad + 4 * (int64_t)kListBlocks));
   const char *path = getenv("GP_PATH");
   h->use_march = !(path && strcmp(path, "twopass") == 0);
   /* the cell lists and k_cbulk's row offsets are 32-bit: grids beyond that bound (cells_fit, about 46000^2 cells)
@@ -495,6 +495,7 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
   ok = ok && hipMalloc((void **)&h->inv_dev, sizeof(double) * (GP_MAXNC + 1)) == hipSuccess;
   ok = ok && hipMalloc((void **)&h->flags[0], sizeof(int) * h->march_nwaves) == hipSuccess;
   ok = ok && hipMalloc((void **)&h->flags[1], sizeof(int) * h->march_nwaves) == hipSuccess;
+  ok = ok && hipMalloc((void **)&h->tflags, 2 * (size_t)h->cell_nwaves) == hipSuccess;
   ok = ok && hipMalloc((void **)&h->clist, (size_t)h->fs * sizeof(int32_t)) == hipSuccess &&
        hipMalloc((void **)&h->ilist, (size_t)h->fs * sizeof(int32_t)) == hipSuccess &&
        hipMalloc((void **)&h->lcount, 4 * sizeof(int)) == hipSuccess;
@@ -583,7 +584,7 @@ void gp_destroy(gp_handle *h) {
   void *bufs[] = {h->phi[0], h->phi[1], h->mu[0],    h->mu[1],    h->dphi,   h->partials, h->stats_dev,
                   h->model,  h->flags[0], h->flags[1], h->inv_dev, h->codes[0], h->codes[1], h->clist,
                   h->ilist,  h->lcount, h->lo[0],    h->lo[1],    h->model64, h->wide[0],  h->wide[1],
-                  h->trow,   h->thp,    h->thc,      h->front};
+                  h->trow,   h->thp,    h->thc,      h->front,    h->tflags};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   if (h->stream) (void)hipStreamDestroy(h->stream);

@@ -79,8 +79,10 @@ struct gp_handle {
   int64_t nparts_max;       /* rows of the partials buffer */
   int march_seg, march_nstrips, march_nsegs; /* tile grid of the single-pass step (see gp_march.h) */
   int64_t march_nwaves;     /* tiles = wavefronts of k_march and of k_bulk */
-  int cell_seg, cell_nsegs;  /* tile grid of k_cbulk (same strips as the march, shorter segments) */
+  int cell_seg, cell_nstrips; /* tile grid of k_cbulk: strips of kCellOut cells by segments of cell_seg rows */
   int64_t cell_nwaves;
+  int cell_npad;             /* wavefronts of the statistics' padding rows (none when mesh_x is a multiple of four) */
+  int8_t *tflags;            /* its tile flags of two alternating steps (by lsel) */
   int32_t *clist, *ilist;    /* delta-phi candidates and interface cells of the current step (cell offsets) */
   int *lcount;               /* their lengths: two pairs, used by alternate steps (lcount + 2 * lsel) */
   int lsel;

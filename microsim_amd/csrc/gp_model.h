@@ -990,6 +990,15 @@ GP_HD uint32_t f32_bits(float f) {
   return u;
 #endif
 }
+GP_HD uint32_t f64_low(double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint32_t)__double_as_longlong(d);
+#else
+  uint64_t u;
+  memcpy(&u, &d, sizeof u);
+  return (uint32_t)u;
+#endif
+}
 /* 2^k for -1022 <= k <= 1023, exactly */
 GP_HD double pow2d(int k) {
   const uint64_t b = (uint64_t)(k + 1023) << 52;
@@ -1001,19 +1010,19 @@ GP_HD double pow2d(int k) {
   return d;
 #endif
 }
+/* Branch-free: q is 0 where hi has no extension, and adds a zero there. The products are by powers of two, hence exact,
+ * and the fused forms round once, as the separate sum would. */
 GP_HD double c32_decode(float hi, int8_t q) {
-  if (q == 0) return (double)hi;
   const int E = (int)((f32_bits(hi) >> 23) & 0xffu);
-  return (double)hi + (double)q * pow2d(E - 157);
+  return __builtin_fma((double)q, pow2d(E - 157), (double)hi);
 }
 GP_HD void c32_encode(double v, float &hi, int8_t &q) {
   hi = (float)v;
   const int E = (int)((f32_bits(hi) >> 23) & 0xffu);
-  q = 0;
-  if (E == 0 || E == 255) return;
-  double s = rint((v - (double)hi) * pow2d(157 - E));
-  s = s > 127.0 ? 127.0 : (s < -127.0 ? -127.0 : s);
-  q = (int8_t)s;
+  /* the count of units, |v - hi| <= ulp32(hi) / 2 and so within +-64, rounded to nearest even by the sum with
+   * 1.5 2^52, whose low bits then hold the integer */
+  const double s = __builtin_fma(v - (double)hi, pow2d(157 - E), 6755399441055744.0);
+  q = (unsigned)(E - 1) < 254u ? (int8_t)f64_low(s) : (int8_t)0;
 }
 GP_HD double df_decode(float hi, float lo) { return (double)hi + (double)lo; }
 GP_HD void df_encode(double v, float &hi, float &lo) {

@@ -315,6 +315,43 @@ static int launch_invariants(gp_handle *h) {
 
 /* ------------------------------------------------------------------------------------------------ dispatch */
 
+/* statistics partials of a cell-classified step, per statistic: one per wavefront of k_cbulk's tiles and padding rows,
+ * then of k_ilist (from cell_ipart on) */
+static int64_t cell_ipart(const gp_handle *h) { return h->cell_nwaves + h->cell_npad; }
+static int64_t cell_parts(const gp_handle *h) { return cell_ipart(h) + 4 * h->lgrid_i; }
+
+/* k_cbulk of one step: the tiles, then the blocks that list the boundary ring's candidates (one thread per ring
+ * cell). This step's list lengths are zero (the previous step's k_cbulk, or the set-up, cleared them); k_cbulk clears
+ * the other pair for the next step. Returns this step's lengths (interface cells, candidates). C: compensated mode. */
+template <int N, int NC, typename R, bool P2, bool C, bool STATS, int SEG>
+static int *launch_cbulk_seg(gp_handle *h, const Model<R> *m) {
+  const int64_t mx = h->p.mesh_x, my = h->p.mesh_y;
+  const int ct = (int)h->cell_nwaves, b = h->cur, o = 1 - h->cur;
+  const unsigned cblk = (unsigned)((ct + 3) / 4), rblk = (unsigned)((2 * (my + 2) + 2 * mx + 255) / 256);
+  const int npad = STATS ? h->cell_npad : 0;
+  const int64_t cstride = cell_parts(h);
+  int *lc = h->lcount + 2 * h->lsel, *lnext = h->lcount + 2 * (1 - h->lsel);
+  int8_t *tin = h->tflags + (int64_t)h->lsel * ct, *tout = h->tflags + (int64_t)(1 - h->lsel) * ct;
+  h->lsel = 1 - h->lsel;
+  ProfScope ps(h, GP_KERNEL_CBULK);
+  hipLaunchKernelGGL((k_cbulk<N, NC, R, P2, STATS, SEG, C>), dim3(cblk + rblk + (npad + 3) / 4), dim3(256), 0, h->stream, m,
+                     (const R *)h->mu[b], (const int8_t *)h->codes[h->ccur], (R *)h->phi[o], (R *)h->mu[o],
+                     h->codes[1 - h->ccur], h->partials, cstride, h->fs, h->ps, mx, my, h->cell_nstrips, ct,
+                     (int)h->prev_valid, (const int8_t *)tin, tout, h->ilist, h->clist, lc, lnext, (int)cblk,
+                     (int)rblk, C ? (const int8_t *)c32_mlo(h, b) : (const int8_t *)nullptr,
+                     C ? c32_plo(h, o) : (float *)nullptr, C ? c32_mlo(h, o) : (int8_t *)nullptr);
+  return lc;
+}
+template <int N, int NC, typename R, bool P2, bool C>
+static int *launch_cbulk(gp_handle *h, const Model<R> *m, bool stats) {
+  const bool full = h->cell_seg == kCellSegMax;
+  if (stats)
+    return full ? launch_cbulk_seg<N, NC, R, P2, C, true, kCellSegMax>(h, m)
+                : launch_cbulk_seg<N, NC, R, P2, C, true, kCellSegMin>(h, m);
+  return full ? launch_cbulk_seg<N, NC, R, P2, C, false, kCellSegMax>(h, m)
+              : launch_cbulk_seg<N, NC, R, P2, C, false, kCellSegMin>(h, m);
+}
+
 template <int N, int NC, typename R, bool P2>
 static int launch_step_p(gp_handle *h, int mode) {
   const R *phi = (const R *)h->phi[h->cur], *mu = (const R *)h->mu[h->cur];
@@ -366,49 +403,28 @@ static int launch_step_p(gp_handle *h, int mode) {
     }
     if (h->use_cells) {
       /* statistics partials: k_cbulk's wavefronts, then k_ilist's */
-      const int ct = (int)h->cell_nwaves;
-      const unsigned cblk = (unsigned)((ct + 3) / 4);
       if (!h->lgrid_d) {
         h->lgrid_d = list_grid(h, k_dlist<N, NC, R, P2>);
         h->lgrid_i = list_grid(h, k_ilist<N, NC, R, P2, true>);
       }
-      const int64_t cstride = (int64_t)ct + 4 * h->lgrid_i;
-      /* this step's list lengths are zero (the previous step's k_cbulk, or the set-up, cleared them); this
-       * step's k_cbulk clears the other pair for the next step, which the previous step's kernels read */
-      int *lc = h->lcount + 2 * h->lsel, *lnext = h->lcount + 2 * (1 - h->lsel);
-      h->lsel = 1 - h->lsel;
-      /* k_cbulk's blocks past the tiles list the candidates of the boundary ring, one thread per ring cell */
-      const int64_t nring = 2 * (my + 2) + 2 * mx;
-      const unsigned rblk = (unsigned)((nring + 255) / 256);
-      {
-        ProfScope ps(h, GP_KERNEL_CBULK);
-        if (stats)
-          hipLaunchKernelGGL((k_cbulk<N, NC, R, P2, true>), dim3(cblk + rblk), dim3(256), 0, h->stream, m, mu, codes,
-                             phi_o, mu_o, codes_o, h->partials, cstride, h->fs, h->ps, mx, my, h->cell_seg,
-                             h->march_nstrips, ct, (int)h->prev_valid, h->ilist, h->clist, lc, lnext, (int)cblk,
-                             (const int8_t *)nullptr, (float *)nullptr, (int8_t *)nullptr);
-        else
-          hipLaunchKernelGGL((k_cbulk<N, NC, R, P2, false>), dim3(cblk + rblk), dim3(256), 0, h->stream, m, mu, codes,
-                             phi_o, mu_o, codes_o, h->partials, cstride, h->fs, h->ps, mx, my, h->cell_seg,
-                             h->march_nstrips, ct, (int)h->prev_valid, h->ilist, h->clist, lc, lnext, (int)cblk,
-                             (const int8_t *)nullptr, (float *)nullptr, (int8_t *)nullptr);
-      }
+      const int64_t cstride = cell_parts(h);
+      const int *lc = launch_cbulk<N, NC, R, P2, false>(h, m, stats);
       {
         /* delta-phi of the listed candidates, full wavefronts */
         ProfScope ps(h, GP_KERNEL_DPHI);
         hipLaunchKernelGGL((k_dlist<N, NC, R, P2>), dim3(h->lgrid_d), dim3(256), 0, h->stream, m, phi, mu, dphi,
-                           h->fs, h->ps, (const int32_t *)h->clist, (const int *)lc + 1);
+                           h->fs, h->ps, (const int32_t *)h->clist, lc + 1);
       }
       {
         ProfScope ps(h, GP_KERNEL_CIFACE);
         if (stats)
           hipLaunchKernelGGL((k_ilist<N, NC, R, P2, true>), dim3(h->lgrid_i), dim3(256), 0, h->stream, m, phi, mu,
-                             dphi, codes, phi_o, mu_o, codes_o, h->partials + ct, cstride, h->fs, h->ps,
-                             (const int32_t *)h->ilist, (const int *)lc);
+                             dphi, codes, phi_o, mu_o, codes_o, h->partials + cell_ipart(h), cstride, h->fs, h->ps,
+                             (const int32_t *)h->ilist, lc);
         else
           hipLaunchKernelGGL((k_ilist<N, NC, R, P2, false>), dim3(h->lgrid_i), dim3(256), 0, h->stream, m, phi, mu,
-                             dphi, codes, phi_o, mu_o, codes_o, h->partials + ct, cstride, h->fs, h->ps,
-                             (const int32_t *)h->ilist, (const int *)lc);
+                             dphi, codes, phi_o, mu_o, codes_o, h->partials + cell_ipart(h), cstride, h->fs, h->ps,
+                             (const int32_t *)h->ilist, lc);
       }
       /* the new state's halo, from the interior cells both kernels wrote; with the statistics fold when asked */
       const int64_t nh = halo_cells(mx, my);
@@ -714,45 +730,27 @@ static int launch_step_c(gp_handle *h, int mode) {
   if (!h->codes_valid)
     hipLaunchKernelGGL((k_c32_codes<N>), dim3((unsigned)((h->ry + 63) / 64), (unsigned)((h->rx + 3) / 4)), dim3(256),
                        0, h->stream, phi, plo, h->codes[h->ccur], fs, h->ps, h->rx, h->ry);
-  const int ct = (int)h->cell_nwaves;
-  const unsigned cblk = (unsigned)((ct + 3) / 4);
   if (!h->lgrid_d) {
     h->lgrid_d = list_grid(h, k_dlist_c<N, NC, P2>);
     h->lgrid_i = list_grid(h, k_ilist_c<N, NC, P2, true>);
   }
-  const int64_t cstride = (int64_t)ct + 4 * h->lgrid_i;
-  int *lc = h->lcount + 2 * h->lsel, *lnext = h->lcount + 2 * (1 - h->lsel);
-  h->lsel = 1 - h->lsel;
-  const int64_t nring = 2 * (my + 2) + 2 * mx;
-  const unsigned rblk = (unsigned)((nring + 255) / 256);
-  {
-    ProfScope ps(h, GP_KERNEL_CBULK);
-    if (stats)
-      hipLaunchKernelGGL((k_cbulk<N, NC, float, P2, true, true>), dim3(cblk + rblk), dim3(256), 0, h->stream, m, mu,
-                         codes, phi_o, mu_o, codes_o, h->partials, cstride, fs, h->ps, mx, my, h->cell_seg,
-                         h->march_nstrips, ct, (int)h->prev_valid, h->ilist, h->clist, lc, lnext, (int)cblk, mlo, plo_o,
-                         mlo_o);
-    else
-      hipLaunchKernelGGL((k_cbulk<N, NC, float, P2, false, true>), dim3(cblk + rblk), dim3(256), 0, h->stream, m, mu,
-                         codes, phi_o, mu_o, codes_o, h->partials, cstride, fs, h->ps, mx, my, h->cell_seg,
-                         h->march_nstrips, ct, (int)h->prev_valid, h->ilist, h->clist, lc, lnext, (int)cblk, mlo, plo_o,
-                         mlo_o);
-  }
+  const int64_t cstride = cell_parts(h);
+  const int *lc = launch_cbulk<N, NC, float, P2, true>(h, m, stats);
   {
     ProfScope ps(h, GP_KERNEL_DPHI);
     hipLaunchKernelGGL((k_dlist_c<N, NC, P2>), dim3(h->lgrid_d), dim3(256), 0, h->stream, md, phi, plo, mu, mlo, dphi,
-                       fs, h->ps, (const int32_t *)h->clist, (const int *)lc + 1);
+                       fs, h->ps, (const int32_t *)h->clist, lc + 1);
   }
   {
     ProfScope ps(h, GP_KERNEL_CIFACE);
     if (stats)
       hipLaunchKernelGGL((k_ilist_c<N, NC, P2, true>), dim3(h->lgrid_i), dim3(256), 0, h->stream, md, phi, plo, mu,
-                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, h->partials + ct,
-                         cstride, fs, h->ps, (const int32_t *)h->ilist, (const int *)lc);
+                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, h->partials + cell_ipart(h),
+                         cstride, fs, h->ps, (const int32_t *)h->ilist, lc);
     else
       hipLaunchKernelGGL((k_ilist_c<N, NC, P2, false>), dim3(h->lgrid_i), dim3(256), 0, h->stream, md, phi, plo, mu,
-                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, h->partials + ct,
-                         cstride, fs, h->ps, (const int32_t *)h->ilist, (const int *)lc);
+                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, h->partials + cell_ipart(h),
+                         cstride, fs, h->ps, (const int32_t *)h->ilist, lc);
   }
   const int64_t nh = halo_cells(mx, my);
   if (stats) {
