@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void k_dlist_c(const Model<double> *__restrict
     c32_gather<N, NC>(phi, plo, mu, mlo, c, fs, ps, false, rs);
     const RegView<N, NC, double, P2, true> v{&rs, 0, 0};
     double d[N];
-    phi_delta<N, NC>(*mp, v, false, d);
+    phi_delta_pairs<N, NC>(*mp, v, d);
 #pragma unroll
     for (int a = 0; a < N; a++) dphi[a * fs + c] = d[a];
   }
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256) void k_dlist_c(const Model<double> *__restrict
 /* The general update of the listed interface cells in FP64 from the decoded state (k_ilist's gather and
  * arithmetic), the new values encoded on store and their codes taken from the decoded stored values. */
 template <int N, int NC, bool P2, bool STATS>
-__global__ __launch_bounds__(256) void k_ilist_c(const Model<double> *__restrict__ mp, const float *__restrict__ phi,
+__global__ __launch_bounds__(256, 2) void k_ilist_c(const Model<double> *__restrict__ mp, const float *__restrict__ phi,
                                                  const float *__restrict__ plo, const float *__restrict__ mu,
                                                  const int8_t *__restrict__ mlo, const double *__restrict__ dphi,
                                                  const int8_t *__restrict__ codes_in, float *__restrict__ phi_o,
@@ -191,10 +191,7 @@ __global__ __launch_bounds__(256) void k_ilist_c(const Model<double> *__restrict
     }
     const RegView<N, NC, double, P2, true> v{&rs, 0, 0};
     double jx0[NC], jxb[NC], jy0[NC], jyl[NC], d[N], pn[N], mn[NC], dm[NC];
-    jat_x<N, NC>(m, v, 0, 0, jx0);
-    jat_x<N, NC>(m, v, -1, 0, jxb);
-    jat_y<N, NC>(m, v, 0, 0, y, jy0);
-    jat_y<N, NC>(m, v, 0, -1, y - 1, jyl);
+    jat_faces<N, NC>(m, v, y, jx0, jxb, jy0, jyl);
 #pragma unroll
     for (int a = 0; a < N; a++) d[a] = v.dp(a, 0, 0);
     mu_update<N, NC>(m, v, false, d, jx0, jxb, jy0, jyl, pn, mn, dm);

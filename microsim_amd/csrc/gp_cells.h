@@ -681,7 +681,7 @@ __global__ __launch_bounds__(256) void k_halo(R *__restrict__ phi, R *__restrict
  * delta-phi values are k_dphi's (candidates) and which are exactly 0. Statistics: one partial per wavefront of the
  * grid (the grid is fixed, the order of the cells within it is not). */
 template <int N, int NC, typename R, bool P2, bool STATS>
-__global__ __launch_bounds__(256) void k_ilist(const Model<R> *__restrict__ mp, const R *__restrict__ phi,
+__global__ __launch_bounds__(256, 2) void k_ilist(const Model<R> *__restrict__ mp, const R *__restrict__ phi,
                                                const R *__restrict__ mu, const R *__restrict__ dphi,
                                                const int8_t *__restrict__ codes_in, R *__restrict__ phi_o,
                                                R *__restrict__ mu_o, int8_t *__restrict__ codes_out,
@@ -731,10 +731,14 @@ __global__ __launch_bounds__(256) void k_ilist(const Model<R> *__restrict__ mp, 
     }
     const RegView<N, NC, R, P2, kFastOf<R>> v{&rs, 0, 0};
     R jx0[NC], jxb[NC], jy0[NC], jyl[NC], d[N], pn[N], mn[NC], dm[NC];
-    jat_x<N, NC>(m, v, 0, 0, jx0);
-    jat_x<N, NC>(m, v, -1, 0, jxb);
-    jat_y<N, NC>(m, v, 0, 0, y, jy0);
-    jat_y<N, NC>(m, v, 0, -1, y - 1, jyl);
+    if constexpr (kBySolids<R>) {
+      jat_faces<N, NC>(m, v, y, jx0, jxb, jy0, jyl);
+    } else {
+      jat_x<N, NC>(m, v, 0, 0, jx0);
+      jat_x<N, NC>(m, v, -1, 0, jxb);
+      jat_y<N, NC>(m, v, 0, 0, y, jy0);
+      jat_y<N, NC>(m, v, 0, -1, y - 1, jyl);
+    }
 #pragma unroll
     for (int a = 0; a < N; a++) d[a] = v.dp(a, 0, 0);
     mu_update<N, NC>(m, v, false, d, jx0, jxb, jy0, jyl, pn, mn, dm);

@@ -26,6 +26,7 @@
 
 #include "gp_common.h"
 #include "gp_model.h"
+#include "gp_pairs.h"
 
 namespace gpk {
 
@@ -844,7 +845,7 @@ __global__ __launch_bounds__(256) void k_codes(const R *__restrict__ phi, int8_t
  * projection) for 64 candidates at a time, so every lane works on an interface cell. */
 constexpr int kDTileRows = 16;
 
-/* phi on the 3x3 stencil and mu at the centre gathered once into registers, then phi_delta */
+/* phi on the 3x3 stencil and mu at the centre gathered once into registers, then delta-phi */
 template <int N, int NC, typename R, bool P2>
 __device__ __forceinline__ void dphi_cell(const Model<R> &m, const R *__restrict__ phi, const R *__restrict__ mu,
                                           R *__restrict__ dphi, int64_t fs, int64_t ps, int64_t c) {
@@ -859,7 +860,8 @@ __device__ __forceinline__ void dphi_cell(const Model<R> &m, const R *__restrict
   for (int k = 0; k < NC; k++) rs.u[k][0] = mu[k * fs + c];
   const RegView<N, NC, R, P2, kFastOf<R>> v{&rs, 0, 0};
   R d[N];
-  phi_delta<N, NC>(m, v, false, d);
+  if constexpr (kByPairs<R, P2>) phi_delta_pairs<N, NC>(m, v, d);
+  else phi_delta<N, NC>(m, v, false, d);
 #pragma unroll
   for (int a = 0; a < N; a++) dphi[a * fs + c] = d[a];
 }

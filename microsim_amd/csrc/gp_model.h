@@ -53,7 +53,8 @@ struct Model {
   R inv_eps;     /* 1.0/epsilon */
   R two_dy;      /* 2.0*deltay */
   R inv_dx, inv_dy, inv_2dy; /* exact reciprocals when dx, dy are powers of two (pow2 != 0) */
-  int32_t pow2, pad2;
+  int32_t pow2;
+  int32_t pairs_sym; /* the pair coefficients are finite and equal for (a, b) and (b, a) (gp_pairs.h) */
   R w_obst;      /* 16.0/(M_PI*M_PI) */
   R jat_well;    /* 0.5/sqrt(2.0) */
   R jat_fac;     /* -0.25*M_PI*epsilon (obstacle) or -1.0*epsilon (well) */
@@ -1071,6 +1072,20 @@ inline int make_model(const gp_params *p, Model<R> *m) {
           m->rot[a][b][i][j] = (R)p->rot[((a * P + b) * 2 + i) * 2 + j];
           m->rot_inv[a][b][i][j] = (R)p->rot_inv[((a * P + b) * 2 + i) * 2 + j];
         }
+    }
+  m->pairs_sym = 1;
+  auto same = [&](double x, double y) {
+    if (!(x == y && fabs(x) <= 3.0e38)) m->pairs_sym = 0; /* finite in either precision */
+  };
+  for (int a = 0; a < N; a++)
+    for (int b = a + 1; b < N; b++) {
+      const int ab = a * P + b, ba = b * P + a;
+      same(p->gamma[ab], p->gamma[ba]);
+      same(p->dab[ab], p->dab[ba]);
+      for (int i = 0; i < 4; i++) {
+        same(p->rot[ab * 4 + i], p->rot[ba * 4 + i]);
+        same(p->rot_inv[ab * 4 + i], p->rot_inv[ba * 4 + i]);
+      }
     }
   for (int a = 0; a < P; a++) {
     for (int i = 0; i < NCM; i++) {
