@@ -21,6 +21,7 @@
 #include <mutex>
 
 #include "gp_internal.h"
+#include "gp_pack.h"
 #include "gp_adjoint.h"
 #include "gp_cells.h"
 
@@ -119,64 +120,85 @@ static void stats_reset_host(gp_handle *h, double *s) {
   s[3 * N + 3 * NC] = 0.0;
 }
 
-/* halo-inclusive host planes (rows_x*rows_y, y fastest) -> device planes, with the BC maps applied; in GP_FP32C
- * each value is encoded into its FP32 part (dst) and its second part (dst_lo: the FP32 low part of phi, field 0,
- * or the 8-bit extension of mu, field 1) */
-static int upload_planes(gp_handle *h, void *dst, void *dst_lo, const double *src, int ncomp, int field) {
-  const int64_t rx = h->rx, ry = h->ry, n = rx * ry;
-  std::vector<double> tmp(src, src + (size_t)ncomp * n);
-  const int64_t hx[6] = {0, 1, 2, rx - 3, rx - 2, rx - 1}, hy[6] = {0, 1, 2, ry - 3, ry - 2, ry - 1};
-  for (int c = 0; c < ncomp; c++) {
-    double *v = tmp.data() + (size_t)c * n;
-    for (int s = 0; s < 6; s++)
-      for (int64_t y = 0; y < ry; y++) v[hx[s] * ry + y] = v[(int64_t)h->p.halo_src_x[field][s] * ry + y];
-    for (int s = 0; s < 6; s++)
-      for (int64_t x = 0; x < rx; x++) v[x * ry + hy[s]] = v[x * ry + h->p.halo_src_y[field][s]];
+/* grid of the layout kernels: 256 elements of a row by rows (a stride loop past the limit of the y dimension) */
+static dim3 pack_grid(int64_t width, int64_t nrows) {
+  return dim3((unsigned)((width + 255) / 256), (unsigned)std::min<int64_t>(nrows, 32768));
+}
+
+/* `rows` rows of ry doubles go through the staging buffer in runs of whole rows: step(first row, rows, staging) enqueues a
+ * run's copy and kernel on the handle's stream, in order, so that a run reuses the buffer after the one before it */
+template <class F>
+static int staged_rows(gp_handle *h, int64_t rows, F step) {
+  const int64_t per = std::max<int64_t>(1, (int64_t)(h->stage_bytes / ((size_t)h->ry * sizeof(double))));
+  for (int64_t r = 0; r < rows; r += per) {
+    const int rc = step(r, std::min(per, rows - r), (double *)h->clist);
+    if (rc) return rc;
   }
-  const size_t es = esize(h);
-  std::vector<char> stage((size_t)ncomp * h->fs * es, 0);
-  const size_t les = field == 0 ? sizeof(float) : 1;
-  std::vector<char> stage_lo(h->precision == GP_FP32C ? (size_t)ncomp * h->fs * les : 0, 0);
-  for (int c = 0; c < ncomp; c++)
-    for (int64_t x = 0; x < rx; x++)
-      for (int64_t y = 0; y < ry; y++) {
-        const double v = tmp[(size_t)c * n + x * ry + y];
-        const size_t o = ((size_t)c * h->fs + x * h->ps + y + kYOff);
-        if (h->precision == GP_FP64) ((double *)stage.data())[o] = v;
-        else if (h->precision == GP_FP32C && field == 0) df_encode(v, ((float *)stage.data())[o], ((float *)stage_lo.data())[o]);
-        else if (h->precision == GP_FP32C) c32_encode(v, ((float *)stage.data())[o], ((int8_t *)stage_lo.data())[o]);
-        else ((float *)stage.data())[o] = (float)v;
-      }
-  HIPCHK(h, hipMemcpyAsync(dst, stage.data(), stage.size(), hipMemcpyHostToDevice, h->stream));
-  if (h->precision == GP_FP32C)
-    HIPCHK(h, hipMemcpyAsync(dst_lo, stage_lo.data(), stage_lo.size(), hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return GP_OK;
 }
 
-/* device planes -> halo-inclusive host planes. es: element size of the planes (8: FP64, 4: FP32); src_lo: the
- * GP_FP32C second parts of FP32 planes (decoded into the values: FP32 low parts of phi, field 0, or 8-bit
- * extensions of mu, field 1), or NULL */
-static int download_planes(gp_handle *h, double *dst, const void *src, const void *src_lo, int field, int ncomp,
-                           size_t es) {
-  const int64_t rx = h->rx, ry = h->ry, n = rx * ry;
-  std::vector<char> stage((size_t)ncomp * h->fs * es);
-  const size_t les = field == 0 ? sizeof(float) : 1;
-  std::vector<char> stage_lo(src_lo ? (size_t)ncomp * h->fs * les : 0);
-  HIPCHK(h, hipMemcpyAsync(stage.data(), src, stage.size(), hipMemcpyDeviceToHost, h->stream));
-  if (src_lo) HIPCHK(h, hipMemcpyAsync(stage_lo.data(), src_lo, stage_lo.size(), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  for (int c = 0; c < ncomp; c++)
-    for (int64_t x = 0; x < rx; x++)
-      for (int64_t y = 0; y < ry; y++) {
-        const size_t o = ((size_t)c * h->fs + x * h->ps + y + kYOff);
-        double v;
-        if (es == sizeof(double)) v = ((double *)stage.data())[o];
-        else if (src_lo && field == 0) v = df_decode(((float *)stage.data())[o], ((float *)stage_lo.data())[o]);
-        else if (src_lo) v = c32_decode(((float *)stage.data())[o], ((int8_t *)stage_lo.data())[o]);
-        else v = (double)((float *)stage.data())[o];
-        dst[(size_t)c * n + x * ry + y] = v;
-      }
+/* halo-inclusive host planes of a field (0: phi, 1: mu) -> the planes d0 and d1 (unless NULL) in the given form (second
+ * parts l0, l1); the halo as the host holds it */
+static int rows_to_device(gp_handle *h, int form, void *d0, void *d1, void *l0, void *l1, const double *src, int ncomp) {
+  const int64_t ry = h->ry, ps = h->ps;
+  return staged_rows(h, ncomp * h->rx, [&](int64_t r, int64_t n, double *st) -> int {
+    HIPCHK(h, hipMemcpyAsync(st, src + r * ry, (size_t)(n * ry) * sizeof(double), hipMemcpyHostToDevice, h->stream));
+    const dim3 g = pack_grid(ps, n), b(256);
+    if (form == PACK_F64) hipLaunchKernelGGL((k_pack<PACK_F64>), g, b, 0, h->stream, st, d0, d1, l0, l1, r, n, ry, ps);
+    else if (form == PACK_F32) hipLaunchKernelGGL((k_pack<PACK_F32>), g, b, 0, h->stream, st, d0, d1, l0, l1, r, n, ry, ps);
+    else if (form == PACK_DF) hipLaunchKernelGGL((k_pack<PACK_DF>), g, b, 0, h->stream, st, d0, d1, l0, l1, r, n, ry, ps);
+    else hipLaunchKernelGGL((k_pack<PACK_C32>), g, b, 0, h->stream, st, d0, d1, l0, l1, r, n, ry, ps);
+    HIPCHK(h, hipGetLastError());
+    return GP_OK;
+  });
+}
+
+/* device planes -> halo-inclusive host planes, decoded from the given form (second parts l) */
+static int rows_to_host(gp_handle *h, int form, double *dst, const void *s, const void *l, int ncomp) {
+  const int64_t ry = h->ry, ps = h->ps;
+  return staged_rows(h, ncomp * h->rx, [&](int64_t r, int64_t n, double *st) -> int {
+    const dim3 g = pack_grid(ry, n), b(256);
+    if (form == PACK_F64) hipLaunchKernelGGL((k_unpack<PACK_F64>), g, b, 0, h->stream, st, s, l, r, n, ry, ps);
+    else if (form == PACK_F32) hipLaunchKernelGGL((k_unpack<PACK_F32>), g, b, 0, h->stream, st, s, l, r, n, ry, ps);
+    else if (form == PACK_DF) hipLaunchKernelGGL((k_unpack<PACK_DF>), g, b, 0, h->stream, st, s, l, r, n, ry, ps);
+    else hipLaunchKernelGGL((k_unpack<PACK_C32>), g, b, 0, h->stream, st, s, l, r, n, ry, ps);
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, hipMemcpyAsync(dst + r * ry, st, (size_t)(n * ry) * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    return GP_OK;
+  });
+}
+
+/* the stored form of field f of the handle's states */
+static int field_form(const gp_handle *h, int f) {
+  return h->precision == GP_FP64 ? PACK_F64 : h->precision == GP_FP32 ? PACK_F32 : f == 0 ? PACK_DF : PACK_C32;
+}
+
+/* field f of a host state into both state buffers, with the boundary copies */
+static int upload_field(gp_handle *h, int f, const double *src) {
+  const int ncomp = f == 0 ? h->N : h->NC, form = field_form(h, f);
+  const int64_t mx = h->p.mesh_x, my = h->p.mesh_y;
+  void *d[2], *l[2] = {nullptr, nullptr};
+  for (int b = 0; b < 2; b++) {
+    d[b] = f == 0 ? h->phi[b] : h->mu[b];
+    if (h->precision == GP_FP32C) l[b] = f == 0 ? (void *)c32_plo(h, b) : (void *)c32_mlo(h, b);
+  }
+  const int rc = rows_to_device(h, form, d[0], d[1], l[0], l[1], src, ncomp);
+  if (rc) return rc;
+  const dim3 g((unsigned)((6 * (my + 6) + 6 * mx + 255) / 256), (unsigned)ncomp), b(256);
+  if (form == PACK_F64)
+    hipLaunchKernelGGL((k_pack_halo<double>), g, b, 0, h->stream, (double *)d[0], (double *)d[1], h->maps, f, h->fs,
+                       h->ps, mx, my);
+  else
+    hipLaunchKernelGGL((k_pack_halo<float>), g, b, 0, h->stream, (float *)d[0], (float *)d[1], h->maps, f, h->fs, h->ps,
+                       mx, my);
+  if (form == PACK_DF)
+    hipLaunchKernelGGL((k_pack_halo<float>), g, b, 0, h->stream, (float *)l[0], (float *)l[1], h->maps, f, h->fs, h->ps,
+                       mx, my);
+  else if (form == PACK_C32)
+    hipLaunchKernelGGL((k_pack_halo<int8_t>), g, b, 0, h->stream, (int8_t *)l[0], (int8_t *)l[1], h->maps, f, h->fs,
+                       h->ps, mx, my);
+  HIPCHK(h, hipGetLastError());
   return GP_OK;
 }
 
@@ -224,21 +246,6 @@ static int state_load(gp_handle *h, const double *src) {
   h->flags_valid = false;
   h->codes_valid = false;
   h->prev_valid = false;
-  return GP_OK;
-}
-
-/* halo-inclusive host planes (rows_x*rows_y, y fastest) <-> device planes, without boundary copies: one strided
- * copy (the planes are rows_x rows apart on both sides) */
-static int planes_to_device(gp_handle *h, double *dst, const double *src, int ncomp) {
-  HIPCHK(h, hipMemcpy2DAsync(dst + kYOff, h->ps * sizeof(double), src, h->ry * sizeof(double), h->ry * sizeof(double),
-                             (size_t)ncomp * h->rx, hipMemcpyHostToDevice, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  return GP_OK;
-}
-static int planes_to_host(gp_handle *h, double *dst, const double *src, int ncomp) {
-  HIPCHK(h, hipMemcpy2DAsync(dst, h->ry * sizeof(double), src + kYOff, h->ps * sizeof(double), h->ry * sizeof(double),
-                             (size_t)ncomp * h->rx, hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
   return GP_OK;
 }
 
@@ -496,9 +503,13 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
   ok = ok && hipMalloc((void **)&h->flags[0], sizeof(int) * h->march_nwaves) == hipSuccess;
   ok = ok && hipMalloc((void **)&h->flags[1], sizeof(int) * h->march_nwaves) == hipSuccess;
   ok = ok && hipMalloc((void **)&h->tflags, 2 * (size_t)h->cell_nwaves) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->clist, (size_t)h->fs * sizeof(int32_t)) == hipSuccess &&
-       hipMalloc((void **)&h->ilist, (size_t)h->fs * sizeof(int32_t)) == hipSuccess &&
-       hipMalloc((void **)&h->lcount, 4 * sizeof(int)) == hipSuccess;
+  /* the two cell lists in one piece (8 bytes a cell): between steps it stages the rows of uploads and downloads, the phi
+   * planes of a small grid in one run */
+  h->stage_bytes = std::max((size_t)h->fs * 2 * sizeof(int32_t),
+                            std::min((size_t)h->N * h->fs * sizeof(double), kStageBytes));
+  ok = ok && hipMalloc((void **)&h->clist, h->stage_bytes) == hipSuccess;
+  h->ilist = ok ? h->clist + h->fs : nullptr;
+  ok = ok && hipMalloc((void **)&h->lcount, 4 * sizeof(int)) == hipSuccess;
   ok = ok && hipMalloc((void **)&h->codes[0], (size_t)h->rx * h->ps) == hipSuccess &&
        hipMalloc((void **)&h->codes[1], (size_t)h->rx * h->ps) == hipSuccess;
   h->ccur = 0;
@@ -583,7 +594,7 @@ void gp_destroy(gp_handle *h) {
   delete h->adj;
   void *bufs[] = {h->phi[0], h->phi[1], h->mu[0],    h->mu[1],    h->dphi,   h->partials, h->stats_dev,
                   h->model,  h->flags[0], h->flags[1], h->inv_dev, h->codes[0], h->codes[1], h->clist,
-                  h->ilist,  h->lcount, h->lo[0],    h->lo[1],    h->model64, h->wide[0],  h->wide[1],
+                  h->lcount,  h->lo[0],    h->lo[1],    h->model64, h->wide[0],  h->wide[1],
                   h->trow,   h->thp,    h->thc,      h->front,    h->tflags};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
@@ -593,15 +604,8 @@ void gp_destroy(gp_handle *h) {
 
 int gp_upload(gp_handle *h, const double *phi, const double *mu) {
   if (!h || !phi || !mu) return h ? gp_fail(h, GP_E_ARG, "null argument") : GP_E_ARG;
-  const bool c = h->precision == GP_FP32C;
-  int rc = upload_planes(h, h->phi[h->cur], c ? (void *)c32_plo(h, h->cur) : nullptr, phi, h->N, 0);
-  if (rc) return rc;
-  rc = upload_planes(h, h->mu[h->cur], c ? (void *)c32_mlo(h, h->cur) : nullptr, mu, h->NC, 1);
-  if (rc) return rc;
-  /* the other copy starts identical so its halo rows are defined */
-  HIPCHK(h, hipMemcpyAsync(h->phi[1 - h->cur], h->phi[h->cur], (size_t)h->N * h->fs * esize(h), hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(h->mu[1 - h->cur], h->mu[h->cur], (size_t)h->NC * h->fs * esize(h), hipMemcpyDeviceToDevice, h->stream));
-  if (c) HIPCHK(h, hipMemcpyAsync(h->lo[1 - h->cur], h->lo[h->cur], c32_lo_bytes(h), hipMemcpyDeviceToDevice, h->stream));
+  int rc;
+  if ((rc = upload_field(h, 0, phi)) || (rc = upload_field(h, 1, mu))) return rc;
   HIPCHK(h, hipMemsetAsync(h->dphi, 0, (size_t)h->N * h->fs * dphi_esize(h), h->stream));
   double s[kNStatMax] = {0};
   stats_reset_host(h, s);
@@ -619,14 +623,15 @@ int gp_download(gp_handle *h, double *phi, double *mu, double *dphi) {
   int rc;
   const bool c = h->precision == GP_FP32C;
   const void *plo = c ? (const void *)c32_plo(h, h->cur) : nullptr, *mlo = c ? (const void *)c32_mlo(h, h->cur) : nullptr;
-  if (phi && (rc = download_planes(h, phi, h->phi[h->cur], plo, 0, h->N, esize(h)))) return rc;
-  if (mu && (rc = download_planes(h, mu, h->mu[h->cur], mlo, 1, h->NC, esize(h)))) return rc;
+  if (phi && (rc = rows_to_host(h, field_form(h, 0), phi, h->phi[h->cur], plo, h->N))) return rc;
+  if (mu && (rc = rows_to_host(h, field_form(h, 1), mu, h->mu[h->cur], mlo, h->NC))) return rc;
   if (dphi) {
     if (h->prev_valid) {
       /* single-pass steps do not store delta-phi: recompute the last step's from the previous state */
       if ((rc = h->ops->step(h, MODE_DPHI_PREV))) return rc;
     }
-    if ((rc = download_planes(h, dphi, h->dphi, nullptr, 0, h->N, dphi_esize(h)))) return rc;
+    const int form = dphi_esize(h) == sizeof(double) ? PACK_F64 : PACK_F32;
+    if ((rc = rows_to_host(h, form, dphi, h->dphi, nullptr, h->N))) return rc;
   }
   return GP_OK;
 }
@@ -843,9 +848,8 @@ int gp_adjoint_backward(gp_handle *h, const double *gphi_T, const double *gmu_T,
     if (!ok) return gp_fail(h, GP_E_OOM, "adjoint: buffers do not fit in device memory");
   }
   int rc;
-  HIPCHK(h, hipMemsetAsync(A->g[1], 0, se * sizeof(double), h->stream));
-  if ((rc = planes_to_device(h, A->g[1], gphi_T, h->N))) return rc;
-  if ((rc = planes_to_device(h, A->g[1] + (size_t)h->N * h->fs, gmu_T, h->NC))) return rc;
+  if ((rc = rows_to_device(h, PACK_F64, A->g[1], nullptr, nullptr, nullptr, gphi_T, h->N))) return rc;
+  if ((rc = rows_to_device(h, PACK_F64, A->g[1] + (size_t)h->N * h->fs, nullptr, nullptr, nullptr, gmu_T, h->NC))) return rc;
   HIPCHK(h, hipMemsetAsync(A->gth, 0, sizeof(double) * nth, h->stream));
   step_fn f = h->ops->step;
   adj_fn fa = h->ops->adj_step;
@@ -884,8 +888,8 @@ int gp_adjoint_backward(gp_handle *h, const double *gphi_T, const double *gmu_T,
     }
   }
   if ((rc = adj_fold(h))) return rc;
-  if ((rc = planes_to_host(h, gphi_0, A->g[1], h->N))) return rc;
-  if ((rc = planes_to_host(h, gmu_0, A->g[1] + (size_t)h->N * h->fs, h->NC))) return rc;
+  if ((rc = rows_to_host(h, PACK_F64, gphi_0, A->g[1], nullptr, h->N))) return rc;
+  if ((rc = rows_to_host(h, PACK_F64, gmu_0, A->g[1] + (size_t)h->N * h->fs, nullptr, h->NC))) return rc;
   HIPCHK(h, hipMemcpyAsync(gtheta, A->gth, sizeof(double) * nth, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   h->steps = 0; /* the handle holds the initial state again */

@@ -37,6 +37,7 @@ constexpr int kNStatMax = 3 * GP_MAXP + 3 * GP_MAXNC + 1;
 #define GP_LIST_BLOCKS 2048
 #endif
 constexpr int kListBlocks = GP_LIST_BLOCKS; /* largest grid of the list-driven kernels (grid-stride loops), 4 wavefronts each */
+constexpr size_t kStageBytes = 32u << 20; /* bytes of host rows a handle stages at once, unless its cell lists are larger */
 #ifndef GP_ADJ_BLOCKS
 #define GP_ADJ_BLOCKS 1024
 #endif
@@ -83,7 +84,8 @@ struct gp_handle {
   int64_t cell_nwaves;
   int cell_npad;             /* wavefronts of the statistics' padding rows (none when mesh_x is a multiple of four) */
   int8_t *tflags;            /* its tile flags of two alternating steps (by lsel) */
-  int32_t *clist, *ilist;    /* delta-phi candidates and interface cells of the current step (cell offsets) */
+  int32_t *clist, *ilist;    /* delta-phi candidates and interface cells of the current step (cell offsets), one allocation */
+  size_t stage_bytes;        /* its bytes: between steps it stages host rows (gp_pack.h) */
   int *lcount;               /* their lengths: two pairs, used by alternate steps (lcount + 2 * lsel) */
   int lsel;
   int lgrid_d, lgrid_i;      /* grids of this handle's delta-phi and interface list kernels (0: not yet set) */
