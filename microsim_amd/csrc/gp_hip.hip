@@ -316,7 +316,7 @@ static int adj_fold(gp_handle *h) {
 
 /* temperature of allocated row 0 and the gradient per row, as the serial driver forms them before the loop (t = 0,
  * GPs/microsim_gp.c:77-80) and after step t (:108-111) */
-static double frame_bottom(const gp_handle *h, int64_t t, double *grad) {
+double gp_frame_bottom(const gp_handle *h, int64_t t, double *grad) {
   const gp_params *p = &h->p;
   const double G = (p->tg_deltaT) * p->dy / (p->tg_distance);
   double base;
@@ -330,9 +330,10 @@ static double frame_bottom(const gp_handle *h, int64_t t, double *grad) {
  * before the loop (GPs/microsim_gp.c:81-84) */
 static int frame_reset(gp_handle *h) {
   h->shift_off = 0;
+  h->thermo_valid = false;
   if (!h->p.tempgrady) return GP_OK;
   double G;
-  const double tb = frame_bottom(h, 0, &G);
+  const double tb = gp_frame_bottom(h, 0, &G);
   std::vector<double> T((size_t)h->ry);
   for (int64_t y = 0; y < h->ry; y++) T[y] = tb + (double)y * G;
   for (int k = 0; k < 6; k++) T[h->tp.hy[k]] = T[h->tp.srcT[k]];
@@ -341,15 +342,8 @@ static int frame_reset(gp_handle *h) {
   return GP_OK;
 }
 
-/* after step t: the new temperature gradient, and every 100 steps the moving frame */
+/* after step t (which has set the new temperature gradient): every 100 steps the moving frame */
 static int frame_after_step(gp_handle *h, int64_t t) {
-  if (h->p.tempgrady) {
-    double G;
-    const double tb = frame_bottom(h, t, &G);
-    hipLaunchKernelGGL(k_trow_set, dim3((unsigned)((h->ry + 255) / 256)), dim3(256), 0, h->stream, h->trow, h->ry, tb,
-                       G);
-    HIPCHK(h, hipGetLastError());
-  }
   if (!h->p.shift || t % 100 != 0) return GP_OK;
   const int N = h->N, NC = h->NC, L = N - 1;
   const size_t es = esize(h);
@@ -394,6 +388,7 @@ static int frame_after_step(gp_handle *h, int64_t t) {
     HIPCHK(h, hipStreamSynchronize(h->stream));
   }
   h->shift_off += sh;
+  h->thermo_valid = false;
   h->codes_valid = false;
   h->flags_valid = false;
   h->prev_valid = false;

@@ -68,6 +68,7 @@ struct gp_handle {
    * (device) and the cells the frame has moved since gp_upload */
   double *trow;
   void *thp, *thc;
+  bool thermo_valid;        /* thp, thc hold the coefficients of trow */
   int *front;
   int64_t shift_off;
   gpk::ThermoParams tp;
@@ -133,6 +134,9 @@ struct ProfScope {
     e0 = e1 = nullptr;
   }
 };
+
+/* temperature of allocated row 0 and the gradient per row after step t (t = 0: before the loop) */
+double gp_frame_bottom(const gp_handle *h, int64_t t, double *grad);
 
 /* record the message of a failing call on h (or of gp_create when h is NULL) and return code */
 int gp_fail(gp_handle *h, int code, const char *fmt, ...);

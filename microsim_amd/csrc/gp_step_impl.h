@@ -177,6 +177,28 @@ __global__ __launch_bounds__(kStatThreads) void k_stats(const double *__restrict
   stats_fold_block<N, NC>(partials, stride, nparts, cum, (int)blockIdx.x);
 }
 
+/* The statistics fold of a non-isothermal step and, in the blocks past it, the row temperatures after the step
+ * (bottom + y grad, Temperature_gradient.h) with their coefficients for the next one: a block takes kStatThreads rows of
+ * one phase and sweep (the fold leaves most of the chip idle, and both are chains of a few memory accesses). */
+template <int N, int NC, typename R>
+__global__ __launch_bounds__(kStatThreads) void k_stats_thermo(const double *__restrict__ partials, int64_t stride,
+                                                               int64_t nparts, double *__restrict__ cum, ThermoParams tp,
+                                                               double *__restrict__ trow, RowThermo<R> *__restrict__ thp,
+                                                               RowThermo<R> *__restrict__ thc, int64_t ry, double bottom,
+                                                               double grad) {
+  constexpr int NS = 3 * N + 3 * NC + 1;
+  if ((int)blockIdx.x < NS) {
+    stats_fold_block<N, NC>(partials, stride, nparts, cum, (int)blockIdx.x);
+    return;
+  }
+  const int q = (int)blockIdx.x - NS, a = (q >> 1) % N, sweep = q & 1;
+  const int64_t y = (int64_t)(q / (2 * N)) * kStatThreads + threadIdx.x;
+  if (y >= ry) return;
+  const auto T = [&](int64_t r) { return bottom + (double)r * grad; };
+  if (a == 0 && sweep == 0) trow[y] = T(y);
+  thermo_cell<N, NC, R>(tp, T, a, sweep, y, thp, thc);
+}
+
 /* The statistics fold and the halo pass of the cell-classified step in one launch (both small and latency-bound,
  * and independent: the fold reads the partials, the halo pass the new state): blocks below the number of
  * statistics fold one statistic each, the others copy kStatThreads halo cells of one plane each (k_halo). */
@@ -366,15 +388,11 @@ static int launch_step_p(gp_handle *h, int mode) {
   const bool tg = h->p.tempgrady != 0;
   const RowThermo<R> *thp = (const RowThermo<R> *)h->thp, *thc = (const RowThermo<R> *)h->thc;
   if (mode == MODE_DPHI_PREV) {
-    /* delta-phi of the last step, recomputed from the previous state (still in the other buffer; non-isothermal
-     * runs: with the last step's row coefficients) */
+    /* delta-phi of the last step, recomputed from the previous state (still in the other buffer). Single-pass steps only,
+     * so never a non-isothermal run: its two sweeps store delta-phi. */
     const R *pp = (const R *)h->phi[1 - h->cur], *mp = (const R *)h->mu[1 - h->cur];
-    if (tg)
-      hipLaunchKernelGGL((k_phi<N, NC, R, false, P2, true>), g1, blk, 0, h->stream, m, pp, mp, dphi, h->fs, h->ps,
-                         mx, my, thp);
-    else
-      hipLaunchKernelGGL((k_phi<N, NC, R, false, P2>), g1, blk, 0, h->stream, m, pp, mp, dphi, h->fs, h->ps, mx, my,
-                         (const RowThermo<R> *)nullptr);
+    hipLaunchKernelGGL((k_phi<N, NC, R, false, P2>), g1, blk, 0, h->stream, m, pp, mp, dphi, h->fs, h->ps, mx, my,
+                       (const RowThermo<R> *)nullptr);
     HIPCHK(h, hipGetLastError());
     return GP_OK;
   }
@@ -489,9 +507,11 @@ static int launch_step_p(gp_handle *h, int mode) {
   h->flags_valid = false; /* the two-pass kernels form neither tile flags nor phase codes */
   h->codes_valid = false;
   if (tg) {
-    /* non-isothermal: this step's row coefficients, then the two sweeps with them */
-    hipLaunchKernelGGL((k_thermo<R>), dim3((unsigned)((h->ry + 255) / 256)), dim3(256), 0, h->stream, h->tp, h->trow,
-                       (RowThermo<R> *)h->thp, (RowThermo<R> *)h->thc, h->ry);
+    /* non-isothermal: this step's row coefficients (unless the step before formed them), then the two sweeps with them */
+    if (!h->thermo_valid)
+      hipLaunchKernelGGL((k_thermo<N, NC, R>), dim3((unsigned)((h->ry + 255) / 256), 2 * N), dim3(256), 0, h->stream,
+                         h->tp, h->trow, (RowThermo<R> *)h->thp, (RowThermo<R> *)h->thc, h->ry);
+    h->thermo_valid = true;
     {
       ProfScope ps(h, GP_KERNEL_PHI);
       if (smooth)
@@ -511,9 +531,14 @@ static int launch_step_p(gp_handle *h, int mode) {
                            h->maps, h->partials, h->fs, h->ps, mx, my, thc);
     }
     if (!smooth) {
+      /* with the temperature gradient after this step, which the next one reads */
       ProfScope ps(h, GP_KERNEL_STATS);
-      hipLaunchKernelGGL((k_stats<N, NC>), dim3(3 * N + 3 * NC + 1), dim3(kStatThreads), 0, h->stream,
-                         h->partials, h->nblocks_mu, h->nblocks_mu, h->stats_dev);
+      double G;
+      const double tb = gp_frame_bottom(h, h->steps + 1, &G);
+      const int64_t nchunk = (h->ry + kStatThreads - 1) / kStatThreads;
+      hipLaunchKernelGGL((k_stats_thermo<N, NC, R>), dim3((unsigned)(3 * N + 3 * NC + 1 + 2 * N * nchunk)),
+                         dim3(kStatThreads), 0, h->stream, h->partials, h->nblocks_mu, h->nblocks_mu, h->stats_dev, h->tp,
+                         h->trow, (RowThermo<R> *)h->thp, (RowThermo<R> *)h->thc, h->ry, tb, G);
     }
     HIPCHK(h, hipGetLastError());
     h->cur = 1 - h->cur;
