@@ -101,4 +101,123 @@ __device__ __forceinline__ float wave_min(float v) {
   return dpp::reduce<float>(v, INFINITY, [](float a, float b) { return fminf(a, b); });
 }
 
+/* Many wavefront reductions at once. Reduced one by one, M values take M times six steps of two registers; here the
+ * first step (v_permlane32_swap) halves the lanes and packs two values into one register, the second
+ * (v_permlane16_swap) two of those, and the four steps within a row of 16 lanes then work on four values at a time:
+ * 16 statistics take about 130 instructions instead of 650, and leave with one store each for the extrema and the sums.
+ * out[j] holds value 4 j + row_value(lane) of v in every lane of a row. op must not care about the order. */
+__device__ __forceinline__ int row_value(int lane) { return ((lane >> 5) & 1) | ((lane >> 3) & 2); }
+namespace dpp {
+template <int HALF>
+__device__ __forceinline__ void swap_words(unsigned &a, unsigned &b) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  u2 r;
+  if constexpr (HALF == 32) r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  else r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r.x;
+  b = r.y;
+}
+/* HALF 32: a's upper half of the lanes against b's lower half; 16: a's odd rows against b's even rows */
+template <int HALF>
+__device__ __forceinline__ void swap(double &a, double &b) {
+  const uint64_t x = (uint64_t)__double_as_longlong(a), y = (uint64_t)__double_as_longlong(b);
+  unsigned al = (unsigned)x, ah = (unsigned)(x >> 32), bl = (unsigned)y, bh = (unsigned)(y >> 32);
+  swap_words<HALF>(al, bl);
+  swap_words<HALF>(ah, bh);
+  a = __longlong_as_double((long long)(((uint64_t)ah << 32) | al));
+  b = __longlong_as_double((long long)(((uint64_t)bh << 32) | bl));
+}
+template <int HALF>
+__device__ __forceinline__ void swap(float &a, float &b) {
+  unsigned x = __float_as_uint(a), y = __float_as_uint(b);
+  swap_words<HALF>(x, y);
+  a = __uint_as_float(x);
+  b = __uint_as_float(y);
+}
+/* v of another lane of the row (every lane has a source in these patterns) */
+template <int CTRL>
+__device__ __forceinline__ double row_mov(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+template <int CTRL>
+__device__ __forceinline__ float row_mov(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+}  // namespace dpp
+template <int M, typename T, class Op>
+__device__ __forceinline__ void wave_reduce(const T (&v)[M], T (&out)[(M + 3) / 4], Op op) {
+  constexpr int H = (M + 1) / 2, Q = (M + 3) / 4;
+  T u[2 * Q];
+#pragma unroll
+  for (int j = 0; j < H; j++) {
+    T a = v[2 * j], b = v[2 * j + 1 < M ? 2 * j + 1 : 2 * j];
+    dpp::swap<32>(a, b);
+    u[j] = op(a, b);
+  }
+  if (H < 2 * Q) u[2 * Q - 1] = u[H - 1];
+#pragma unroll
+  for (int j = 0; j < Q; j++) {
+    T a = u[2 * j], b = u[2 * j + 1];
+    dpp::swap<16>(a, b);
+    T t = op(a, b);
+    t = op(t, dpp::row_mov<dpp::kQuad1032>(t));
+    t = op(t, dpp::row_mov<dpp::kQuad2301>(t));
+    t = op(t, dpp::row_mov<dpp::kRowHalfMirror>(t));
+    out[j] = op(t, dpp::row_mov<dpp::kRowMirror>(t));
+  }
+}
+/* extrema of values that are not signalling NaNs (results of arithmetic): fmax without the quieting of its operands. The two
+ * wait states stand for the ones a lane-crossing read of a just-written register needs, which the compiler counts for its
+ * own instructions only. */
+__device__ __forceinline__ double max_val(double a, double b) {
+#if defined(__AMDGCN__)
+  double r;
+  asm("v_max_f64 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+#else
+  return fmax(a, b);
+#endif
+}
+__device__ __forceinline__ float max_val(float a, float b) {
+#if defined(__AMDGCN__)
+  float r;
+  asm("v_max_f32 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+#else
+  return fmaxf(a, b);
+#endif
+}
+/* The statistics of a wavefront's lanes (layout of stats_init: extrema of phi and mu first, then the sums), reduced:
+ * put(i, value) is called once for every statistic i, by one lane each. Extrema reduce in the statistics' own precision
+ * (exact; a minimum as the maximum of the negated values), sums in FP64. PHI_SUMS_ZERO: the squared phi increments are
+ * +0 on every lane, and so are their sums. */
+template <int N, int NC, bool PHI_SUMS_ZERO, int NSA, typename R, class F>
+__device__ __forceinline__ void stats_reduce(const R (&st)[NSA], int lane, F put) {
+  constexpr int ME = 2 * N + 2 * NC, S0 = PHI_SUMS_ZERO ? 3 * N + 2 * NC : ME, MS = NSA - S0;
+  constexpr int QE = (ME + 3) / 4, QS = (MS + 3) / 4;
+  const auto is_min = [](int i) { return (i >= N && i < 2 * N) || i >= 2 * N + NC; };
+  R e[ME], te[QE];
+  double v[MS], ts[QS];
+#pragma unroll
+  for (int i = 0; i < ME; i++) e[i] = is_min(i) ? -st[i] : st[i];
+#pragma unroll
+  for (int i = 0; i < MS; i++) v[i] = (double)st[S0 + i];
+  wave_reduce(e, te, [](R a, R b) { return max_val(a, b); });
+  wave_reduce(v, ts, [](double a, double b) { return a + b; });
+  /* lane q of a row stores its j = q value, so that each group leaves in one store */
+  const int q = lane & 15, i = 4 * q + row_value(lane);
+  R x = te[0];
+  double y = ts[0];
+#pragma unroll
+  for (int j = 1; j < QE; j++) x = q == j ? te[j] : x;
+#pragma unroll
+  for (int j = 1; j < QS; j++) y = q == j ? ts[j] : y;
+  if (i < ME) put(i, (double)(is_min(i) ? -x : x));
+  if (i < MS) put(S0 + i, y);
+  if (PHI_SUMS_ZERO && i < N) put(ME + i, 0.0);
+}
+
 }  // namespace gpk

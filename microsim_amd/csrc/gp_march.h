@@ -202,17 +202,11 @@ __device__ __forceinline__ void stats_add(R (&st)[NSA], const R *pn, const R *dp
 template <int N, int NC, bool PHI_SUMS_ZERO = false, int NSA, typename R>
 __device__ __forceinline__ void stats_partials(R (&st)[NSA], double *__restrict__ partials, int64_t pstride,
                                                int w, int nwaves, int lane) {
-  /* extrema reduce in the statistics' own precision (exact), sums in FP64. PHI_SUMS_ZERO: the kernel updates
-   * bulk cells only, whose squared phi increments are +0 on every lane, so those sums are +0 */
-#pragma unroll
-  for (int i = 0; i < NSA; i++) {
-    double r;
-    if (i < N || (i >= 2 * N && i < 2 * N + NC)) r = (double)wave_max(st[i]);
-    else if (i < 2 * N + 2 * NC) r = (double)wave_min(st[i]);
-    else if (PHI_SUMS_ZERO && i < 3 * N + 2 * NC) r = 0.0;
-    else r = wave_sum((double)st[i]);
-    if (lane == 0 && w < nwaves) partials[(int64_t)i * pstride + w] = r;
-  }
+  /* PHI_SUMS_ZERO: the kernel updates bulk cells only, whose squared phi increments are +0 on every lane */
+  if constexpr (NSA > 1) /* (kernels without statistics hold one slot and do not come here) */
+    stats_reduce<N, NC, PHI_SUMS_ZERO>(st, lane, [&](int i, double r) {
+      if (w < nwaves) partials[(int64_t)i * pstride + w] = r;
+    });
 }
 
 /* Tiles: wavefront w of a step kernel handles tile w = (strip w % nstrips, segment w / nstrips), i.e. the 60

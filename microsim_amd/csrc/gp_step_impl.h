@@ -102,15 +102,9 @@ __global__ __launch_bounds__(kBX *kBY) void k_mu(const Model<R> *__restrict__ mp
       if (!isfinite(mv)) st[NS - 1] += 1.0;
     }
   }
-  /* block reduction: wave shuffles, then the kBY waves through LDS */
+  /* block reduction: each wavefront's, then the kBY of them through LDS */
   __shared__ double red[kBY][NS];
-  for (int i = 0; i < NS; i++) {
-    double r;
-    if (i < N || (i >= 2 * N && i < 2 * N + NC)) r = wave_max(st[i]);
-    else if (i < 2 * N + 2 * NC) r = wave_min(st[i]);
-    else r = wave_sum(st[i]);
-    if (threadIdx.x == 0) red[threadIdx.y][i] = r;
-  }
+  stats_reduce<N, NC, false>(st, threadIdx.x, [&](int i, double r) { red[threadIdx.y][i] = r; });
   __syncthreads();
   if (threadIdx.y == 0 && threadIdx.x < NS) {
     const int i = threadIdx.x;
