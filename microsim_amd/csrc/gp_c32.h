@@ -124,15 +124,17 @@ __device__ __forceinline__ void c32_gather(const float *__restrict__ phi, const 
   }
 }
 
-/* delta-phi (FP64) of the listed candidate cells from the decoded state: a grid-stride loop of full wavefronts */
+/* delta-phi (FP64) of the listed candidate cells from the decoded state: a grid-stride loop of full wavefronts; the blocks
+ * before the list's carry StepExtras */
 template <int N, int NC, bool P2>
 __global__ __launch_bounds__(256) void k_dlist_c(const Model<double> *__restrict__ mp, const float *__restrict__ phi,
                                                  const float *__restrict__ plo, const float *__restrict__ mu,
                                                  const int8_t *__restrict__ mlo, double *__restrict__ dphi, int64_t fs,
                                                  int64_t ps, const int32_t *__restrict__ clist,
-                                                 const int *__restrict__ ccount) {
-  const int n = *ccount;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+                                                 const int *__restrict__ ccount, StepExtras<float> ex) {
+  if (step_extras<N, NC, float, true>(ex, fs, ps)) return;
+  const int nex = ex.nfold + ex.nhalo, n = *ccount, stride = ((int)gridDim.x - nex) * 256;
+  for (int i = ((int)blockIdx.x - nex) * 256 + (int)threadIdx.x; i < n; i += stride) {
     const int64_t c = clist[i];
     RegStore<N, NC, double> rs;
     c32_gather<N, NC>(phi, plo, mu, mlo, c, fs, ps, false, rs);
@@ -155,7 +157,8 @@ __global__ __launch_bounds__(256, 2) void k_ilist_c(const Model<double> *__restr
                                                  int8_t *__restrict__ mlo_o, int8_t *__restrict__ codes_out,
                                                  double *__restrict__ partials, int64_t pstride, int64_t fs,
                                                  int64_t ps, const int32_t *__restrict__ ilist,
-                                                 const int *__restrict__ icount) {
+                                                 const int *__restrict__ icount,
+                                               const uint64_t *__restrict__ mlist, const int *__restrict__ mcount) {
   constexpr int NS = 3 * N + 3 * NC + 1;
   constexpr int NSA = STATS ? NS : 1;
   const Model<double> &m = *mp;
@@ -163,11 +166,12 @@ __global__ __launch_bounds__(256, 2) void k_ilist_c(const Model<double> *__restr
   const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int nw = gridDim.x * 4;
   double st[NSA];
-  if (STATS) stats_init<N, NC>(st);
-  const int n = *icount;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int64_t c = ilist[i];
-    const int64_t y = (c - kYOff) % ps;
+  if constexpr (STATS) stats_init<N, NC>(st);
+  const int n = *icount, ntot = n + *mcount;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ntot; i += gridDim.x * blockDim.x) {
+    const IfaceItem it(i, n, ilist, mlist);
+    const int64_t c = it.c;
+    const int y = (int)((uint32_t)c % (uint32_t)ps) - kYOff;
     int8_t cd[5][5];
 #pragma unroll
     for (int di = -2; di <= 2; di++)
@@ -202,21 +206,31 @@ __global__ __launch_bounds__(256, 2) void k_ilist_c(const Model<double> *__restr
     for (int a = 0; a < N; a++) {
       df_encode(pn[a], ph[a], pl[a]);
       pd[a] = df_decode(ph[a], pl[a]);
-      phi_o[a * fs + c] = ph[a];
-      plo_o[a * fs + c] = pl[a];
     }
 #pragma unroll
     for (int k = 0; k < NC; k++) {
       c32_encode(mn[k], mh[k], mq[k]);
       md[k] = c32_decode(mh[k], mq[k]);
-      mu_o[k * fs + c] = mh[k];
-      mlo_o[k * fs + c] = mq[k];
     }
-    codes_out[c] = (int8_t)pure_phase<N>(pd);
-    if (STATS) stats_add<N, NC>(st, pd, d, md, dm);
+    if (it.groups & 1u) {
+#pragma unroll
+      for (int a = 0; a < N; a++) {
+        phi_o[a * fs + it.dst] = ph[a];
+        plo_o[a * fs + it.dst] = pl[a];
+      }
+      codes_out[it.dst] = (int8_t)pure_phase<N>(pd);
+    }
+    if (it.groups & 2u) {
+#pragma unroll
+      for (int k = 0; k < NC; k++) {
+        mu_o[k * fs + it.dst] = mh[k];
+        mlo_o[k * fs + it.dst] = mq[k];
+      }
+    }
+    if constexpr (STATS)
+      if (it.own) stats_add<N, NC>(st, pd, d, md, dm);
   }
-  if (!STATS) return;
-  stats_partials<N, NC>(st, partials, pstride, w, nw, lane);
+  if constexpr (STATS) stats_partials<N, NC>(st, partials, pstride, w, nw, lane);
 }
 
 }  // namespace gpk

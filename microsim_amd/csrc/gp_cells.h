@@ -19,7 +19,7 @@
  * reference by construction) on the listed cells in a grid-stride loop, so that every lane of every wavefront
  * works on an interface cell (a march row has about one in five) and no wavefront holds more than its share.
  * Every interior cell is written by exactly one of the two. They read the phase codes of the current state and
- * write those of the new one (a second buffer). k_halo then fills the new state's halo from its interior.
+ * write those of the new one (a second buffer). The halo of the new state is filled along the way (halo_cell).
  */
 #pragma once
 
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
              R *__restrict__ phi_o, R *__restrict__ mu_o, int8_t *__restrict__ codes_out,
              double *__restrict__ partials, int64_t pstride, int64_t fs, int64_t ps, int64_t mx, int64_t my,
              int nstrips, int nwaves, int keep, const int8_t *__restrict__ tin, int8_t *__restrict__ tout,
-             int32_t *__restrict__ ilist, int32_t *__restrict__ clist, int *counts, int *counts_next, int tile_blocks,
+             int32_t *__restrict__ ilist, int32_t *__restrict__ clist, int *counts, int *counts_next, int *mcount_next, int tile_blocks,
              int ring_blocks, const int8_t *__restrict__ mlo, float *__restrict__ plo_o, int8_t *__restrict__ mlo_o) {
   using Vw = View<R, P2, false, kFastOf<R>>;
   constexpr int NS = 3 * N + 3 * NC + 1;
@@ -341,6 +341,7 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
   }
   /* the next step's list lengths start at zero (the kernels that read them last ran before this one) */
   if (blockIdx.x == 0 && threadIdx.x < 2) counts_next[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 2) *mcount_next = 0;
   /* blocks go round the eight XCDs in turn: each XCD takes a contiguous run of tiles, so that the lines and rows two
    * neighbouring tiles share meet in one L2 */
   const int chunk = tile_blocks >> 3, bid = (int)blockIdx.x;
@@ -359,7 +360,7 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
   const unsigned c0i = (unsigned)(yl + kYOff), cyi = (unsigned)(y + kYOff);
 
   R st[NSA];
-  if (STATS) stats_init<N, NC>(st);
+  if constexpr (STATS) stats_init<N, NC>(st);
   unsigned seen = 0u; /* phases of the lane's bulk cells (their phi extrema, folded at the end) */
 
   /* mu rows in a ring of kCellRing register slots, row r in slot (r - xa) mod kCellRing, so that no slot is
@@ -595,41 +596,87 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
       }
     }
   }
-  if (!STATS) return;
-  bulk_seen_fold<N>(st, seen);
-  stats_partials<N, NC, true>(st, partials, pstride, w, nwaves, lane);
+  if constexpr (STATS) {
+    bulk_seen_fold<N>(st, seen);
+    stats_partials<N, NC, true>(st, partials, pstride, w, nwaves, lane);
+  }
 }
 
 
-/* The halo of the new state, after k_cbulk and k_ilist wrote every interior cell: each halo cell takes the value
- * of its proxy, as write_images scatters it (apply_boundary_conditions as a gather). Halo row X = hx[k] has the
- * proxy row sx[f][k] when that is an interior row and at most one k' < k shares it (write_images takes the first
- * two images of a row); an interior row is its own (likewise for columns). Field group f = 0 holds phi, its low
- * parts and the phase codes, f = 1 mu and its extensions. A halo cell without a proxy is left as it is. */
+/* The halo of the new state: each halo cell takes the value of its proxy, as write_images scatters it
+ * (apply_boundary_conditions as a gather). Halo row X = hx[k] has the proxy row sx[f][k] when that is an interior row and
+ * at most one k' < k shares it (write_images takes the first two images of a row); an interior row is its own (likewise
+ * for columns). Field group f = 0 holds phi, its low parts and the phase codes, f = 1 mu and its extensions. A halo cell
+ * without a proxy is left as it is.
+ * No launch of its own: k_cbulk has written the bulk cells when the delta-phi launch runs, so extra blocks of that launch
+ * copy the halo cells whose proxy is a bulk cell and list the others, and k_ilist updates a listed proxy once more with
+ * the halo cell as its target (the separate pass was 4 to 10 us a step, nearly all of it launch and memory latency; images
+ * scattered by the lane that updates the proxy lengthened every k_ilist by 4 us: 1024^2 FP64 12.3 -> 16.5). */
 __device__ __forceinline__ int64_t halo_source(const int32_t *src, const int32_t *h, int64_t X, int64_t lo,
                                                int64_t hi) {
   if (X >= lo && X <= hi) return X;
   int64_t s = -1;
 #pragma unroll
   for (int k = 0; k < 6; k++) {
-    if (h[k] != X) continue;
     int before = 0;
+#pragma unroll
     for (int j = 0; j < k; j++) before += src[j] == src[k];
-    if (src[k] >= lo && src[k] <= hi && before < 2) s = src[k];
+    if (h[k] == X && src[k] >= lo && src[k] <= hi && before < 2) s = src[k];
   }
   return s;
 }
 
-/* planes of the state the halo pass copies: the phase codes, phi, (C: phi's low parts), mu, (C: mu's extensions) */
-template <int N, int NC, bool C>
-constexpr int kHaloPlanes = 1 + N + NC + (C ? N + NC : 0);
+/* the phase of a bulk cell at offset s (its radius-2 diamond is purely that phase), else -1 */
+__device__ __forceinline__ int bulk_code(const int8_t *__restrict__ codes, int64_t s, int64_t ps) {
+  const int b = codes[s];
+  bool same = b >= 0;
+#pragma unroll
+  for (int di = -2; di <= 2; di++)
+#pragma unroll
+    for (int dj = -2; dj <= 2; dj++)
+      if ((di < 0 ? -di : di) + (dj < 0 ? -dj : dj) <= 2) same = same & (codes[s + di * ps + dj] == b);
+  return same ? b : -1;
+}
 
-/* halo cell j (the six halo rows over the full width, then the six halo cells of each interior row) of plane p */
+/* the output buffers of a step (plo, mlo: compensated mode) */
+template <typename R>
+struct NewState {
+  R *phi, *mu;
+  int8_t *codes;
+  float *plo;
+  int8_t *mlo;
+};
+
+/* An image in k_ilist's second list: the proxy's offset, the halo cell's, and the field groups to write there (bit 0: phi
+ * and codes, bit 1: mu). Offsets have 31 bits (cells_fit). */
+__device__ __forceinline__ uint64_t image_entry(int64_t src, int64_t dst, unsigned groups) {
+  return (uint64_t)src | ((uint64_t)dst << 31) | ((uint64_t)groups << 62);
+}
+/* item i of k_ilist: cell c and target dst, groups and whether it counts in the statistics; i < n: listed cells */
+struct IfaceItem {
+  int64_t c, dst;
+  unsigned groups;
+  bool own;
+  __device__ __forceinline__ IfaceItem(int i, int n, const int32_t *__restrict__ ilist, const uint64_t *__restrict__ mlist) {
+    own = i < n;
+    if (own) {
+      c = dst = ilist[i];
+      groups = 3u;
+    } else {
+      const uint64_t e = mlist[i - n];
+      c = (int64_t)(e & 0x7fffffffu);
+      dst = (int64_t)((e >> 31) & 0x7fffffffu);
+      groups = (unsigned)(e >> 62);
+    }
+  }
+};
+
+/* halo cell j (the six halo rows over the full width, then the six halo cells of each interior row): copied where the
+ * proxy is a bulk cell of the step from codes_in, listed where it is an interface cell */
 template <int N, int NC, typename R, bool C>
-__device__ __forceinline__ void halo_cell(int64_t j, int p, R *__restrict__ phi, R *__restrict__ mu,
-                                          int8_t *__restrict__ codes, float *__restrict__ plo,
-                                          int8_t *__restrict__ mlo, const Maps &maps, int64_t fs, int64_t ps,
-                                          int64_t mx, int64_t my) {
+__device__ __forceinline__ void halo_cell(int64_t j, const int8_t *__restrict__ codes_in, const NewState<R> &o,
+                                          uint64_t *__restrict__ mlist, int *mcount, const Maps &maps, int64_t fs,
+                                          int64_t ps, int64_t mx, int64_t my) {
   const int64_t ry = my + 6, nrow = 6 * ry, ncol = 6 * mx;
   if (j >= nrow + ncol) return;
   /* the index arithmetic in 32 bits (the halo has fewer than 2^31 cells; 64-bit division is a long sequence) */
@@ -644,39 +691,137 @@ __device__ __forceinline__ void halo_cell(int64_t j, int p, R *__restrict__ phi,
     Y = q < 3u ? (int64_t)q : my + q;
     X = 3 + (int64_t)row;
   }
-  constexpr int P0 = 1 + N + (C ? N : 0); /* planes of field group 0 (codes, phi, plo); the rest are group 1 */
-  const int f = p < P0 ? 0 : 1;
-  const int64_t sx = halo_source(maps.sx[f], maps.hx, X, 3, mx + 2);
-  const int64_t sy = halo_source(maps.sy[f], maps.hy, Y, 3, my + 2);
-  if (sx < 0 || sy < 0) return;
-  const int64_t c = X * ps + Y + kYOff, s = sx * ps + sy + kYOff;
-  if (p == 0) {
-    codes[c] = codes[s];
-  } else if (p <= N) {
-    phi[(p - 1) * fs + c] = phi[(p - 1) * fs + s];
-  } else if (C && p < P0) {
-    plo[(p - 1 - N) * fs + c] = plo[(p - 1 - N) * fs + s];
-  } else if (p < P0 + NC) {
-    mu[(p - P0) * fs + c] = mu[(p - P0) * fs + s];
-  } else if (C) {
-    mlo[(p - P0 - NC) * fs + c] = mlo[(p - P0 - NC) * fs + s];
+  const int64_t c = X * ps + Y + kYOff;
+  int64_t s[2];
+  int b[2];
+#pragma unroll
+  for (int f = 0; f < 2; f++) {
+    const int64_t sx = halo_source(maps.sx[f], maps.hx, X, 3, mx + 2);
+    const int64_t sy = halo_source(maps.sy[f], maps.hy, Y, 3, my + 2);
+    s[f] = sx < 0 || sy < 0 ? -1 : sx * ps + sy + kYOff;
+    b[f] = s[f] < 0 ? -1 : bulk_code(codes_in, s[f], ps);
+  }
+  if (b[0] >= 0) {
+    o.codes[c] = (int8_t)b[0];
+#pragma unroll
+    for (int a = 0; a < N; a++) {
+      o.phi[a * fs + c] = a == b[0] ? R(1.0) : R(0.0);
+      if constexpr (C) o.plo[a * fs + c] = 0.0f;
+    }
+  }
+  if (b[1] >= 0) {
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+      o.mu[k * fs + c] = o.mu[k * fs + s[1]];
+      if constexpr (C) o.mlo[k * fs + c] = o.mlo[k * fs + s[1]];
+    }
+  }
+  /* interface proxies: one entry, or one per field group where the groups' proxies differ */
+  const bool i0 = s[0] >= 0 && b[0] < 0, i1 = s[1] >= 0 && b[1] < 0, one = i0 && i1 && s[0] == s[1];
+  const int n = one ? 1 : (int)i0 + (int)i1;
+  if (n) {
+    const int at = atomicAdd(mcount, n);
+    if (one) {
+      mlist[at] = image_entry(s[0], c, 3);
+    } else {
+      if (i0) mlist[at] = image_entry(s[0], c, 1);
+      if (i1) mlist[at + (i0 ? 1 : 0)] = image_entry(s[1], c, 2);
+    }
   }
 }
 
 /* number of halo cells halo_cell covers */
 __host__ __device__ constexpr int64_t halo_cells(int64_t mx, int64_t my) { return 6 * (my + 6) + 6 * mx; }
 
-/* one thread per halo cell and plane (blockIdx.y is the plane) */
-template <int N, int NC, typename R, bool C>
-__global__ __launch_bounds__(256) void k_halo(R *__restrict__ phi, R *__restrict__ mu, int8_t *__restrict__ codes,
-                                              float *__restrict__ plo, int8_t *__restrict__ mlo, Maps maps,
-                                              int64_t fs, int64_t ps, int64_t mx, int64_t my) {
-  halo_cell<N, NC, R, C>((int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int)blockIdx.y, phi, mu, codes, plo, mlo,
-                         maps, fs, ps, mx, my);
+/* blocks of the halo pass at the front of a delta-phi launch */
+__host__ __device__ constexpr unsigned halo_blocks(int64_t mx, int64_t my) {
+  return (unsigned)((halo_cells(mx, my) + 255) / 256);
 }
 
-/* The general update of the interface cells listed by k_cbulk (any order): a grid-stride loop of full
- * wavefronts. Each cell gathers its stencil from memory in one batch: phi on the 3x3 neighbourhood, mu and
+/* Fold the partials of a step's wavefronts into the cumulative statistics: one block per statistic, each reading its
+ * contiguous row of partials (statistic-major layout) in a fixed order, so the result is deterministic. */
+template <int N, int NC, int THREADS>
+__device__ __forceinline__ void stats_fold_block(const double *__restrict__ partials, int64_t stride, int64_t nparts,
+                                                 double *__restrict__ cum, int i) {
+  constexpr int NS = 3 * N + 3 * NC + 1;
+  __shared__ double red[THREADS];
+  if (i >= NS) return;
+  const bool mx = (i < N || (i >= 2 * N && i < 2 * N + NC));
+  const bool mn = !mx && i < 2 * N + 2 * NC;
+  double r = mx ? -INFINITY : mn ? INFINITY : 0.0;
+  const double *row = partials + (int64_t)i * stride;
+  /* a thread folds its partials in index order; the loads of eight of them are issued before the first is used */
+  int64_t b = threadIdx.x;
+  for (; b + 7 * THREADS < nparts; b += 8 * THREADS) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = row[b + u * THREADS];
+#pragma unroll
+    for (int u = 0; u < 8; u++) r = mx ? fmax(r, v[u]) : mn ? fmin(r, v[u]) : r + v[u];
+  }
+  for (; b < nparts; b += THREADS) {
+    const double v = row[b];
+    r = mx ? fmax(r, v) : mn ? fmin(r, v) : r + v;
+  }
+  red[threadIdx.x] = r;
+  __syncthreads();
+  for (int s = THREADS / 2; s > 0; s >>= 1) {
+    if (threadIdx.x < s) {
+      double o = red[threadIdx.x + s];
+      red[threadIdx.x] = mx ? fmax(red[threadIdx.x], o) : mn ? fmin(red[threadIdx.x], o) : red[threadIdx.x] + o;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    double v = red[0];
+    if (mx) cum[i] = fmax(cum[i], v);
+    else if (mn) cum[i] = fmin(cum[i], v);
+    else if (i < NS - 1) cum[i] = v;
+    else cum[i] += v;
+  }
+}
+
+/* What rides in the delta-phi launch of a step, in blocks before those of the list: the fold of the previous step's
+ * statistics (nfold blocks; its partials lie in the half of the buffer that this step does not write), and the halo of the
+ * new state (nhalo blocks). Launches of their own for the two were 4 to 10 us a step. */
+template <typename R>
+struct StepExtras {
+  int nfold, nhalo;
+  const double *partials;
+  int64_t pstride;
+  double *cum;
+  const int8_t *codes_in;
+  NewState<R> o;
+  uint64_t *mlist;
+  int *mcount;
+  Maps maps;
+  int64_t mx, my;
+};
+/* true when the calling block was one of the extras */
+template <int N, int NC, typename R, bool C>
+__device__ __forceinline__ bool step_extras(const StepExtras<R> &e, int64_t fs, int64_t ps) {
+  const int b = (int)blockIdx.x;
+  if (b >= e.nfold + e.nhalo) return false;
+  if (b < e.nfold) stats_fold_block<N, NC, 256>(e.partials, e.pstride, e.pstride, e.cum, b);
+  else halo_cell<N, NC, R, C>((int64_t)(b - e.nfold) * 256 + threadIdx.x, e.codes_in, e.o, e.mlist, e.mcount, e.maps, fs, ps, e.mx,
+                              e.my);
+  return true;
+}
+
+/* The delta-phi launch of a step: the extras, then the candidates (k_dlist's loop). */
+template <int N, int NC, typename R, bool P2>
+__global__ __launch_bounds__(256) void k_dlist_step(const Model<R> *__restrict__ mp, const R *__restrict__ phi,
+                                                    const R *__restrict__ mu, R *__restrict__ dphi, int64_t fs, int64_t ps,
+                                                    const int32_t *__restrict__ clist, const int *__restrict__ ccount,
+                                                    StepExtras<R> ex) {
+  if (step_extras<N, NC, R, false>(ex, fs, ps)) return;
+  const int nex = ex.nfold + ex.nhalo, n = *ccount, stride = ((int)gridDim.x - nex) * 256;
+  for (int i = ((int)blockIdx.x - nex) * 256 + (int)threadIdx.x; i < n; i += stride)
+    dphi_cell<N, NC, R, P2>(*mp, phi, mu, dphi, fs, ps, clist[i]);
+}
+
+/* The general update of the interface cells listed by k_cbulk (any order), then of the images (IfaceItem): a grid-stride
+ * loop of full wavefronts. Each cell gathers its stencil from memory in one batch: phi on the 3x3 neighbourhood, mu and
  * delta-phi on the 5-point one, and the phase codes of its radius-2 diamond, which decide which of the five
  * delta-phi values are k_dphi's (candidates) and which are exactly 0. Statistics: one partial per wavefront of the
  * grid (the grid is fixed, the order of the cells within it is not). */
@@ -687,7 +832,8 @@ __global__ __launch_bounds__(256, 2) void k_ilist(const Model<R> *__restrict__ m
                                                R *__restrict__ mu_o, int8_t *__restrict__ codes_out,
                                                double *__restrict__ partials, int64_t pstride, int64_t fs,
                                                int64_t ps, const int32_t *__restrict__ ilist,
-                                               const int *__restrict__ icount) {
+                                               const int *__restrict__ icount,
+                                               const uint64_t *__restrict__ mlist, const int *__restrict__ mcount) {
   constexpr int NS = 3 * N + 3 * NC + 1;
   constexpr int NSA = STATS ? NS : 1;
   const Model<R> &m = *mp;
@@ -695,11 +841,12 @@ __global__ __launch_bounds__(256, 2) void k_ilist(const Model<R> *__restrict__ m
   const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int nw = gridDim.x * 4;
   R st[NSA];
-  if (STATS) stats_init<N, NC>(st);
-  const int n = *icount;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int64_t c = ilist[i];
-    const int64_t y = (c - kYOff) % ps;
+  if constexpr (STATS) stats_init<N, NC>(st);
+  const int n = *icount, ntot = n + *mcount;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ntot; i += gridDim.x * blockDim.x) {
+    const IfaceItem it(i, n, ilist, mlist);
+    const int64_t c = it.c;
+    const int y = (int)((uint32_t)c % (uint32_t)ps) - kYOff;
     /* codes of the diamond: slot (di, dj) for |di| + |dj| <= 2 */
     int8_t cd[5][5];
 #pragma unroll
@@ -742,15 +889,19 @@ __global__ __launch_bounds__(256, 2) void k_ilist(const Model<R> *__restrict__ m
 #pragma unroll
     for (int a = 0; a < N; a++) d[a] = v.dp(a, 0, 0);
     mu_update<N, NC>(m, v, false, d, jx0, jxb, jy0, jyl, pn, mn, dm);
+    if (it.groups & 1u) {
 #pragma unroll
-    for (int a = 0; a < N; a++) phi_o[a * fs + c] = pn[a];
+      for (int a = 0; a < N; a++) phi_o[a * fs + it.dst] = pn[a];
+      codes_out[it.dst] = (int8_t)pure_phase<N>(pn);
+    }
+    if (it.groups & 2u) {
 #pragma unroll
-    for (int k = 0; k < NC; k++) mu_o[k * fs + c] = mn[k];
-    codes_out[c] = (int8_t)pure_phase<N>(pn);
-    if (STATS) stats_add<N, NC>(st, pn, d, mn, dm);
+      for (int k = 0; k < NC; k++) mu_o[k * fs + it.dst] = mn[k];
+    }
+    if constexpr (STATS)
+      if (it.own) stats_add<N, NC>(st, pn, d, mn, dm);
   }
-  if (!STATS) return;
-  stats_partials<N, NC>(st, partials, pstride, w, nw, lane);
+  if constexpr (STATS) stats_partials<N, NC>(st, partials, pstride, w, nw, lane);
 }
 
 }  // namespace gpk

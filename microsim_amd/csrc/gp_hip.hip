@@ -454,7 +454,7 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
   }
   h->nblocks_mu = ((params->mesh_y + kBX - 1) / kBX) * ((params->mesh_x + kBY - 1) / kBY);
   march_plan(h);
-  h->nparts_max = std::max(h->nblocks_mu, std::max(2 * h->march_nwaves, h->cell_nwaves + h->cell_npad + 4 * (int64_t)kListBlocks));
+  h->nparts_max = std::max(h->nblocks_mu, std::max(2 * h->march_nwaves, 2 * (h->cell_nwaves + h->cell_npad + 4 * (int64_t)kListBlocks)));
   const char *path = getenv("GP_PATH");
   h->use_march = !(path && strcmp(path, "twopass") == 0);
   /* the cell lists and k_cbulk's row offsets are 32-bit: grids beyond that bound (cells_fit, about 46000^2 cells)
@@ -502,9 +502,10 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
    * planes of a small grid in one run */
   h->stage_bytes = std::max((size_t)h->fs * 2 * sizeof(int32_t),
                             std::min((size_t)h->N * h->fs * sizeof(double), kStageBytes));
-  ok = ok && hipMalloc((void **)&h->clist, h->stage_bytes) == hipSuccess;
+  ok = ok && hipMalloc((void **)&h->clist, h->stage_bytes) == hipSuccess &&
+       hipMalloc((void **)&h->mlist, (size_t)halo_cells(params->mesh_x, params->mesh_y) * 2 * sizeof(uint64_t)) == hipSuccess;
   h->ilist = ok ? h->clist + h->fs : nullptr;
-  ok = ok && hipMalloc((void **)&h->lcount, 4 * sizeof(int)) == hipSuccess;
+  ok = ok && hipMalloc((void **)&h->lcount, 6 * sizeof(int)) == hipSuccess;
   ok = ok && hipMalloc((void **)&h->codes[0], (size_t)h->rx * h->ps) == hipSuccess &&
        hipMalloc((void **)&h->codes[1], (size_t)h->rx * h->ps) == hipSuccess;
   h->ccur = 0;
@@ -517,7 +518,7 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
   ok = hipMemsetAsync(h->phi[0], 0, pn, h->stream) == hipSuccess && hipMemsetAsync(h->phi[1], 0, pn, h->stream) == hipSuccess &&
        hipMemsetAsync(h->mu[0], 0, mn, h->stream) == hipSuccess && hipMemsetAsync(h->mu[1], 0, mn, h->stream) == hipSuccess &&
        hipMemsetAsync(h->dphi, 0, (size_t)h->N * h->fs * dphi_esize(h), h->stream) == hipSuccess &&
-       hipMemsetAsync(h->lcount, 0, 4 * sizeof(int), h->stream) == hipSuccess;
+       hipMemsetAsync(h->lcount, 0, 6 * sizeof(int), h->stream) == hipSuccess;
   h->lsel = 0;
   if (precision == GP_FP64) {
     Model<double> m;
@@ -589,7 +590,7 @@ void gp_destroy(gp_handle *h) {
   delete h->adj;
   void *bufs[] = {h->phi[0], h->phi[1], h->mu[0],    h->mu[1],    h->dphi,   h->partials, h->stats_dev,
                   h->model,  h->flags[0], h->flags[1], h->inv_dev, h->codes[0], h->codes[1], h->clist,
-                  h->lcount,  h->lo[0],    h->lo[1],    h->model64, h->wide[0],  h->wide[1],
+                  h->lcount, h->mlist, h->lo[0],    h->lo[1],    h->model64, h->wide[0],  h->wide[1],
                   h->trow,   h->thp,    h->thc,      h->front,    h->tflags};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
@@ -747,12 +748,17 @@ int gp_step(gp_handle *h, int64_t nsteps, gp_stats *stats) {
   {
     ProfScope ps(h, GP_KERNEL_CALL);
     const bool framed = h->p.tempgrady || h->p.shift;
+    h->stats_pending = false;
     for (int64_t t = 0; t < nsteps; t++) {
       int rc = f(h, h->use_march ? (stats ? MODE_MARCH_STATS : MODE_MARCH) : MODE_TWOPASS);
       if (rc) return rc;
       h->steps++;
       h->prev_valid = h->use_march;
       if (framed && (rc = frame_after_step(h, h->steps))) return rc;
+    }
+    if (stats && nsteps > 0 && h->use_cells) {
+      int rc = f(h, MODE_STATS_FOLD);
+      if (rc) return rc;
     }
   }
   if (stats) {

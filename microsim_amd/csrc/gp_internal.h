@@ -79,6 +79,8 @@ struct gp_handle {
   int64_t nblocks_mu;
   int64_t steps;
   int64_t nparts_max;       /* rows of the partials buffer */
+  int stats_half;           /* cells path: the half of the partials that the current step writes */
+  bool stats_pending;       /* the other half holds a step that is not folded yet */
   int march_seg, march_nstrips, march_nsegs; /* tile grid of the single-pass step (see gp_march.h) */
   int64_t march_nwaves;     /* tiles = wavefronts of k_march and of k_bulk */
   int cell_seg, cell_nstrips; /* tile grid of k_cbulk: strips of kCellOut cells by segments of cell_seg rows */
@@ -87,7 +89,8 @@ struct gp_handle {
   int8_t *tflags;            /* its tile flags of two alternating steps (by lsel) */
   int32_t *clist, *ilist;    /* delta-phi candidates and interface cells of the current step (cell offsets), one allocation */
   size_t stage_bytes;        /* its bytes: between steps it stages host rows (gp_pack.h) */
-  int *lcount;               /* their lengths: two pairs, used by alternate steps (lcount + 2 * lsel) */
+  uint64_t *mlist;           /* the step's images: halo cells whose proxy is an interface cell (gp_cells.h, image_entry) */
+  int *lcount;               /* their lengths: two pairs, used by alternate steps (lcount + 2 * lsel), then mlist's two */
   int lsel;
   int lgrid_d, lgrid_i;      /* grids of this handle's delta-phi and interface list kernels (0: not yet set) */
   int *flags[2];            /* per-tile purity flags of the last two steps */
@@ -147,7 +150,7 @@ int gp_fail(gp_handle *h, int code, const char *fmt, ...);
     if (e_ != hipSuccess) return gp_fail((h), GP_E_HIP, "%s: %s", #call, hipGetErrorString(e_)); \
   } while (0)
 
-enum { MODE_SMOOTH = 0, MODE_TWOPASS = 1, MODE_MARCH = 2, MODE_DPHI_PREV = 3, MODE_MARCH_STATS = 4 };
+enum { MODE_SMOOTH = 0, MODE_TWOPASS = 1, MODE_MARCH = 2, MODE_DPHI_PREV = 3, MODE_MARCH_STATS = 4, MODE_STATS_FOLD = 5 };
 
 inline size_t esize(const gp_handle *h) { return h->precision == GP_FP64 ? sizeof(double) : sizeof(float); }
 inline size_t state_elems(const gp_handle *h) { return (size_t)(h->N + h->NC) * h->fs; }

@@ -120,55 +120,12 @@ __global__ __launch_bounds__(kBX *kBY) void k_mu(const Model<R> *__restrict__ mp
   }
 }
 
-/* Fold the per-block partials into the cumulative statistics: one block per statistic, each reading its
- * contiguous row of partials (statistic-major layout) in a fixed order, so the result is deterministic. */
 constexpr int kStatThreads = 1024;
-
-template <int N, int NC>
-__device__ __forceinline__ void stats_fold_block(const double *__restrict__ partials, int64_t stride, int64_t nparts,
-                                                 double *__restrict__ cum, int i) {
-  constexpr int NS = 3 * N + 3 * NC + 1;
-  __shared__ double red[kStatThreads];
-  if (i >= NS) return;
-  const bool mx = (i < N || (i >= 2 * N && i < 2 * N + NC));
-  const bool mn = !mx && i < 2 * N + 2 * NC;
-  double r = mx ? -INFINITY : mn ? INFINITY : 0.0;
-  const double *row = partials + (int64_t)i * stride;
-  /* a thread folds its partials in index order; the loads of eight of them are issued before the first is used */
-  int64_t b = threadIdx.x;
-  for (; b + 7 * kStatThreads < nparts; b += 8 * kStatThreads) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) v[u] = row[b + u * kStatThreads];
-#pragma unroll
-    for (int u = 0; u < 8; u++) r = mx ? fmax(r, v[u]) : mn ? fmin(r, v[u]) : r + v[u];
-  }
-  for (; b < nparts; b += kStatThreads) {
-    const double v = row[b];
-    r = mx ? fmax(r, v) : mn ? fmin(r, v) : r + v;
-  }
-  red[threadIdx.x] = r;
-  __syncthreads();
-  for (int s = kStatThreads / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      double o = red[threadIdx.x + s];
-      red[threadIdx.x] = mx ? fmax(red[threadIdx.x], o) : mn ? fmin(red[threadIdx.x], o) : red[threadIdx.x] + o;
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    double v = red[0];
-    if (mx) cum[i] = fmax(cum[i], v);
-    else if (mn) cum[i] = fmin(cum[i], v);
-    else if (i < NS - 1) cum[i] = v;
-    else cum[i] += v;
-  }
-}
 
 template <int N, int NC>
 __global__ __launch_bounds__(kStatThreads) void k_stats(const double *__restrict__ partials, int64_t stride,
                                                         int64_t nparts, double *__restrict__ cum) {
-  stats_fold_block<N, NC>(partials, stride, nparts, cum, (int)blockIdx.x);
+  stats_fold_block<N, NC, kStatThreads>(partials, stride, nparts, cum, (int)blockIdx.x);
 }
 
 /* The statistics fold of a non-isothermal step and, in the blocks past it, the row temperatures after the step
@@ -182,7 +139,7 @@ __global__ __launch_bounds__(kStatThreads) void k_stats_thermo(const double *__r
                                                                double grad) {
   constexpr int NS = 3 * N + 3 * NC + 1;
   if ((int)blockIdx.x < NS) {
-    stats_fold_block<N, NC>(partials, stride, nparts, cum, (int)blockIdx.x);
+    stats_fold_block<N, NC, kStatThreads>(partials, stride, nparts, cum, (int)blockIdx.x);
     return;
   }
   const int q = (int)blockIdx.x - NS, a = (q >> 1) % N, sweep = q & 1;
@@ -191,26 +148,6 @@ __global__ __launch_bounds__(kStatThreads) void k_stats_thermo(const double *__r
   const auto T = [&](int64_t r) { return bottom + (double)r * grad; };
   if (a == 0 && sweep == 0) trow[y] = T(y);
   thermo_cell<N, NC, R>(tp, T, a, sweep, y, thp, thc);
-}
-
-/* The statistics fold and the halo pass of the cell-classified step in one launch (both small and latency-bound,
- * and independent: the fold reads the partials, the halo pass the new state): blocks below the number of
- * statistics fold one statistic each, the others copy kStatThreads halo cells of one plane each (k_halo). */
-template <int N, int NC, typename R, bool C>
-__global__ __launch_bounds__(kStatThreads) void k_stats_halo(const double *__restrict__ partials, int64_t stride,
-                                                             int64_t nparts, double *__restrict__ cum,
-                                                             R *__restrict__ phi, R *__restrict__ mu,
-                                                             int8_t *__restrict__ codes, float *__restrict__ plo,
-                                                             int8_t *__restrict__ mlo, Maps maps, int64_t fs,
-                                                             int64_t ps, int64_t mx, int64_t my) {
-  constexpr int NS = 3 * N + 3 * NC + 1;
-  if ((int)blockIdx.x < NS) {
-    stats_fold_block<N, NC>(partials, stride, nparts, cum, (int)blockIdx.x);
-    return;
-  }
-  const int64_t nchunk = (halo_cells(mx, my) + kStatThreads - 1) / kStatThreads, q = blockIdx.x - NS;
-  halo_cell<N, NC, R, C>((q % nchunk) * kStatThreads + threadIdx.x, (int)(q / nchunk), phi, mu, codes, plo, mlo, maps,
-                         fs, ps, mx, my);
 }
 
 /* Global solute and grand-potential energy of the current state (no reference counterpart; the FP64 oracle's
@@ -336,6 +273,42 @@ static int launch_invariants(gp_handle *h) {
 static int64_t cell_ipart(const gp_handle *h) { return h->cell_nwaves + h->cell_npad; }
 static int64_t cell_parts(const gp_handle *h) { return cell_ipart(h) + 4 * h->lgrid_i; }
 
+/* the partials of the current step, and (other) of the one before: two halves used in turn */
+template <int N, int NC>
+static double *cell_partials(const gp_handle *h, bool other = false) {
+  return h->partials + ((h->stats_half != 0) != other ? (3 * N + 3 * NC + 1) * cell_parts(h) : 0);
+}
+
+/* the number of images of the current step (next: of the one after it, which k_cbulk clears); launch_cbulk has flipped lsel
+ * to the next step's counts when the step's other launches are formed */
+static int *image_count(const gp_handle *h, bool next = false) { return h->lcount + 4 + (next ? h->lsel : 1 - h->lsel); }
+
+/* what the delta-phi launch of the current step carries */
+template <int N, int NC, typename R>
+static StepExtras<R> step_extras_of(const gp_handle *h, bool stats, const int8_t *codes, const NewState<R> &o) {
+  const int64_t mx = h->p.mesh_x, my = h->p.mesh_y;
+  return {stats && h->stats_pending ? 3 * N + 3 * NC + 1 : 0, (int)halo_blocks(mx, my), cell_partials<N, NC>(h, true),
+          cell_parts(h), h->stats_dev, codes, o, h->mlist, image_count(h), h->maps, mx, my};
+}
+
+/* the end of a step's launches: with statistics, its partials wait for the fold in the next step's delta-phi launch */
+static void step_partials_done(gp_handle *h, bool stats) {
+  h->stats_pending = stats;
+  if (stats) h->stats_half = 1 - h->stats_half;
+}
+
+/* the fold of the last step of a run */
+template <int N, int NC>
+static int launch_stats_fold(gp_handle *h) {
+  if (!h->stats_pending) return GP_OK;
+  h->stats_pending = false;
+  ProfScope ps(h, GP_KERNEL_STATS);
+  hipLaunchKernelGGL((k_stats<N, NC>), dim3(3 * N + 3 * NC + 1), dim3(kStatThreads), 0, h->stream,
+                     (const double *)cell_partials<N, NC>(h, true), cell_parts(h), cell_parts(h), h->stats_dev);
+  HIPCHK(h, hipGetLastError());
+  return GP_OK;
+}
+
 /* k_cbulk of one step: the tiles, then the blocks that list the boundary ring's candidates (one thread per ring
  * cell). This step's list lengths are zero (the previous step's k_cbulk, or the set-up, cleared them); k_cbulk clears
  * the other pair for the next step. Returns this step's lengths (interface cells, candidates). C: compensated mode. */
@@ -352,8 +325,9 @@ static int *launch_cbulk_seg(gp_handle *h, const Model<R> *m) {
   ProfScope ps(h, GP_KERNEL_CBULK);
   hipLaunchKernelGGL((k_cbulk<N, NC, R, P2, STATS, SEG, C>), dim3(cblk + rblk + (npad + 3) / 4), dim3(256), 0, h->stream, m,
                      (const R *)h->mu[b], (const int8_t *)h->codes[h->ccur], (R *)h->phi[o], (R *)h->mu[o],
-                     h->codes[1 - h->ccur], h->partials, cstride, h->fs, h->ps, mx, my, h->cell_nstrips, ct,
-                     (int)h->prev_valid, (const int8_t *)tin, tout, h->ilist, h->clist, lc, lnext, (int)cblk,
+                     h->codes[1 - h->ccur], cell_partials<N, NC>(h), cstride, h->fs, h->ps, mx, my, h->cell_nstrips, ct,
+                     (int)h->prev_valid, (const int8_t *)tin, tout, h->ilist, h->clist, lc, lnext,
+                     image_count(h, true), (int)cblk,
                      (int)rblk, C ? (const int8_t *)c32_mlo(h, b) : (const int8_t *)nullptr,
                      C ? c32_plo(h, o) : (float *)nullptr, C ? c32_mlo(h, o) : (int8_t *)nullptr);
   return lc;
@@ -381,6 +355,7 @@ static int launch_step_p(gp_handle *h, int mode) {
   const bool smooth = mode == MODE_SMOOTH;
   const bool tg = h->p.tempgrady != 0;
   const RowThermo<R> *thp = (const RowThermo<R> *)h->thp, *thc = (const RowThermo<R> *)h->thc;
+  if (mode == MODE_STATS_FOLD) return launch_stats_fold<N, NC>(h);
   if (mode == MODE_DPHI_PREV) {
     /* delta-phi of the last step, recomputed from the previous state (still in the other buffer). Single-pass steps only,
      * so never a non-isothermal run: its two sweeps store delta-phi. */
@@ -416,43 +391,33 @@ static int launch_step_p(gp_handle *h, int mode) {
     if (h->use_cells) {
       /* statistics partials: k_cbulk's wavefronts, then k_ilist's */
       if (!h->lgrid_d) {
-        h->lgrid_d = list_grid(h, k_dlist<N, NC, R, P2>);
+        h->lgrid_d = list_grid(h, k_dlist_step<N, NC, R, P2>);
         h->lgrid_i = list_grid(h, k_ilist<N, NC, R, P2, true>);
       }
       const int64_t cstride = cell_parts(h);
       const int *lc = launch_cbulk<N, NC, R, P2, false>(h, m, stats);
       {
-        /* delta-phi of the listed candidates, full wavefronts */
+        /* delta-phi of the listed candidates, full wavefronts; the halo and the fold */
         ProfScope ps(h, GP_KERNEL_DPHI);
-        hipLaunchKernelGGL((k_dlist<N, NC, R, P2>), dim3(h->lgrid_d), dim3(256), 0, h->stream, m, phi, mu, dphi,
-                           h->fs, h->ps, (const int32_t *)h->clist, lc + 1);
+        const StepExtras<R> ex =
+            step_extras_of<N, NC, R>(h, stats, codes, NewState<R>{phi_o, mu_o, codes_o, nullptr, nullptr});
+        hipLaunchKernelGGL((k_dlist_step<N, NC, R, P2>), dim3((unsigned)(ex.nfold + ex.nhalo + h->lgrid_d)), dim3(256), 0,
+                           h->stream, m, phi, mu, dphi, h->fs, h->ps, (const int32_t *)h->clist, lc + 1, ex);
       }
       {
         ProfScope ps(h, GP_KERNEL_CIFACE);
         if (stats)
           hipLaunchKernelGGL((k_ilist<N, NC, R, P2, true>), dim3(h->lgrid_i), dim3(256), 0, h->stream, m, phi, mu,
-                             dphi, codes, phi_o, mu_o, codes_o, h->partials + cell_ipart(h), cstride, h->fs, h->ps,
-                             (const int32_t *)h->ilist, lc);
+                             dphi, codes, phi_o, mu_o, codes_o, cell_partials<N, NC>(h) + cell_ipart(h), cstride,
+                             h->fs, h->ps, (const int32_t *)h->ilist, lc,
+                             (const uint64_t *)h->mlist, (const int *)image_count(h));
         else
           hipLaunchKernelGGL((k_ilist<N, NC, R, P2, false>), dim3(h->lgrid_i), dim3(256), 0, h->stream, m, phi, mu,
-                             dphi, codes, phi_o, mu_o, codes_o, h->partials + cell_ipart(h), cstride, h->fs, h->ps,
-                             (const int32_t *)h->ilist, lc);
+                             dphi, codes, phi_o, mu_o, codes_o, cell_partials<N, NC>(h) + cell_ipart(h), cstride,
+                             h->fs, h->ps, (const int32_t *)h->ilist, lc,
+                             (const uint64_t *)h->mlist, (const int *)image_count(h));
       }
-      /* the new state's halo, from the interior cells both kernels wrote; with the statistics fold when asked */
-      const int64_t nh = halo_cells(mx, my);
-      if (stats) {
-        ProfScope ps(h, GP_KERNEL_STATS);
-        hipLaunchKernelGGL((k_stats_halo<N, NC, R, false>),
-                           dim3((unsigned)(3 * N + 3 * NC + 1 +
-                                           kHaloPlanes<N, NC, false> * ((nh + kStatThreads - 1) / kStatThreads))),
-                           dim3(kStatThreads), 0, h->stream, h->partials, cstride, cstride, h->stats_dev, phi_o, mu_o,
-                           codes_o, (float *)nullptr, (int8_t *)nullptr, h->maps, h->fs, h->ps, mx, my);
-      } else {
-        ProfScope ps(h, GP_KERNEL_HALO);
-        hipLaunchKernelGGL((k_halo<N, NC, R, false>), dim3((unsigned)((nh + 255) / 256), kHaloPlanes<N, NC, false>),
-                           dim3(256), 0, h->stream,
-                           phi_o, mu_o, codes_o, (float *)nullptr, (int8_t *)nullptr, h->maps, h->fs, h->ps, mx, my);
-      }
+      step_partials_done(h, stats);
       HIPCHK(h, hipGetLastError());
       h->cur = 1 - h->cur;
       h->ccur = 1 - h->ccur;
@@ -704,6 +669,7 @@ static int launch_step_c(gp_handle *h, int mode) {
   dim3 g1((unsigned)((my + 2 + kBX - 1) / kBX), (unsigned)((mx + 2 + kBY - 1) / kBY));
   dim3 g2((unsigned)((my + kBX - 1) / kBX), (unsigned)((mx + kBY - 1) / kBY));
   int rc;
+  if (mode == MODE_STATS_FOLD) return launch_stats_fold<N, NC>(h);
   if (mode == MODE_DPHI_PREV) {
     const int b = 1 - h->cur;
     if ((rc = c32_wide_buffer(h, 0)) || (rc = c32_widen_state(h, b, h->wide[0]))) return rc;
@@ -757,34 +723,25 @@ static int launch_step_c(gp_handle *h, int mode) {
   const int *lc = launch_cbulk<N, NC, float, P2, true>(h, m, stats);
   {
     ProfScope ps(h, GP_KERNEL_DPHI);
-    hipLaunchKernelGGL((k_dlist_c<N, NC, P2>), dim3(h->lgrid_d), dim3(256), 0, h->stream, md, phi, plo, mu, mlo, dphi,
-                       fs, h->ps, (const int32_t *)h->clist, lc + 1);
+    const StepExtras<float> ex =
+        step_extras_of<N, NC, float>(h, stats, codes, NewState<float>{phi_o, mu_o, codes_o, plo_o, mlo_o});
+    hipLaunchKernelGGL((k_dlist_c<N, NC, P2>), dim3((unsigned)(ex.nfold + ex.nhalo + h->lgrid_d)), dim3(256), 0, h->stream,
+                       md, phi, plo, mu, mlo, dphi, fs, h->ps, (const int32_t *)h->clist, lc + 1, ex);
   }
   {
     ProfScope ps(h, GP_KERNEL_CIFACE);
     if (stats)
       hipLaunchKernelGGL((k_ilist_c<N, NC, P2, true>), dim3(h->lgrid_i), dim3(256), 0, h->stream, md, phi, plo, mu,
-                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, h->partials + cell_ipart(h),
-                         cstride, fs, h->ps, (const int32_t *)h->ilist, lc);
+                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, cell_partials<N, NC>(h) + cell_ipart(h),
+                         cstride, fs, h->ps, (const int32_t *)h->ilist, lc,
+                             (const uint64_t *)h->mlist, (const int *)image_count(h));
     else
       hipLaunchKernelGGL((k_ilist_c<N, NC, P2, false>), dim3(h->lgrid_i), dim3(256), 0, h->stream, md, phi, plo, mu,
-                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, h->partials + cell_ipart(h),
-                         cstride, fs, h->ps, (const int32_t *)h->ilist, lc);
+                         mlo, (const double *)dphi, codes, phi_o, plo_o, mu_o, mlo_o, codes_o, cell_partials<N, NC>(h) + cell_ipart(h),
+                         cstride, fs, h->ps, (const int32_t *)h->ilist, lc,
+                             (const uint64_t *)h->mlist, (const int *)image_count(h));
   }
-  const int64_t nh = halo_cells(mx, my);
-  if (stats) {
-    ProfScope ps(h, GP_KERNEL_STATS);
-    hipLaunchKernelGGL((k_stats_halo<N, NC, float, true>),
-                       dim3((unsigned)(3 * N + 3 * NC + 1 +
-                                       kHaloPlanes<N, NC, true> * ((nh + kStatThreads - 1) / kStatThreads))),
-                       dim3(kStatThreads), 0, h->stream, h->partials, cstride, cstride, h->stats_dev, phi_o, mu_o,
-                       codes_o, plo_o, mlo_o, h->maps, fs, h->ps, mx, my);
-  } else {
-    ProfScope ps(h, GP_KERNEL_HALO);
-    hipLaunchKernelGGL((k_halo<N, NC, float, true>), dim3((unsigned)((nh + 255) / 256), kHaloPlanes<N, NC, true>),
-                       dim3(256), 0, h->stream,
-                       phi_o, mu_o, codes_o, plo_o, mlo_o, h->maps, fs, h->ps, mx, my);
-  }
+  step_partials_done(h, stats);
   HIPCHK(h, hipGetLastError());
   h->cur = 1 - h->cur;
   h->ccur = 1 - h->ccur;
