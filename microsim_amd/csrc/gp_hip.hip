@@ -249,6 +249,47 @@ static int state_load(gp_handle *h, const double *src) {
   return GP_OK;
 }
 
+/* The handle's state pointers, bound to stored states (state_save's layout) for a while. direct: steps may run from one
+ * stored state into another, which holds when every halo cell is written by a step (a cell without a proxy keeps what an
+ * upload left there) and by the cell-classified step, whose output buffer needs no earlier contents. */
+struct StateBinding {
+  gp_handle *h;
+  void *phi[2], *mu[2];
+  int8_t *lo[2];
+  bool direct;
+  explicit StateBinding(gp_handle *hh) : h(hh), direct(hh->use_cells) {
+    for (int b = 0; b < 2; b++) {
+      phi[b] = h->phi[b];
+      mu[b] = h->mu[b];
+      lo[b] = h->lo[b];
+    }
+    const Maps &m = h->maps;
+    for (int f = 0; f < 2; f++)
+      for (int k = 0; k < 6; k++) {
+        int bx = 0, by = 0; /* earlier images of the same row or column: a step writes two (halo_source) */
+        for (int j = 0; j < k; j++) {
+          bx += m.sx[f][j] == m.sx[f][k];
+          by += m.sy[f][j] == m.sy[f][k];
+        }
+        if (bx >= 2 || by >= 2) direct = false;
+      }
+  }
+  void bind(int b, double *state) {
+    const size_t es = esize(h), pb = (size_t)h->N * h->fs * es, mb = (size_t)h->NC * h->fs * es;
+    h->phi[b] = state;
+    h->mu[b] = (char *)state + pb;
+    if (h->precision == GP_FP32C) h->lo[b] = (int8_t *)state + pb + mb;
+  }
+  void release() {
+    for (int b = 0; b < 2; b++) {
+      h->phi[b] = phi[b];
+      h->mu[b] = mu[b];
+      h->lo[b] = lo[b];
+    }
+  }
+  ~StateBinding() { release(); }
+};
+
 /* GP_ADJOINT_CHECK: the smallest index of a non-finite value of g[0, n) into out[0] (atomicMin; stays at ~0 when
  * there is none) and the largest |g| among the finite ones, as the bits of a non-negative double, into out[1] */
 static __global__ __launch_bounds__(256) void k_adj_scan(const double *__restrict__ g, int64_t n,
@@ -479,38 +520,39 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
   const size_t pn = (size_t)h->N * h->fs * es, mn = (size_t)h->NC * h->fs * es;
   hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   bool ok = e == hipSuccess;
-  ok = ok && hipMalloc(&h->phi[0], pn) == hipSuccess && hipMalloc(&h->phi[1], pn) == hipSuccess;
-  ok = ok && hipMalloc(&h->mu[0], mn) == hipSuccess && hipMalloc(&h->mu[1], mn) == hipSuccess;
-  ok = ok && hipMalloc(&h->dphi, (size_t)h->N * h->fs * dphi_esize(h)) == hipSuccess;
+  Arena *mem = h->mem = new Arena();
+  for (int b = 0; b < 2; b++) {
+    mem->take(&h->phi[b], pn);
+    mem->take(&h->mu[b], mn);
+    if (precision == GP_FP32C) mem->take(&h->lo[b], c32_lo_bytes(h));
+    mem->take(&h->flags[b], sizeof(int) * h->march_nwaves);
+    mem->take(&h->codes[b], (size_t)h->rx * h->ps);
+  }
+  mem->take(&h->dphi, (size_t)h->N * h->fs * dphi_esize(h));
   if (params->tempgrady) {
     const size_t rt = precision == GP_FP64 ? sizeof(RowThermo<double>) : sizeof(RowThermo<float>);
-    ok = ok && hipMalloc((void **)&h->trow, (size_t)h->ry * sizeof(double)) == hipSuccess &&
-         hipMalloc(&h->thp, (size_t)h->ry * rt) == hipSuccess && hipMalloc(&h->thc, (size_t)h->ry * rt) == hipSuccess;
+    mem->take(&h->trow, (size_t)h->ry * sizeof(double));
+    mem->take(&h->thp, (size_t)h->ry * rt);
+    mem->take(&h->thc, (size_t)h->ry * rt);
   }
-  if (params->shift) ok = ok && hipMalloc((void **)&h->front, sizeof(int)) == hipSuccess;
-  if (precision == GP_FP32C)
-    ok = ok && hipMalloc((void **)&h->lo[0], c32_lo_bytes(h)) == hipSuccess &&
-         hipMalloc((void **)&h->lo[1], c32_lo_bytes(h)) == hipSuccess &&
-         hipMalloc(&h->model64, sizeof(Model<double>)) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->partials, sizeof(double) * kNStatMax * h->nparts_max) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->stats_dev, sizeof(double) * kNStatMax) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->inv_dev, sizeof(double) * (GP_MAXNC + 1)) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->flags[0], sizeof(int) * h->march_nwaves) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->flags[1], sizeof(int) * h->march_nwaves) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->tflags, 2 * (size_t)h->cell_nwaves) == hipSuccess;
+  if (params->shift) mem->take(&h->front, sizeof(int));
+  if (precision == GP_FP32C) mem->take(&h->model64, sizeof(Model<double>));
+  mem->take(&h->partials, sizeof(double) * kNStatMax * h->nparts_max);
+  mem->take(&h->stats_dev, sizeof(double) * kNStatMax);
+  mem->take(&h->inv_dev, sizeof(double) * (GP_MAXNC + 1));
+  mem->take(&h->tflags, 2 * (size_t)h->cell_nwaves);
   /* the two cell lists in one piece (8 bytes a cell): between steps it stages the rows of uploads and downloads, the phi
    * planes of a small grid in one run */
   h->stage_bytes = std::max((size_t)h->fs * 2 * sizeof(int32_t),
                             std::min((size_t)h->N * h->fs * sizeof(double), kStageBytes));
-  ok = ok && hipMalloc((void **)&h->clist, h->stage_bytes) == hipSuccess &&
-       hipMalloc((void **)&h->mlist, (size_t)halo_cells(params->mesh_x, params->mesh_y) * 2 * sizeof(uint64_t)) == hipSuccess;
-  h->ilist = ok ? h->clist + h->fs : nullptr;
-  ok = ok && hipMalloc((void **)&h->lcount, 6 * sizeof(int)) == hipSuccess;
-  ok = ok && hipMalloc((void **)&h->codes[0], (size_t)h->rx * h->ps) == hipSuccess &&
-       hipMalloc((void **)&h->codes[1], (size_t)h->rx * h->ps) == hipSuccess;
+  mem->take(&h->clist, h->stage_bytes);
+  mem->take(&h->mlist, (size_t)halo_cells(params->mesh_x, params->mesh_y) * 2 * sizeof(uint64_t));
+  mem->take(&h->lcount, 6 * sizeof(int));
   h->ccur = 0;
   const size_t msize = precision == GP_FP64 ? sizeof(Model<double>) : sizeof(Model<float>);
-  ok = ok && hipMalloc(&h->model, msize) == hipSuccess;
+  mem->take(&h->model, msize);
+  ok = ok && mem->allocate();
+  h->ilist = ok ? h->clist + h->fs : nullptr;
   if (!ok) {
     gp_destroy(h);
     return gp_fail(nullptr, GP_E_OOM, "device allocation failed (%zu bytes per phi copy)", pn);
@@ -588,11 +630,8 @@ void gp_destroy(gp_handle *h) {
   }
   h->prof.clear();
   delete h->adj;
-  void *bufs[] = {h->phi[0], h->phi[1], h->mu[0],    h->mu[1],    h->dphi,   h->partials, h->stats_dev,
-                  h->model,  h->flags[0], h->flags[1], h->inv_dev, h->codes[0], h->codes[1], h->clist,
-                  h->lcount, h->mlist, h->lo[0],    h->lo[1],    h->model64, h->wide[0],  h->wide[1],
-                  h->trow,   h->thp,    h->thc,      h->front,    h->tflags};
-  for (void *b : bufs)
+  delete h->mem;
+  for (double *b : h->wide)
     if (b) (void)hipFree(b);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
@@ -800,12 +839,12 @@ int gp_adjoint_forward(gp_handle *h, int64_t nsteps, int64_t every) {
   A->nsteps = nsteps;
   A->every = every;
   const int64_t nck = (nsteps + every - 1) / every;
+  A->ckpt.resize((size_t)nck);
+  for (double *&b : A->ckpt) A->ckpts.take(&b, state_bytes(h));
+  if (!A->ckpts.allocate())
+    return gp_fail(h, GP_E_OOM, "adjoint: %lld checkpoints do not fit in device memory", (long long)nck);
   for (int64_t k = 0; k < nck; k++) {
-    double *b = nullptr;
-    if (hipMalloc((void **)&b, state_bytes(h)) != hipSuccess)
-      return gp_fail(h, GP_E_OOM, "adjoint: checkpoint %lld does not fit in device memory", (long long)k);
-    A->ckpt.push_back(b);
-    int rc = state_save(h, b);
+    int rc = state_save(h, A->ckpt[(size_t)k]);
     if (!rc) rc = gp_step(h, std::min(every, nsteps - k * every), nullptr);
     if (rc) return rc;
   }
@@ -820,30 +859,28 @@ int gp_adjoint_backward(gp_handle *h, const double *gphi_T, const double *gmu_T,
   const int nth = theta_count(h->N, h->NC);
   const size_t se = state_elems(h);
   if (!A->g[0]) {
-    bool ok = hipMalloc((void **)&A->g[0], se * sizeof(double)) == hipSuccess &&
-              hipMalloc((void **)&A->g[1], se * sizeof(double)) == hipSuccess &&
-              hipMalloc((void **)&A->gdphi, (size_t)h->N * h->fs * sizeof(double)) == hipSuccess &&
-              hipMalloc((void **)&A->gth, sizeof(double) * nth) == hipSuccess &&
-              hipMalloc((void **)&A->cbar, (size_t)h->NC * h->fs * sizeof(double)) == hipSuccess &&
-              hipMalloc((void **)&A->qlist, (size_t)h->fs * sizeof(int32_t)) == hipSuccess &&
-              hipMalloc((void **)&A->plist, (size_t)h->fs * sizeof(int32_t)) == hipSuccess &&
-              hipMalloc((void **)&A->counts, 4 * sizeof(int)) == hipSuccess &&
-              hipMemsetAsync(A->counts, 0, 4 * sizeof(int), h->stream) == hipSuccess &&
-              hipMalloc((void **)&A->pcode, (size_t)h->fs) == hipSuccess &&
-              hipMalloc((void **)&A->bq, (size_t)h->fs) == hipSuccess &&
-              hipMalloc((void **)&A->cand, (size_t)h->fs) == hipSuccess;
-    for (int64_t j = 0; ok && j < std::min(A->every, A->nsteps); j++) {
-      double *b = nullptr;
-      ok = hipMalloc((void **)&b, state_bytes(h)) == hipSuccess;
-      if (ok) A->seg.push_back(b);
+    Arena &w = A->work;
+    const bool other = h->precision != GP_FP64;
+    for (double *&g : A->g) w.take(&g, se * sizeof(double));
+    w.take(&A->gdphi, (size_t)h->N * h->fs * sizeof(double));
+    w.take(&A->gth, sizeof(double) * nth);
+    w.take(&A->cbar, (size_t)h->NC * h->fs * sizeof(double));
+    w.take(&A->qlist, (size_t)h->fs * sizeof(int32_t));
+    w.take(&A->plist, (size_t)h->fs * sizeof(int32_t));
+    w.take(&A->counts, 4 * sizeof(int));
+    for (int8_t **q : {&A->pcode, &A->bq, &A->cand}) w.take(q, (size_t)h->fs);
+    A->seg.resize((size_t)std::max<int64_t>(0, std::min(A->every, A->nsteps) - 1));
+    for (double *&b : A->seg) w.take(&b, state_bytes(h));
+    if (other) {
+      w.take(&A->st64, se * sizeof(double));
+      w.take(&A->dphi64, (size_t)h->N * h->fs * sizeof(double));
+      w.take(&A->model64, sizeof(Model<double>));
     }
-    if (ok && h->precision != GP_FP64) {
+    bool ok = w.allocate() && hipMemsetAsync(w.base(), 0, w.size(), h->stream) == hipSuccess;
+    if (ok && other) {
       Model<double> m;
       make_model(&h->p, &m);
-      ok = hipMalloc((void **)&A->st64, se * sizeof(double)) == hipSuccess &&
-           hipMalloc((void **)&A->dphi64, (size_t)h->N * h->fs * sizeof(double)) == hipSuccess &&
-           hipMalloc(&A->model64, sizeof m) == hipSuccess &&
-           hipMemcpyAsync(A->model64, &m, sizeof m, hipMemcpyHostToDevice, h->stream) == hipSuccess &&
+      ok = hipMemcpyAsync(A->model64, &m, sizeof m, hipMemcpyHostToDevice, h->stream) == hipSuccess &&
            hipStreamSynchronize(h->stream) == hipSuccess;
     }
     if (!ok) return gp_fail(h, GP_E_OOM, "adjoint: buffers do not fit in device memory");
@@ -861,16 +898,29 @@ int gp_adjoint_backward(gp_handle *h, const double *gphi_T, const double *gmu_T,
   const char *ck = getenv("GP_ADJOINT_CHECK");
   const bool check = ck && *ck && strcmp(ck, "0") != 0;
   const int64_t check_every = check ? atoll(ck) : 0;
+  /* A segment's states S[0 .. n) are its checkpoint and the segment buffers, and the handle steps from one into the next
+   * (no copies): its state pointers are bound to them meanwhile and come back on every way out. Nothing of a bound buffer
+   * is taken as kept from an earlier step. */
+  StateBinding own(h);
   for (int64_t k = (int64_t)A->ckpt.size() - 1; k >= 0; k--) {
     const int64_t n = std::min(A->every, A->nsteps - k * A->every);
-    if ((rc = state_load(h, A->ckpt[k]))) return rc;
-    for (int64_t j = 0; j < n; j++) {
-      if ((rc = state_save(h, A->seg[j]))) return rc;
-      if (j + 1 < n && (rc = gp_step(h, 1, nullptr))) return rc;
+    const auto S = [&](int64_t j) { return j == 0 ? A->ckpt[(size_t)k] : A->seg[(size_t)(j - 1)]; };
+    if (!own.direct) {
+      own.release();
+      if ((rc = state_load(h, S(0)))) return rc;
+    } else {
+      own.bind(h->cur, S(0));
+      h->codes_valid = h->flags_valid = false;
+    }
+    for (int64_t j = 0; j + 1 < n; j++) {
+      if (own.direct) own.bind(1 - h->cur, S(j + 1));
+      h->prev_valid = false;
+      if ((rc = gp_step(h, 1, nullptr))) return rc;
+      if (!own.direct && (rc = state_save(h, S(j + 1)))) return rc;
     }
     for (int64_t j = n - 1; j >= 0; j--) {
       ProfScope ps(h, GP_KERNEL_ADJ);
-      if ((rc = state_load(h, A->seg[j]))) return rc;
+      own.bind(h->cur, S(j));
       if (wide) {
         const double *p64 = (const double *)h->phi[h->cur], *m64 = (const double *)h->mu[h->cur];
         if ((rc = h->ops->adj_dphi(h, p64, m64, (double *)h->dphi, h->model))) return rc;
@@ -888,6 +938,8 @@ int gp_adjoint_backward(gp_handle *h, const double *gphi_T, const double *gmu_T,
       }
     }
   }
+  own.release();
+  if (!A->ckpt.empty() && (rc = state_load(h, A->ckpt[0]))) return rc;
   if ((rc = adj_fold(h))) return rc;
   if ((rc = rows_to_host(h, PACK_F64, gphi_0, A->g[1], nullptr, h->N))) return rc;
   if ((rc = rows_to_host(h, PACK_F64, gmu_0, A->g[1] + (size_t)h->N * h->fs, nullptr, h->NC))) return rc;
