@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256) void k_adj_codes(const double *__restrict__ ph
   list_append(cand, (int32_t)c, plist, pcount);
 }
 
-/* Stage P transposed by reverse mode (gp_reverse.h: phi_delta_vjp), one pass per listed candidate (k_adj_codes'
+/* Stage P transposed by reverse mode (gp_reverse.h: phi_delta_vjp_pairs), one pass per listed candidate (k_adj_codes'
  * list) with a nonzero delta-phi adjoint */
 template <int N, int NC, bool P2>
 __global__ __launch_bounds__(256) void k_adj_prev(const Model<double> *__restrict__ mp, const double *__restrict__ phi,
@@ -432,10 +432,9 @@ __global__ __launch_bounds__(256) void k_adj_prev(const Model<double> *__restric
                                                   double *gphi, double *gmu, double *gtheta,
                                                   const int32_t *__restrict__ list, const int *__restrict__ count,
                                                   int64_t fs, int64_t ps) {
-  constexpr int NTH = kThetaN<N, NC>;
-  double th[NTH];
-  for (int t = 0; t < NTH; t++) th[t] = 0.0;
   const Model<double> &m = *mp;
+  RevAcc<N, NC> acc; /* theta accumulates over the thread's cells */
+  acc.clear();
   const int n = *count;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int64_t c = list[i];
@@ -448,13 +447,16 @@ __global__ __launch_bounds__(256) void k_adj_prev(const Model<double> *__restric
     if (!nz) continue; /* a candidate with no incoming delta-phi adjoint */
     RegStore<N, NC, double> rs;
     gather_stencil<N, NC>(phi, mu, nullptr, c, fs, ps, rs);
-    RevAcc<N, NC> acc;
-    acc.clear();
-    phi_delta_vjp<N, NC>(m, RegView<N, NC, double, P2>{&rs, 0, 0}, go, acc);
-    scatter_acc<N, NC>(acc, c, fs, ps, gphi, gmu, nullptr);
-    for (int t = 0; t < NTH; t++) th[t] += acc.th[t];
+#pragma unroll
+    for (int k = 0; k < NC; k++) acc.m(k, 0, 0) = 0.0;
+    phi_delta_vjp_pairs<N, NC>(m, RegView<N, NC, double, P2>{&rs, 0, 0}, go, acc, [&](int a, int di, int dj, double v) {
+      if (v != 0.0) atomicAdd(&gphi[a * fs + c + di * ps + dj], v);
+    });
+#pragma unroll
+    for (int k = 0; k < NC; k++)
+      if (acc.m(k, 0, 0) != 0.0) atomicAdd(&gmu[k * fs + c], acc.m(k, 0, 0));
   }
-  theta_flush<NTH>(th, NTH, gtheta);
+  theta_flush<kThetaN<N, NC>>(acc.th, kThetaN<N, NC>, gtheta);
 }
 
 /* Stage B transposed over the allocated grid; blockIdx.z is the field group (0: the N phi planes at g, 1: the NC mu

@@ -103,31 +103,12 @@ GP_HD void pair_face(const Model<R> &m, const PairCoef<R> &k, const V &v, int i,
   }
 }
 
-/* delta-phi of the centre cell: phi_delta (not its smoothing form). V: a RegView. */
-template <int N, int NC, typename R, class V>
-GP_HD void phi_delta_pairs(const Model<R> &m, const V &v, R *out) {
-  R phi[N], divphi[N];
-  bool any = false;
-  unsigned active = 0u;
-#pragma unroll
-  for (int a = 0; a < N; a++) {
-    phi[a] = v.ph(a, 0, 0);
-    divphi[a] = divx<V>(m, (gx(m, v, a, 0, 0) - gx(m, v, a, -1, 0)));
-    divphi[a] += divy<V>(m, (gy(m, v, a, 0, 0) - gy(m, v, a, 0, -1)));
-    const bool on = fabs(divphi[a]) > R(0.0);
-    any = any || on;
-    active |= on ? 1u << a : 0u;
-  }
-  if (!any) {
-    /* no lambda, no tau; the projection still clamps a negative phi (its < 0 test is not gated) */
-#pragma unroll
-    for (int a = 0; a < N; a++) out[a] = R(0.0);
-    project_simplex<N>(phi, divphi, out);
-    return;
-  }
+/* the pairs to visit, bit a N + b: a < b with both present and `on` set for one of them, or (coefficients that are not
+ * symmetric) every ordered pair of an `on` phase a */
+template <int N, typename R, class V>
+GP_HD unsigned pairs_to_visit(const Model<R> &m, const V &v, unsigned on) {
   const bool sym = m.pairs_sym != 0;
   const unsigned present = sym ? phases_present<N, R>(v) : (1u << N) - 1u;
-  /* the pairs to visit, bit a N + b: a < b with both present and one active, or every ordered pair of an active a */
   unsigned todo = 0u;
 #pragma unroll
   for (int a = 0; a < N; a++)
@@ -135,9 +116,75 @@ GP_HD void phi_delta_pairs(const Model<R> &m, const V &v, R *out) {
     for (int b = 0; b < N; b++) {
       if (b == a) continue;
       const bool both = (present >> a) & (present >> b) & 1u;
-      const bool on = (active >> a) & 1u, onb = (active >> b) & 1u;
-      if (a < b ? both && (on || (sym && onb)) : !sym && on) todo |= 1u << (a * N + b);
+      const bool ona = (on >> a) & 1u, onb = (on >> b) & 1u;
+      if (a < b ? both && (ona || (sym && onb)) : !sym && ona) todo |= 1u << (a * N + b);
     }
+  return todo;
+}
+
+/* the stencils of phases a and b of v as phases 0 and 1 */
+template <int N, typename R, class V>
+GP_HD void pair_stencil(const V &v, int a, int b, RegStore<2, 0, R> &rs) {
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      rs.p[0][i][j] = pick<N>(a, [&](int c) { return v.ph(c, i - 1, j - 1); });
+      rs.p[1][i][j] = pick<N>(b, [&](int c) { return v.ph(c, i - 1, j - 1); });
+    }
+}
+
+/* the coefficients of pair p = a N + b */
+template <int N, typename R>
+GP_HD PairCoef<R> pair_coef(const Model<R> &m, int p) {
+  PairCoef<R> k;
+  auto load = [&](auto coef) {
+    k.gamma = coef([&](int i, int j) { return m.gamma[i][j]; });
+    if (!m.fn_aniso) return;
+    k.dab = coef([&](int i, int j) { return m.dab[i][j]; });
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        k.rot[r][c] = coef([&](int i, int j) { return m.rot[i][j][r][c]; });
+        k.rot_inv[r][c] = coef([&](int i, int j) { return m.rot_inv[i][j][r][c]; });
+      }
+  };
+  if (m.pairs_sym) {
+    /* wave-uniform coefficients of the pairs i < j, picked per lane */
+    load([&](auto f) {
+      R r = f(0, 1);
+#pragma unroll
+      for (int i = 0; i < N; i++)
+#pragma unroll
+        for (int j = i + 1; j < N; j++) {
+          const R x = f(i, j);
+          r = p == i * N + j ? x : r;
+        }
+      return r;
+    });
+  } else {
+    load([&](auto f) { return f(p / N, p % N); });
+  }
+  return k;
+}
+
+/* delta-phi of the centre cell before the simplex projection, with phi, its Laplacians, psi and the active phases (those of
+ * nonzero Laplacian; none: out is zero and psi is not formed). V: a RegView. */
+template <int N, int NC, typename R, class V>
+GP_HD unsigned phi_rates_pairs(const Model<R> &m, const V &v, R *phi, R *divphi, R *psi, R *out) {
+  unsigned active = 0u;
+#pragma unroll
+  for (int a = 0; a < N; a++) {
+    phi[a] = v.ph(a, 0, 0);
+    divphi[a] = divx<V>(m, (gx(m, v, a, 0, 0) - gx(m, v, a, -1, 0)));
+    divphi[a] += divy<V>(m, (gy(m, v, a, 0, 0) - gy(m, v, a, 0, -1)));
+    active |= fabs(divphi[a]) > R(0.0) ? 1u << a : 0u;
+    out[a] = R(0.0);
+  }
+  if (!active) return 0u; /* no lambda, no tau */
+  const bool sym = m.pairs_sym != 0;
+  unsigned todo = pairs_to_visit<N>(m, v, active);
   R A1[N], A2[N], D1[N], D2[N];
 #pragma unroll
   for (int a = 0; a < N; a++) A1[a] = A2[a] = D1[a] = D2[a] = R(0.0);
@@ -145,42 +192,8 @@ GP_HD void phi_delta_pairs(const Model<R> &m, const V &v, R *out) {
     const int p = __builtin_ctz(todo), a = p / N, b = p % N;
     todo &= todo - 1u;
     RegStore<2, 0, R> rs;
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int j = 0; j < 3; j++) {
-        rs.p[0][i][j] = pick<N>(a, [&](int c) { return v.ph(c, i - 1, j - 1); });
-        rs.p[1][i][j] = pick<N>(b, [&](int c) { return v.ph(c, i - 1, j - 1); });
-      }
-    PairCoef<R> k;
-    auto load = [&](auto coef) {
-      k.gamma = coef([&](int i, int j) { return m.gamma[i][j]; });
-      if (!m.fn_aniso) return;
-      k.dab = coef([&](int i, int j) { return m.dab[i][j]; });
-#pragma unroll
-      for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-          k.rot[r][c] = coef([&](int i, int j) { return m.rot[i][j][r][c]; });
-          k.rot_inv[r][c] = coef([&](int i, int j) { return m.rot_inv[i][j][r][c]; });
-        }
-    };
-    if (sym) {
-      /* wave-uniform coefficients of the pairs i < j, picked per lane */
-      load([&](auto f) {
-        R r = f(0, 1);
-#pragma unroll
-        for (int i = 0; i < N; i++)
-#pragma unroll
-          for (int j = i + 1; j < N; j++) {
-            const R x = f(i, j);
-            r = p == i * N + j ? x : r;
-          }
-        return r;
-      });
-    } else {
-      load([&](auto f) { return f(a, b); });
-    }
+    pair_stencil<N>(v, a, b, rs);
+    const PairCoef<R> k = pair_coef<N>(m, p);
     const RegView<2, 0, R, V::kPow2, V::kFast> w{&rs, 0, 0};
     /* the centre term dA/dphi: x1 + x2 of phase a, y1 + y2 of phase b */
     R x1, x2 = R(0.0), y1, y2 = R(0.0);
@@ -239,7 +252,7 @@ GP_HD void phi_delta_pairs(const Model<R> &m, const V &v, R *out) {
       D2[c] += ia ? u2 : ib ? w2 : R(0.0);
     }
   }
-  R mu[NC > 0 ? NC : 1], psi[N];
+  R mu[NC > 0 ? NC : 1];
 #pragma unroll
   for (int k = 0; k < NC; k++) mu[k] = v.m(k, 0, 0);
   psi_all<N, NC>(m, mu, psi);
@@ -262,6 +275,15 @@ GP_HD void phi_delta_pairs(const Model<R> &m, const V &v, R *out) {
   const R den = tau_of<N>(m, phi) * m.eps;
 #pragma unroll
   for (int a = 0; a < N; a++) out[a] = (active >> a) & 1u ? qdiv(m.dt * (lambda[a] - sum_lambda), den) : R(0.0);
+  return active;
+}
+
+/* delta-phi of the centre cell: phi_delta (not its smoothing form; the projection clamps a negative phi of an inactive
+ * phase too). V: a RegView. */
+template <int N, int NC, typename R, class V>
+GP_HD void phi_delta_pairs(const Model<R> &m, const V &v, R *out) {
+  R phi[N], divphi[N], psi[N];
+  phi_rates_pairs<N, NC>(m, v, phi, divphi, psi, out);
   project_simplex<N>(phi, divphi, out);
 }
 

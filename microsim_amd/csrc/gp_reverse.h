@@ -24,6 +24,7 @@
 #pragma once
 
 #include "gp_model.h"
+#include "gp_pairs.h"
 
 namespace gpk {
 
@@ -592,6 +593,214 @@ GP_HD void phi_delta_vjp(const Model<double> &m, const V &v, const double *gout,
     add_cx(m, acc, a, 0, 0, gcx[a]);
     add_cy(m, acc, a, 0, 0, gcy[a]);
   }
+}
+
+/* ---------------------------------------------------------------- stage P by phase pairs
+ * phi_delta_vjp visits the ordered pairs (a, b), forward and back: per pair five anisotropies with their second
+ * derivatives, all of N (N - 1) pairs unrolled, 256 registers, 216 accumulation registers and a scratch frame. With
+ * q_ba = -q_ab the terms of (a, b) and (b, a) join: a face contributes (S1 + S2) W, S1 = a_c^2 r_n,
+ * S2 = a_c |q|^2 (R^-1 G)_n, W = lambda'_b s_a - lambda'_a s_b, and the centre gamma (a_c^2 q + a_c |q|^2 G) . R z,
+ * z = lambda'_a grad phi_b - lambda'_b grad phi_a (lambda' the adjoints of lambda). A pair with an absent phase has
+ * neither value nor derivative (each term is of second order in that phase), so the pairs of gp_pairs.h are visited.
+ * k_adj_prev: 256^2 binary 42.2 -> 13.4 us, 1024^2 ternary 118 -> 27.5 us (bound by one wavefront per SIMD). */
+
+/* one face of the pair, transposed: s the face's weight (its sign and spacing; the pair's gamma apart), la and lb the adjoints
+ * of lambda_a and lambda_b; adds to gf, gdab and ggam */
+GP_HD void pair_face_vjp(bool aniso, const PairCoef<double> &k, int n, const FaceIn &f, double s, double la, double lb,
+                         FaceIn &gf, double &gdab, double &ggam) {
+  const int t = 1 - n;
+  double r[2];
+  r[n] = f.sa * f.gb - f.sb * f.ga;
+  r[t] = 0.5 * (f.sa * f.Cb - f.sb * f.Ca);
+  const double W = lb * f.sa - la * f.sb, gS = s * k.gamma * W;
+  double gr[2] = {0.0, 0.0}, S = r[n];
+  if (aniso) {
+    double q[2], rg[2], rg0[2], gq[2];
+    rot2(k.rot, r, q);
+    const AcTerms a = ac_terms(k.dab, q);
+    rot2(k.rot_inv, a.G, rg);
+    rot2(k.rot_inv, a.G0, rg0);
+    const double q2 = q[0] * q[0] + q[1] * q[1];
+    S = a.ac * a.ac * r[n] + a.ac * q2 * rg[n];
+    for (int j = 0; j < 2; j++) {
+      const double HRi = a.H[j][0] * k.rot_inv[n][0] + a.H[j][1] * k.rot_inv[n][1];
+      gq[j] = gS * (2.0 * a.ac * a.G[j] * r[n] + a.G[j] * q2 * rg[n] + a.ac * 2.0 * q[j] * rg[n] + a.ac * q2 * HRi);
+    }
+    rot2t(k.rot, gq, gr);
+    gr[n] += gS * a.ac * a.ac;
+    gdab += gS * (2.0 * a.ac * a.dac * r[n] + a.dac * q2 * rg[n] + a.ac * q2 * rg0[n]);
+  } else {
+    gr[n] = gS;
+  }
+  ggam += s * S * W;
+  const double gW = s * k.gamma * S;
+  gf.sa = lb * gW + gr[n] * f.gb + 0.5 * gr[t] * f.Cb;
+  gf.sb = -(la * gW) - (gr[n] * f.ga + 0.5 * gr[t] * f.Ca);
+  gf.gb = gr[n] * f.sa;
+  gf.ga = -gr[n] * f.sb;
+  gf.Cb = 0.5 * gr[t] * f.sa;
+  gf.Ca = -0.5 * gr[t] * f.sb;
+}
+
+/* phi_delta_vjp by pairs: acc.th and acc.m(k, 0, 0) accumulate as there; the adjoint of phi leaves through
+ * emit(phase, i, j, value), where the phase of a pair's terms varies from lane to lane. */
+template <int N, int NC, class V, class F>
+GP_HD void phi_delta_vjp_pairs(const Model<double> &m, const V &v, const double *gout, RevAcc<N, NC> &acc, F emit) {
+  double phi[N], divphi[N], psi[N], out[N], g[N], gphi[N];
+  const unsigned active = phi_rates_pairs<N, NC>(m, v, phi, divphi, psi, out);
+#pragma unroll
+  for (int a = 0; a < N; a++) {
+    g[a] = gout[a];
+    gphi[a] = 0.0;
+  }
+  project_simplex_vjp<N>(phi, divphi, out, g, gphi);
+  if (active) {
+    /* out_a = dt (lambda_a - mean) / (tau eps) */
+    const double tauv = tau_of<N>(m, phi), sc = m.dt / (tauv * m.eps);
+    double glam[N], gmean = 0.0, gtau = 0.0;
+    int count = 0;
+#pragma unroll
+    for (int a = 0; a < N; a++) {
+      glam[a] = 0.0;
+      if ((active >> a) & 1u) {
+        glam[a] = g[a] * sc;
+        gmean -= g[a] * sc;
+        gtau -= g[a] * out[a] / tauv;
+        count++;
+      }
+    }
+    tau_vjp<N, NC>(m, phi, gtau, gphi, acc);
+    gmean /= (double)count;
+    unsigned on = 0u;
+#pragma unroll
+    for (int a = 0; a < N; a++) {
+      if ((active >> a) & 1u) glam[a] += gmean;
+      on |= glam[a] != 0.0 ? 1u << a : 0u;
+    }
+    /* lambda_a = eps (-dA + dD) - w' / eps - sum_b psi_b dh_b/dphi_a: the last two */
+    double gpsi[N], gmu[NC > 0 ? NC : 1], mu[NC > 0 ? NC : 1];
+#pragma unroll
+    for (int a = 0; a < N; a++) gpsi[a] = 0.0;
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+      gmu[k] = 0.0;
+      mu[k] = v.m(k, 0, 0);
+    }
+#pragma unroll
+    for (int a = 0; a < N; a++)
+      if ((on >> a) & 1u) {
+        dwdphi_vjp<N, NC>(m, phi, divphi, a, -m.inv_eps * glam[a], gphi, acc);
+#pragma unroll
+        for (int b = 0; b < N; b++) {
+          gpsi[b] -= glam[a] * dhphi<N>(phi, b, a);
+#pragma unroll
+          for (int e = 0; e < N; e++) gphi[e] -= glam[a] * psi[b] * d2hphi<N>(phi, b, a, e);
+        }
+      }
+    psi_vjp<N, NC>(m, mu, gpsi, gmu);
+#pragma unroll
+    for (int k = 0; k < NC; k++) acc.m(k, 0, 0) += gmu[k];
+    unsigned todo = pairs_to_visit<N>(m, v, on);
+    while (todo) {
+      const int p = __builtin_ctz(todo), a = p / N, b = p % N;
+      todo &= todo - 1u;
+      RegStore<2, 0, double> rs;
+      pair_stencil<N>(v, a, b, rs);
+      const PairCoef<double> k = pair_coef<N>(m, p);
+      const RegView<2, 0, double, V::kPow2, V::kFast> w{&rs, 0, 0};
+      const double la = pick<N>(a, [&](int c) { return glam[c]; });
+      const double lb = m.pairs_sym ? pick<N>(b, [&](int c) { return glam[c]; }) : 0.0;
+      double gdab = 0.0, ggam = 0.0;
+      RevAcc<2, 1> loc;
+      loc.clear();
+      {
+        const double ua[2] = {cx(m, w, 0, 0, 0), cy(m, w, 0, 0, 0)}, ub[2] = {cx(m, w, 1, 0, 0), cy(m, w, 1, 0, 0)};
+        const double pa = w.ph(0, 0, 0), pb = w.ph(1, 0, 0);
+        const double e = -2.0 * m.eps, ea = e * la, eb = e * lb;
+        const double r[2] = {pa * ub[0] - pb * ua[0], pa * ub[1] - pb * ua[1]};
+        const double z[2] = {ea * ub[0] - eb * ua[0], ea * ub[1] - eb * ua[1]};
+        double gr[2], gz[2];
+        if (m.fn_aniso) {
+          double q[2], Z[2], gq[2], gZ[2];
+          rot2(k.rot, r, q);
+          rot2(k.rot, z, Z);
+          const AcTerms t = ac_terms(k.dab, q);
+          const double q2 = q[0] * q[0] + q[1] * q[1];
+          const double qZ = q[0] * Z[0] + q[1] * Z[1], GZ = t.G[0] * Z[0] + t.G[1] * Z[1];
+          const double G0Z = t.G0[0] * Z[0] + t.G0[1] * Z[1];
+          for (int j = 0; j < 2; j++) {
+            const double HZ = t.H[j][0] * Z[0] + t.H[j][1] * Z[1];
+            gq[j] = k.gamma * (2.0 * t.ac * t.G[j] * qZ + t.ac * t.ac * Z[j] + t.G[j] * q2 * GZ +
+                               t.ac * 2.0 * q[j] * GZ + t.ac * q2 * HZ);
+            gZ[j] = k.gamma * (t.ac * t.ac * q[j] + t.ac * q2 * t.G[j]);
+          }
+          ggam += t.ac * t.ac * qZ + t.ac * q2 * GZ;
+          gdab += k.gamma * (2.0 * t.ac * t.dac * qZ + t.dac * q2 * GZ + t.ac * q2 * G0Z);
+          rot2t(k.rot, gq, gr);
+          rot2t(k.rot, gZ, gz);
+        } else {
+          for (int j = 0; j < 2; j++) {
+            gr[j] = k.gamma * z[j];
+            gz[j] = k.gamma * r[j];
+          }
+          ggam += r[0] * z[0] + r[1] * z[1];
+        }
+        loc.ph(0, 0, 0) += gr[0] * ub[0] + gr[1] * ub[1];
+        loc.ph(1, 0, 0) -= gr[0] * ua[0] + gr[1] * ua[1];
+        add_cx(m, loc, 0, 0, 0, -(pb * gr[0] + eb * gz[0]));
+        add_cy(m, loc, 0, 0, 0, -(pb * gr[1] + eb * gz[1]));
+        add_cx(m, loc, 1, 0, 0, pa * gr[0] + ea * gz[0]);
+        add_cy(m, loc, 1, 0, 0, pa * gr[1] + ea * gz[1]);
+      }
+      const bool aniso = m.fn_aniso != 0;
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const int i = s == 0 ? 0 : -1;
+        const double sg = s == 0 ? 2.0 * m.eps : -2.0 * m.eps;
+        FaceIn gf;
+        const FaceIn fx{sx(m, w, 0, i, 0), sx(m, w, 1, i, 0), gx(m, w, 0, i, 0), gx(m, w, 1, i, 0),
+                        cy(m, w, 0, i, 0) + cy(m, w, 0, i + 1, 0), cy(m, w, 1, i, 0) + cy(m, w, 1, i + 1, 0)};
+        pair_face_vjp(aniso, k, 0, fx, sg * m.inv_dx, la, lb, gf, gdab, ggam);
+        add_sx(loc, 0, i, 0, gf.sa);
+        add_sx(loc, 1, i, 0, gf.sb);
+        add_gx(m, loc, 0, i, 0, gf.ga);
+        add_gx(m, loc, 1, i, 0, gf.gb);
+        add_cy(m, loc, 0, i, 0, gf.Ca);
+        add_cy(m, loc, 0, i + 1, 0, gf.Ca);
+        add_cy(m, loc, 1, i, 0, gf.Cb);
+        add_cy(m, loc, 1, i + 1, 0, gf.Cb);
+        const FaceIn fy{sy(m, w, 0, 0, i), sy(m, w, 1, 0, i), gy(m, w, 0, 0, i), gy(m, w, 1, 0, i),
+                        cx(m, w, 0, 0, i) + cx(m, w, 0, 0, i + 1), cx(m, w, 1, 0, i) + cx(m, w, 1, 0, i + 1)};
+        pair_face_vjp(aniso, k, 1, fy, sg * m.inv_dy, la, lb, gf, gdab, ggam);
+        add_sy(loc, 0, 0, i, gf.sa);
+        add_sy(loc, 1, 0, i, gf.sb);
+        add_gy(m, loc, 0, 0, i, gf.ga);
+        add_gy(m, loc, 1, 0, i, gf.gb);
+        add_cx(m, loc, 0, 0, i, gf.Ca);
+        add_cx(m, loc, 0, 0, i + 1, gf.Ca);
+        add_cx(m, loc, 1, 0, i, gf.Cb);
+        add_cx(m, loc, 1, 0, i + 1, gf.Cb);
+      }
+      /* theta of the pair {a, b}, in pair order */
+#pragma unroll
+      for (int c = 0; c < N; c++)
+#pragma unroll
+        for (int d = c + 1; d < N; d++) {
+          const bool hit = (a == c && b == d) || (a == d && b == c);
+          acc.gamma(c, d) += hit ? ggam : 0.0;
+          acc.dab(c, d) += hit ? gdab : 0.0;
+        }
+#pragma unroll
+      for (int i = -1; i <= 1; i++)
+#pragma unroll
+        for (int j = -1; j <= 1; j++) {
+          emit(a, i, j, loc.ph(0, i, j));
+          emit(b, i, j, loc.ph(1, i, j));
+        }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < N; a++) emit(a, 0, 0, gphi[a]);
 }
 
 /* ---------------------------------------------------------------- anti-trapping current */

@@ -3,6 +3,7 @@
 #include <cmath>
 
 #include "gp_pairs.h"
+#include "gp_reverse.h"
 
 using namespace gpk;
 
@@ -59,5 +60,43 @@ extern "C" int pairs_check(const gp_params *p, int form, const double *in, doubl
   if (N == 3 && NC == 2) return pick_form<3, 2>(p, form, in, out);
   if (N == 4 && NC == 2) return pick_form<4, 2>(p, form, in, out);
   if (N == 3 && NC == 3) return pick_form<3, 3>(p, form, in, out);
+  return -2;
+}
+
+// Stage P transposed, of the same cell: the adjoint gout[N] follows the cell's values in `in`. Writes (full loops, by pairs)
+// of the stencil adjoint, the mu adjoint and theta; returns the number of values.
+template <int N, int NC>
+static int compare_vjp(const gp_params *p, const double *in, double *out) {
+  Model<double> m;
+  if (make_model(p, &m)) return -1;
+  RegStore<N, NC, double> rs;
+  for (int a = 0; a < N; a++)
+    for (int i = 0; i < 9; i++) rs.p[a][i / 3][i % 3] = *in++;
+  for (int k = 0; k < NC; k++)
+    for (int o = 0; o < 5; o++) rs.u[k][o] = *in++;
+  in += 5 * N + 1;
+  const RegView<N, NC, double, false> v{&rs, 0, 0};
+  RevAcc<N, NC> r, q;
+  r.clear();
+  q.clear();
+  phi_delta_vjp<N, NC>(m, v, in, r);
+  phi_delta_vjp_pairs<N, NC>(m, v, in, q, [&](int a, int i, int j, double x) { q.ph(a, i, j) += x; });
+  int n = 0;
+  auto put = [&](double x, double y) {
+    out[n++] = x;
+    out[n++] = y;
+  };
+  for (int a = 0; a < N; a++)
+    for (int i = 0; i < 9; i++) put(r.p[a][i / 3][i % 3], q.p[a][i / 3][i % 3]);
+  for (int k = 0; k < NC; k++) put(r.u[k][0], q.u[k][0]);
+  for (int t = 0; t < kThetaN<N, NC>; t++) put(r.th[t], q.th[t]);
+  return n;
+}
+extern "C" int pairs_check_vjp(const gp_params *p, const double *in, double *out) {
+  const int N = p->nphases, NC = p->ncomp - 1;
+  if (N == 2 && NC == 1) return compare_vjp<2, 1>(p, in, out);
+  if (N == 3 && NC == 2) return compare_vjp<3, 2>(p, in, out);
+  if (N == 4 && NC == 2) return compare_vjp<4, 2>(p, in, out);
+  if (N == 3 && NC == 3) return compare_vjp<3, 3>(p, in, out);
   return -2;
 }

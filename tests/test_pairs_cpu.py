@@ -21,6 +21,7 @@ def lib(tmp_path_factory):
                     "-o", out, os.path.join(REPO, "tests", "cpu_model", "pairs_check.cpp")], check=True)
     lib = C.CDLL(out)
     lib.pairs_check.argtypes = [C.POINTER(_abi.GPParams), C.c_int, _abi._dp, _abi._dp]
+    lib.pairs_check_vjp.argtypes = [C.POINTER(_abi.GPParams), _abi._dp, _abi._dp]
     return lib
 
 
@@ -29,6 +30,7 @@ def _params(rng, N, NC):
     p = _abi.GPParams.from_buffer_copy(load_golden(golden_cases()[0])[0].params)
     P, NCM = _abi.P, _abi.NCM
     p.nphases, p.ncomp, p.dx, p.dy, p.dt, p.epsilon = N, NC + 1, 1.0, 2.0, 0.01, 4.0
+    p.tau = 0.3
     p.solve, p.fn_aniso, p.fn_w = 0, int(rng.integers(0, 2)), int(rng.integers(1, 3))
     for a in range(N):
         for b in range(a + 1, N):
@@ -90,3 +92,32 @@ def test_pairs_equal_the_full_loops(lib, shape, form, sym):
                     assert np.array_equal(np.isfinite(r[:, 0]), np.isfinite(r[:, 1]))
                     r = r[np.isfinite(r[:, 0])]
                 assert np.array_equal(r[:, 0], r[:, 1]), (kind, r)
+
+
+@pytest.mark.parametrize("shape", [(2, 1), (3, 2), (4, 2), (3, 3)])
+@pytest.mark.parametrize("sym", [True, False])
+def test_transposed_pairs_match_the_full_loops(lib, shape, sym):
+    """The joined terms of (a, b) and (b, a) are sums of the same products in another order: a few hundred roundings of
+    terms that may cancel, so 1e-11 of the largest entry of the group (stencil and mu, or theta)."""
+    rng = np.random.default_rng(7 + 10 * shape[0] + shape[1])
+    N, NC = shape
+    out, compared = np.zeros(256), 0
+    for _ in range(40):
+        p = _params(rng, N, NC)
+        if not sym:
+            p.rot[_abi.P * 4] += 0.25
+            p.gamma[1] *= 1.5
+        for kind in ("smooth", "sharp", "flat", "wild"):
+            for _ in range(6):
+                cell = np.concatenate([_cell(rng, N, NC, kind), rng.normal(0.0, 1.0, N)])
+                n = lib.pairs_check_vjp(C.byref(p), _abi.dptr(cell), _abi.dptr(out))
+                r = out[:n].reshape(-1, 2)
+                # a non-finite derivative (tau = 0 / 0, a projection over a zero sum) shows in both forms
+                assert np.isfinite(r[:, 0]).all() == np.isfinite(r[:, 1]).all()
+                if not np.isfinite(r).all():
+                    continue
+                compared += 1
+                for part in (r[:9 * N + NC], r[9 * N + NC:]):
+                    scale = np.abs(part).max()
+                    assert np.abs(part[:, 0] - part[:, 1]).max() <= 1e-11 * scale, (kind, part)
+    assert compared > 800
