@@ -156,57 +156,94 @@ __global__ __launch_bounds__(kStatThreads) void k_stats_thermo(const double *__r
  *   energy = [ sum_a h_a psi_a(mu) + eps sum_{a<b} Gamma_ab ac(q_ab)^2 |q_ab|^2 + w(phi) / eps ] dx dy,
  * with q_ab from the centred gradients. Cells are evaluated in the state's precision and accumulated in FP64:
  * a block sum per quantity into partials[i * nblocks + block], folded by k_fold_sum. */
+/* Bound by VALU issue before (one row a thread: every cell's energy terms of all phases and pairs, and three wavefront
+ * reductions per 64 cells: 4096^2 ternary FP64 229 us, 2.9 TB/s). A thread now walks `rows` rows, keeping the rows above and
+ * below in registers (3 loads of phi per cell instead of 5) and reducing once, and a wavefront skips the phases that are
+ * zero on all its five-point stencils, whose terms are zeros: 165 us with the fold. */
 template <int N, int NC, typename R>
 __global__ __launch_bounds__(kBX *kBY) void k_invariants(const Model<R> *__restrict__ mp, const R *__restrict__ phi,
                                                          const R *__restrict__ mu, double *__restrict__ partials,
                                                          int64_t fs, int64_t ps, int64_t yoff, int64_t mx,
-                                                         int64_t my) {
+                                                         int64_t my, int rows) {
   const int64_t y = 3 + (int64_t)blockIdx.x * kBX + threadIdx.x;
-  const int64_t x = 3 + (int64_t)blockIdx.y * kBY + threadIdx.y;
+  const int64_t xa = 3 + ((int64_t)blockIdx.y * kBY + threadIdx.y) * rows;
+  const int64_t xb = xa + rows - 1 < mx + 2 ? xa + rows - 1 : mx + 2;
+  const Model<R> &m = *mp;
+  const double area = (double)m.dx * (double)m.dy;
   double v[NC + 1];
   for (int i = 0; i <= NC; i++) v[i] = 0.0;
-  if (x <= mx + 2 && y <= my + 2) {
-    const Model<R> &m = *mp;
-    const int64_t c = x * ps + y + yoff;
-    const double area = (double)m.dx * (double)m.dy;
-    R ph[N], mv[NC], gxc[N], gyc[N], h[N];
+  if (y <= my + 2 && xa <= xb) {
+    R up[N], ph[N], dn[N];
+    const int64_t c0 = xa * ps + y + yoff;
+#pragma unroll
     for (int a = 0; a < N; a++) {
-      ph[a] = phi[a * fs + c];
-      gxc[a] = (phi[a * fs + c + ps] - phi[a * fs + c - ps]) / (R(2.0) * m.dx);
-      gyc[a] = (phi[a * fs + c + 1] - phi[a * fs + c - 1]) / m.two_dy;
+      up[a] = phi[a * fs + c0 - ps];
+      ph[a] = phi[a * fs + c0];
     }
-    for (int k = 0; k < NC; k++) mv[k] = mu[k * fs + c];
-    for (int a = 0; a < N; a++) h[a] = hphi<N>(ph, a);
-    R e = R(0.0);
-    for (int a = 0; a < N; a++) {
-      R cc[NC], psi = R(0.0);
-      for (int k = 0; k < NC; k++) {
-        cc[k] = c_mu<NC>(m, mv, a, k);
-        v[k] += (double)(h[a] * cc[k]) * area;
-        psi -= mv[k] * cc[k];
+    int64_t c = c0;
+    for (int64_t x = xa; x <= xb; x++, c += ps) {
+      R mv[NC], gxc[N], gyc[N], h[N], lf[N], rt[N];
+#pragma unroll
+      for (int a = 0; a < N; a++) {
+        dn[a] = phi[a * fs + c + ps];
+        lf[a] = phi[a * fs + c - 1];
+        rt[a] = phi[a * fs + c + 1];
       }
-      psi += free_energy<NC>(m, cc, a);
-      e += h[a] * psi;
+#pragma unroll
+      for (int k = 0; k < NC; k++) mv[k] = mu[k * fs + c];
+      bool on[N]; /* wave-uniform: the phase is not zero on some lane's stencil */
+#pragma unroll
+      for (int a = 0; a < N; a++) {
+        on[a] = __any(!(ph[a] == R(0.0) && dn[a] == R(0.0) && up[a] == R(0.0) && rt[a] == R(0.0) && lf[a] == R(0.0)));
+      }
+      R e = R(0.0);
+#pragma unroll
+      for (int a = 0; a < N; a++) {
+        if (!on[a]) continue;
+        /* spacings that are powers of two: the product with the reciprocal is the quotient, exactly */
+        gxc[a] = m.pow2 ? (dn[a] - up[a]) * (R(0.5) * m.inv_dx) : (dn[a] - up[a]) / (R(2.0) * m.dx);
+        gyc[a] = m.pow2 ? (rt[a] - lf[a]) * m.inv_2dy : (rt[a] - lf[a]) / m.two_dy;
+        h[a] = hphi<N>(ph, a);
+        R cc[NC], psi = R(0.0);
+#pragma unroll
+        for (int k = 0; k < NC; k++) {
+          cc[k] = c_mu<NC>(m, mv, a, k);
+          v[k] += (double)(h[a] * cc[k]) * area;
+          psi -= mv[k] * cc[k];
+        }
+        psi += free_energy<NC>(m, cc, a);
+        e += h[a] * psi;
+      }
+      R grad = R(0.0), w = R(0.0);
+      bool some = false;
+#pragma unroll
+      for (int a = 0; a < N; a++)
+#pragma unroll
+        for (int b = a + 1; b < N; b++) {
+          if (!on[a] || !on[b]) continue;
+          some = true;
+          R r[2] = {ph[a] * gxc[b] - ph[b] * gxc[a], ph[a] * gyc[b] - ph[b] * gyc[a]}, q[2];
+          rot2(m.rot[a][b], r, q);
+          const R ac = m.fn_aniso ? aniso_ac(m.dab[a][b], q) : R(1.0);
+          grad += m.gamma[a][b] * ac * ac * qnorm2(q);
+          if (m.fn_w == 1) w += m.w_obst * m.gamma[a][b] * ph[a] * ph[b];
+          else w += R(9.0) * m.gamma[a][b] * ph[a] * ph[a] * ph[b] * ph[b];
+#pragma unroll
+          for (int cc = b + 1; cc < N; cc++) w += m.gamma_abc[a][b][cc] * ph[a] * ph[b] * ph[cc];
+        }
+      if (some) e += m.eps * grad + w / m.eps;
+      v[NC] += (double)e * area;
+#pragma unroll
+      for (int a = 0; a < N; a++) {
+        up[a] = ph[a];
+        ph[a] = dn[a];
+      }
     }
-    R grad = R(0.0), w = R(0.0);
-    for (int a = 0; a < N; a++)
-      for (int b = a + 1; b < N; b++) {
-        R r[2] = {ph[a] * gxc[b] - ph[b] * gxc[a], ph[a] * gyc[b] - ph[b] * gyc[a]}, q[2];
-        rot2(m.rot[a][b], r, q);
-        const R ac = m.fn_aniso ? aniso_ac(m.dab[a][b], q) : R(1.0);
-        grad += m.gamma[a][b] * ac * ac * qnorm2(q);
-        if (m.fn_w == 1) w += m.w_obst * m.gamma[a][b] * ph[a] * ph[b];
-        else w += R(9.0) * m.gamma[a][b] * ph[a] * ph[a] * ph[b] * ph[b];
-        for (int cc = b + 1; cc < N; cc++) w += m.gamma_abc[a][b][cc] * ph[a] * ph[b] * ph[cc];
-      }
-    e += m.eps * grad + w / m.eps;
-    v[NC] = (double)e * area;
   }
   __shared__ double red[NC + 1][kBY];
-  const int lane = threadIdx.x & 63;
   for (int i = 0; i <= NC; i++) {
     const double r = wave_sum(v[i]);
-    if (lane == 0) red[i][threadIdx.y] = r;
+    if (threadIdx.x == 0) red[i][threadIdx.y] = r;
   }
   __syncthreads();
   if (threadIdx.x == 0 && threadIdx.y == 0) {
@@ -235,7 +272,13 @@ static __global__ __launch_bounds__(kStatThreads) void k_fold_sum(const double *
   if (threadIdx.x == 0) out[blockIdx.x] = red[0];
 }
 
-/* solute[NC] and energy of the current state into h->inv_dev */
+/* rows per thread of k_invariants: as many as leave eight wavefronts a SIMD, at most eight (512 x 480 FP64: 8.5 us with one
+ * row, 14 with eight; 2048^2 FP32: 38.8 with one, 28.9 with eight) */
+static int invariant_rows(int64_t mx, int64_t my) {
+  const int64_t waves = (my + kBX - 1) / kBX * mx;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(8, waves / 8192));
+}
+
 /* solute[NC] and energy of a state into out (device, NC + 1 doubles) on `stream`, with the block sums in partials
  * (at least (NC + 1) * invariant_blocks(mesh) doubles): the handle's own state (its plane layout) or a caller's in the
  * reference's plain halo-inclusive layout (fs = rows_x * rows_y, ps = rows_y, yoff = 0) */
@@ -244,9 +287,10 @@ static int launch_invariants_model(gp_handle *h, const void *model, const void *
                                    int64_t ps, int64_t yoff, double *partials, double *out, hipStream_t stream) {
   const int64_t mx = h->p.mesh_x, my = h->p.mesh_y;
   dim3 blk(kBX, kBY);
-  dim3 g2((unsigned)((my + kBX - 1) / kBX), (unsigned)((mx + kBY - 1) / kBY));
+  const int rows = invariant_rows(mx, my);
+  dim3 g2((unsigned)((my + kBX - 1) / kBX), (unsigned)((mx + kBY * rows - 1) / (kBY * rows)));
   hipLaunchKernelGGL((k_invariants<N, NC, R>), g2, blk, 0, stream, (const Model<R> *)model, (const R *)phi,
-                     (const R *)mu, partials, fs, ps, yoff, mx, my);
+                     (const R *)mu, partials, fs, ps, yoff, mx, my, rows);
   hipLaunchKernelGGL(k_fold_sum, dim3(NC + 1), dim3(kStatThreads), 0, stream, (const double *)partials,
                      (int64_t)g2.x * g2.y, out);
   HIPCHK(h, hipGetLastError());
