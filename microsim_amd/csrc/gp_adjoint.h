@@ -58,34 +58,41 @@ __device__ __forceinline__ void theta_flush(const double *th, int nth, double *g
  * plus, when n itself is bulk, gmu_l(n) += sum_k cbar_k(n) cmu_b[k][l], gphi(n) += gphi'(n), gdphi(n) = gphi'(n),
  * and the liquid diffusivities' gradient sum_k Fbar_k(n) sum_f (phi_L(n) + phi_L(e)) / 2 sum_l cmu_L[k][l]
  * (mu_l(e) - mu_l(n)) / d_f^2 (DCs[a][k][l] = sum_q DC[a][k][l][q] = dM/dphi_a). */
-/* Append the cells of this wavefront with `flag` set to list (count: entries so far): one atomic per wavefront,
- * issued by the first flagged lane. */
-__device__ __forceinline__ void list_append(bool flag, int32_t c, int32_t *list, int *count) {
-  const unsigned long long mask = __ballot(flag);
-  if (!mask) return;
-  const int lane = threadIdx.x & 63;
-  const int leader = __ffsll((long long)mask) - 1;
-  int base = 0;
-  if (lane == leader) base = atomicAdd(count, __popcll(mask));
-  base = __shfl(base, leader);
-  if (flag) list[base + __popcll(mask & ((1ull << lane) - 1ull))] = c;
-}
-
-template <int N, int NC>
-__device__ __forceinline__ int bulk_q(const double *phi, const double *dphi, int64_t c, int64_t fs, int64_t ps) {
-  int b = -1;
-  for (int a = 0; a < N; a++)
-    if (b < 0 && phi[a * fs + c] == 1.0) b = a;
-  if (b < 0) return -1;
-  for (int a = 0; a < N - 1; a++) {
-    const double *d = dphi + a * fs + c;
-    if (d[0] != 0.0 || d[ps] != 0.0 || d[-ps] != 0.0 || d[1] != 0.0 || d[-1] != 0.0) return -1;
+/* Append a block's cells with `flag` set to list (count: entries so far), ROWS per thread: one atomic per block of 256
+ * threads. With one per wavefront the grid passes waited for the several thousand that met in one counter (k_adj_codes,
+ * which holds 1024 cells in a block, 1024^2 ternary 39 -> 20 us). */
+template <int ROWS>
+__device__ __forceinline__ void block_append(const bool (&flag)[ROWS], const int32_t (&cell)[ROWS], int32_t *list,
+                                             int *count) {
+  __shared__ int total[4], base;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  unsigned long long mask[ROWS];
+  int n = 0;
+#pragma unroll
+  for (int r = 0; r < ROWS; r++) {
+    mask[r] = __ballot(flag[r]);
+    n += __popcll(mask[r]);
   }
-  return b;
+  if (lane == 0) total[wv] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int all = total[0] + total[1] + total[2] + total[3];
+    base = all ? atomicAdd(count, all) : 0;
+  }
+  __syncthreads();
+  int at = base;
+  for (int w = 0; w < wv; w++) at += total[w];
+#pragma unroll
+  for (int r = 0; r < ROWS; r++) {
+    if (flag[r]) list[at + __popcll(mask[r] & ((1ull << lane) - 1ull))] = cell[r];
+    at += __popcll(mask[r]);
+  }
 }
 
-/* bulk_q from the byte planes of the evaluation state: the pure-phase code (a cell that is not pure falls back to
- * phi) and the candidate flags (delta-phi is read only at candidates; it is +0 at every other cell). Same result. */
+constexpr int kCodeRows = 16; /* rows of 64 cells of a block of the grid passes that list cells */
+
+/* The bulk phase of a cell in stage Q (or -1), from the byte planes of the evaluation state: the pure-phase code (a cell that is not pure falls back to
+ * phi) and the candidate flags (delta-phi is read only at candidates; it is +0 at every other cell). */
 template <int N, int NC>
 __device__ __forceinline__ int bulk_q_codes(const double *phi, const double *dphi, const int8_t *pcode,
                                             const int8_t *cand, int64_t c, int64_t fs, int64_t ps) {
@@ -113,15 +120,16 @@ __global__ __launch_bounds__(256) void k_adj_cbar(const Model<double> *__restric
                                                   const int8_t *__restrict__ cand, int32_t *__restrict__ qlist,
                                                   int *qcount, int64_t fs, int64_t ps, int64_t mx, int64_t my) {
   const int64_t y = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  const Model<double> &m = *mp;
   const int64_t x = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
   const bool valid = x < mx + 6 && y < my + 6;
   const int64_t c = x * ps + y + kYOff;
-  const bool inner = valid && x >= 3 && x <= mx + 2 && y >= 3 && y <= my + 2;
-  const int b = inner ? bulk_q_codes<N, NC>(phi, dphi, pcode, cand, c, fs, ps) : -1;
-  bool dual = false;
+  const int32_t cell[1] = {(int32_t)c};
+  bool dual[1] = {false};
   if (valid) {
+    const bool inner = x >= 3 && x <= mx + 2 && y >= 3 && y <= my + 2;
+    const int b = inner ? bulk_q_codes<N, NC>(phi, dphi, pcode, cand, c, fs, ps) : -1;
     bq[c] = (int8_t)b;
-    const Model<double> &m = *mp;
     for (int k = 0; k < NC; k++) {
       double s = 0.0;
       if (b >= 0)
@@ -129,20 +137,22 @@ __global__ __launch_bounds__(256) void k_adj_cbar(const Model<double> *__restric
       cbar[k * fs + c] = s;
     }
     if (inner && b < 0) {
-      for (int a = 0; a < N; a++) dual = dual || gphi_n[a * fs + c] != 0.0;
-      for (int k = 0; k < NC; k++) dual = dual || gmu_n[k * fs + c] != 0.0;
+      for (int a = 0; a < N; a++) dual[0] = dual[0] || gphi_n[a * fs + c] != 0.0;
+      for (int k = 0; k < NC; k++) dual[0] = dual[0] || gmu_n[k * fs + c] != 0.0;
     }
   }
-  list_append(dual, (int32_t)c, qlist, qcount);
+  block_append(dual, cell, qlist, qcount);
 }
 
-/* the gather above for every cell n of [2, mesh+3]^2: plain stores into gphi / gmu and into gdphi (its value for a
- * bulk n, else 0); every other allocated cell gets zeros in all three, so no clearing pass is needed. The
- * reverse-mode kernels then add the other cells' contributions. */
+/* the gather above for every cell n of [2, mesh+3]^2: plain stores into gphi / gmu and, at candidates, into gdphi (its
+ * value for a bulk n, else 0); every other allocated cell gets zeros in gphi / gmu, so no clearing pass is needed. gdphi is
+ * read at candidates only (k_adj_prev); what it holds elsewhere is not used. The reverse-mode kernels then add the other
+ * cells' contributions. */
 template <int N, int NC>
 __global__ __launch_bounds__(256) void k_adj_bulk(const Model<double> *__restrict__ mp, const double *__restrict__ phi,
                                                   const double *__restrict__ mu, const int8_t *__restrict__ bq,
-                                                  const int8_t *__restrict__ pcode, const double *__restrict__ cbar,
+                                                  const int8_t *__restrict__ pcode, const int8_t *__restrict__ cand,
+                                                  const double *__restrict__ cbar,
                                                   const double *__restrict__ gphi_n, double *__restrict__ gphi,
                                                   double *__restrict__ gmu, double *__restrict__ gdphi, double *gtheta,
                                                   int th0, int64_t fs, int64_t ps, int64_t mx, int64_t my) {
@@ -155,15 +165,13 @@ __global__ __launch_bounds__(256) void k_adj_bulk(const Model<double> *__restric
   const bool alloc = x < mx + 6 && y < my + 6;
   if (alloc && !(x >= 2 && x <= mx + 3 && y >= 2 && y <= my + 3)) {
     const int64_t c = x * ps + y + kYOff;
-    for (int a = 0; a < N; a++) {
-      gphi[a * fs + c] = 0.0;
-      gdphi[a * fs + c] = 0.0;
-    }
+    for (int a = 0; a < N; a++) gphi[a * fs + c] = 0.0;
     for (int k = 0; k < NC; k++) gmu[k * fs + c] = 0.0;
   } else if (alloc) {
     const int64_t c = x * ps + y + kYOff;
     const int b = bq[c]; /* -1 outside the inner cells */
     const int pc = pcode[c];
+    const bool cd = cand[c] != 0;
     double gph[N], gm[NC], cb[NC], mun[NC], phn[N], Mn[NC][NC];
     for (int k = 0; k < NC; k++) {
       cb[k] = cbar[k * fs + c];
@@ -178,11 +186,11 @@ __global__ __launch_bounds__(256) void k_adj_bulk(const Model<double> *__restric
     if (b >= 0) {
       for (int a = 0; a < N; a++) {
         gph[a] = gphi_n[a * fs + c];
-        gdphi[a * fs + c] = gph[a];
+        if (cd) gdphi[a * fs + c] = gph[a];
       }
       for (int l = 0; l < NC; l++)
         for (int k = 0; k < NC; k++) gm[l] += cb[k] * m.cmu[b][k][l];
-    } else {
+    } else if (cd) {
       for (int a = 0; a < N; a++) gdphi[a * fs + c] = 0.0;
     }
     /* M(n); a pure cell's is Mpure, formed with the same operations (bit-identical) */
@@ -289,11 +297,12 @@ __device__ __forceinline__ void scatter_acc(const RevAcc<N, NC> &acc, int64_t c,
   }
 }
 
-/* the stencil of cell c: phi on the 3x3 neighbourhood, mu and (when dphi is given) delta-phi on the 5-point one */
+/* the stencil of cell c: phi on the 3x3 neighbourhood, mu and (when dphi is given) delta-phi on the 5-point one, +0 where
+ * the candidate flag is not set */
 template <int N, int NC>
 __device__ __forceinline__ void gather_stencil(const double *__restrict__ phi, const double *__restrict__ mu,
-                                               const double *__restrict__ dphi, int64_t c, int64_t fs, int64_t ps,
-                                               RegStore<N, NC, double> &rs) {
+                                               const double *__restrict__ dphi, const int8_t *__restrict__ cand,
+                                               int64_t c, int64_t fs, int64_t ps, RegStore<N, NC, double> &rs) {
   const int oi[5] = {0, 1, -1, 0, 0}, oj[5] = {0, 0, 0, 1, -1};
 #pragma unroll
   for (int a = 0; a < N; a++)
@@ -307,7 +316,10 @@ __device__ __forceinline__ void gather_stencil(const double *__restrict__ phi, c
 #pragma unroll
     for (int k = 0; k < NC; k++) rs.u[k][o] = mu[k * fs + co];
 #pragma unroll
-    for (int a = 0; a < N; a++) rs.d[a][o] = dphi ? dphi[a * fs + co] : 0.0;
+    for (int a = 0; a < N; a++) {
+      const double v = dphi ? dphi[a * fs + co] : 0.0;
+      rs.d[a][o] = dphi && cand[co] ? v : 0.0;
+    }
   }
 }
 
@@ -318,7 +330,7 @@ __global__ __launch_bounds__(256) void k_adj_qrev(const Model<double> *__restric
                                                   const double *__restrict__ mu, const double *__restrict__ dphi,
                                                   const double *__restrict__ gphi_n, const double *__restrict__ gmu_n,
                                                   double *gphi, double *gmu, double *gdphi, double *gtheta,
-                                                  const int32_t *__restrict__ list, const int *__restrict__ count,
+                                                  const int8_t *__restrict__ cand, const int32_t *__restrict__ list, const int *__restrict__ count,
                                                   int64_t fs, int64_t ps) {
   constexpr int NTH = kThetaN<N, NC>;
   double th[NTH];
@@ -332,7 +344,7 @@ __global__ __launch_bounds__(256) void k_adj_qrev(const Model<double> *__restric
     for (int a = 0; a < N; a++) go[a] = gphi_n[a * fs + c];
     for (int k = 0; k < NC; k++) gu[k] = gmu_n[k * fs + c];
     RegStore<N, NC, double> rs;
-    gather_stencil<N, NC>(phi, mu, dphi, c, fs, ps, rs);
+    gather_stencil<N, NC>(phi, mu, dphi, cand, c, fs, ps, rs);
     RevAcc<N, NC> acc;
     acc.clear();
     cell_update_vjp<N, NC>(m, RegView<N, NC, double, P2>{&rs, 0, 0}, y, go, gu, acc);
@@ -340,27 +352,6 @@ __global__ __launch_bounds__(256) void k_adj_qrev(const Model<double> *__restric
     for (int t = 0; t < NTH; t++) th[t] += acc.th[t];
   }
   theta_flush<NTH>(th, NTH, gtheta);
-}
-
-/* Stage P transposed runs on the cells of [2, mesh+3]^2 with a nonzero delta-phi adjoint whose 5-point
- * neighbourhood is not purely one phase. (Where it is, every Laplacian of phi is exactly 0 and no phi is
- * negative: phi_delta returns zeros untouched by the projection, with zero derivative.) */
-template <int N>
-__device__ __forceinline__ bool p_candidate(const double *phi, int64_t c, int64_t fs, int64_t ps) {
-  const int64_t o[5] = {0, ps, -ps, 1, -1};
-  int b0 = -2;
-  for (int i = 0; i < 5; i++) {
-    int code = -1, nz = 0;
-    for (int a = 0; a < N; a++) {
-      const double v = phi[a * fs + c + o[i]];
-      if (v == 1.0) code = a;
-      nz += (v != 0.0);
-    }
-    if (nz != 1 || code < 0) return true;
-    if (b0 == -2) b0 = code;
-    else if (code != b0) return true;
-  }
-  return false;
 }
 
 /* Stage B transposed at cell (x, y) for field group f (the ncomp planes at g): a halo cell's adjoint goes to the
@@ -382,46 +373,70 @@ __device__ __forceinline__ void adj_bc_cell(double *g, int ncomp, const Maps &ma
   }
 }
 
-/* the pure-phase code of every allocated cell (pcode) and the list of the P candidates of [2, mesh+3]^2: a cell whose
- * five-point phi is not one pure phase throughout. Every other cell's delta-phi is +0 (no divergence, no clamp):
- * this pass stores +0 at every cell of [2, mesh+3]^2, and k_dlist then forms the candidates' delta-phi
- * (phi_delta, FP64, as the step does) over the list in full wavefronts. */
+/* The pure-phase code of every allocated cell (pcode), the candidate flags and the list of the P candidates of
+ * [2, mesh+3]^2: a cell whose five-point phi is not one pure phase throughout. Every other cell's delta-phi is +0 (every
+ * Laplacian of phi is exactly 0 and no phi is negative, so nothing is clamped), with zero derivative; delta-phi is stored
+ * for the candidates only (k_dlist, over the list in full wavefronts) and read only where the flag is set.
+ * A block takes kCodeRows rows of 64 cells: it forms each code once, and the five-point test reads codes from LDS (every cell
+ * used to form the codes of its whole stencil and to store N zeros: 1024^2 ternary 35 -> 20 us). */
 template <int N, int NC>
-__global__ __launch_bounds__(256) void k_adj_codes(const double *__restrict__ phi, double *__restrict__ dphi,
-                                                   int8_t *__restrict__ pcode, int8_t *__restrict__ cflag,
-                                                   int32_t *__restrict__ plist, int *pcount, int *pclear,
-                                                   double *gfold, Maps maps, int *qclear, int64_t fs, int64_t ps,
-                                                   int64_t mx, int64_t my) {
+__global__ __launch_bounds__(256) void k_adj_codes(const double *__restrict__ phi, int8_t *__restrict__ pcode,
+                                                   int8_t *__restrict__ cflag, int32_t *__restrict__ plist, int *pcount,
+                                                   int *pclear, double *gfold, Maps maps, int *qclear, int64_t fs,
+                                                   int64_t ps, int64_t mx, int64_t my) {
   /* the other P slot (read by the previous transposed step, which ran before this pass) starts the next one at 0,
    * and so does the stage-Q list that the coming transposed step fills */
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
     *pclear = 0;
     *qclear = 0;
   }
-  const int64_t y = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
-  const int64_t x = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
-  const int64_t c = x * ps + y + kYOff;
-  bool cand = false;
-  if (x < mx + 6 && y < my + 6) {
+  constexpr int W = 66;
+  __shared__ int8_t cs[(kCodeRows + 2) * W];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t y0 = (int64_t)blockIdx.x * 64, x0 = (int64_t)blockIdx.y * kCodeRows;
+  const int64_t rx = mx + 6, ry = my + 6;
+  auto code_at = [&](int64_t x, int64_t y) -> int {
+    if (x < 0 || x >= rx || y < 0 || y >= ry) return -1; /* (next to cells that are no candidates) */
+    const int64_t c = x * ps + y + kYOff;
     int code = -1, nz = 0;
+#pragma unroll
     for (int a = 0; a < N; a++) {
       const double v = phi[a * fs + c];
       if (v == 1.0) code = a;
       nz += (v != 0.0);
     }
-    pcode[c] = (int8_t)(nz == 1 ? code : -1);
+    return nz == 1 ? code : -1;
+  };
+  for (int r = wv; r < kCodeRows + 2; r += 4) cs[r * W + lane + 1] = (int8_t)code_at(x0 - 1 + r, y0 + lane);
+  if (threadIdx.x < 2 * (kCodeRows + 2)) {
+    const int r = threadIdx.x >> 1, right = threadIdx.x & 1;
+    cs[r * W + (right ? W - 1 : 0)] = (int8_t)code_at(x0 - 1 + r, right ? y0 + 64 : y0 - 1);
   }
-  if (x >= 2 && x <= mx + 3 && y >= 2 && y <= my + 3) {
-    cand = p_candidate<N>(phi, c, fs, ps);
-    for (int a = 0; a < N; a++) dphi[a * fs + c] = 0.0;
+  __syncthreads();
+  const int64_t y = y0 + lane;
+  bool cand[kCodeRows / 4];
+  int32_t cell[kCodeRows / 4];
+#pragma unroll
+  for (int t = 0; t < kCodeRows / 4; t++) {
+    const int i = wv + 4 * t;
+    const int64_t x = x0 + i, c = x * ps + y + kYOff;
+    cand[t] = false;
+    cell[t] = (int32_t)c;
+    if (x < rx && y < ry) {
+      const int8_t *q = cs + (i + 1) * W + lane + 1;
+      const int8_t k0 = q[0];
+      pcode[c] = k0;
+      if (x >= 2 && x <= mx + 3 && y >= 2 && y <= my + 3)
+        cand[t] = k0 < 0 || q[W] != k0 || q[-W] != k0 || q[1] != k0 || q[-1] != k0;
+      cflag[c] = cand[t] ? 1 : 0;
+      /* stage B of the coming transposed step (its adjoint input gfold), which nothing here reads */
+      if (x < 3 || x > mx + 2 || y < 3 || y > my + 2) {
+        adj_bc_cell(gfold, N, maps, 0, x, y, fs, ps);
+        adj_bc_cell(gfold + (int64_t)N * fs, NC, maps, 1, x, y, fs, ps);
+      }
+    }
   }
-  if (x < mx + 6 && y < my + 6) {
-    cflag[c] = cand ? 1 : 0;
-    /* stage B of the coming transposed step (its adjoint input gfold), which nothing here reads */
-    adj_bc_cell(gfold, N, maps, 0, x, y, fs, ps);
-    adj_bc_cell(gfold + (int64_t)N * fs, NC, maps, 1, x, y, fs, ps);
-  }
-  list_append(cand, (int32_t)c, plist, pcount);
+  block_append(cand, cell, plist, pcount);
 }
 
 /* Stage P transposed by reverse mode (gp_reverse.h: phi_delta_vjp_pairs), one pass per listed candidate (k_adj_codes'
@@ -446,7 +461,7 @@ __global__ __launch_bounds__(256) void k_adj_prev(const Model<double> *__restric
     }
     if (!nz) continue; /* a candidate with no incoming delta-phi adjoint */
     RegStore<N, NC, double> rs;
-    gather_stencil<N, NC>(phi, mu, nullptr, c, fs, ps, rs);
+    gather_stencil<N, NC>(phi, mu, nullptr, nullptr, c, fs, ps, rs);
 #pragma unroll
     for (int k = 0; k < NC; k++) acc.m(k, 0, 0) = 0.0;
     phi_delta_vjp_pairs<N, NC>(m, RegView<N, NC, double, P2>{&rs, 0, 0}, go, acc, [&](int a, int di, int dj, double v) {

@@ -923,6 +923,8 @@ int gp_adjoint_backward(gp_handle *h, const double *gphi_T, const double *gmu_T,
       own.bind(h->cur, S(j));
       if (wide) {
         const double *p64 = (const double *)h->phi[h->cur], *m64 = (const double *)h->mu[h->cur];
+        /* the handle is left with delta-phi of the initial state (a sweep stores it at candidates only) */
+        if (k == 0 && j == 0) HIPCHK(h, hipMemsetAsync(h->dphi, 0, (size_t)h->N * h->fs * sizeof(double), h->stream));
         if ((rc = h->ops->adj_dphi(h, p64, m64, (double *)h->dphi, h->model))) return rc;
         rc = fa(h, p64, m64, (const double *)h->dphi, h->model);
       } else {

@@ -602,12 +602,12 @@ static int adj_step_t(gp_handle *h, const double *phi, const double *mu, const d
                      A->bq, (const int8_t *)A->pcode, (const int8_t *)A->cand, A->qlist, A->counts, fs, h->ps, mx,
                      my);
   hipLaunchKernelGGL((k_adj_bulk<N, NC>), gall, blk, 0, h->stream, md, phi, mu, (const int8_t *)A->bq,
-                     (const int8_t *)A->pcode, (const double *)A->cbar, gn, gc, gc + (size_t)N * fs, A->gdphi, A->gth,
+                     (const int8_t *)A->pcode, (const int8_t *)A->cand, (const double *)A->cbar, gn, gc, gc + (size_t)N * fs, A->gdphi, A->gth,
                      3 * (N * (N - 1) / 2), fs, h->ps, mx, my);
   /* the other cells by reverse mode, one pass per listed cell (grid-stride loops) */
   const dim3 gl(kAdjBlocks);
   hipLaunchKernelGGL((k_adj_qrev<N, NC, P2>), gl, blk, 0, h->stream, md, phi, mu, dphi, gn, gn + (size_t)N * fs, gc,
-                     gc + (size_t)N * fs, A->gdphi, A->gth, (const int32_t *)A->qlist, (const int *)A->counts, fs,
+                     gc + (size_t)N * fs, A->gdphi, A->gth, (const int8_t *)A->cand, (const int32_t *)A->qlist, (const int *)A->counts, fs,
                      h->ps);
   hipLaunchKernelGGL((k_adj_prev<N, NC, P2>), gl, blk, 0, h->stream, md, phi, mu, (const double *)A->gdphi, gc,
                      gc + (size_t)N * fs, A->gth, (const int32_t *)A->plist, (const int *)A->counts + A->pslot, fs,
@@ -626,9 +626,9 @@ static int adj_dphi_t(gp_handle *h, const double *phi, const double *mu, double 
   const int slot = 1 + A->psel, other = 1 + (1 - A->psel);
   A->psel = 1 - A->psel;
   A->pslot = slot;
-  const dim3 gall((unsigned)((h->ry + 63) / 64), (unsigned)((h->rx + 3) / 4));
+  const dim3 gall((unsigned)((h->ry + 63) / 64), (unsigned)((h->rx + kCodeRows - 1) / kCodeRows));
   /* with the codes, stage B of the transposed step that follows (its adjoint input A->g[1]) */
-  hipLaunchKernelGGL((k_adj_codes<N, NC>), gall, dim3(256), 0, h->stream, phi, dphi, A->pcode, A->cand, A->plist,
+  hipLaunchKernelGGL((k_adj_codes<N, NC>), gall, dim3(256), 0, h->stream, phi, A->pcode, A->cand, A->plist,
                      A->counts + slot, A->counts + other, A->g[1], h->maps, A->counts, h->fs, h->ps, mx, my);
   static const int grid = list_grid(h, k_dlist<N, NC, double, P2>);
   hipLaunchKernelGGL((k_dlist<N, NC, double, P2>), dim3(grid), dim3(256), 0, h->stream,
