@@ -99,14 +99,15 @@ __device__ __forceinline__ void bulk_update_ref(const Model<R> &m, int b, const 
 }
 
 /* the mu statistics of one bulk cell: delta-phi is 0 and phi = e_b, so the squared increments of phi add +0 to sums
- * that start at +0 and e_b is finite; the extrema of phi follow from the phases seen (bulk_seen_fold) */
+ * that start at +0 and e_b is finite; the extrema of phi follow from the phases seen (bulk_seen_fold). sum: where the
+ * squared increments of mu add up (st + 3 N + 2 NC, or a lane's second sums) */
 template <int N, int NC, typename R, int NSA>
-__device__ __forceinline__ void bulk_stats(R (&st)[NSA], const R *munew, const R *deltamu) {
+__device__ __forceinline__ void bulk_stats(R (&st)[NSA], R *sum, const R *munew, const R *deltamu) {
 #pragma unroll
   for (int k = 0; k < NC; k++) {
     st[2 * N + k] = fmax(st[2 * N + k], munew[k]);
     st[2 * N + NC + k] = fmin(st[2 * N + NC + k], munew[k]);
-    st[3 * N + 2 * NC + k] += deltamu[k] * deltamu[k];
+    sum[k] += deltamu[k] * deltamu[k];
     if (!isfinite(munew[k])) st[NSA - 1] += R(1.0);
   }
 }
@@ -298,7 +299,7 @@ __device__ __forceinline__ void pad_stats(const Model<R> &m, const R *__restrict
       }
       m0[k] = m1[k];
     }
-    if (out) bulk_stats<N, NC>(st, mn, dm);
+    if (out) bulk_stats<N, NC>(st, st + 3 * N + 2 * NC, mn, dm);
   }
 }
 
@@ -361,6 +362,12 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
 
   R st[NSA];
   if constexpr (STATS) stats_init<N, NC>(st);
+  /* FP32: no sum of squared increments adds more than 16 terms before it is widened, so in long segments the second
+   * column has sums of its own (one sum for both doubled the rounding of rel_change_mu: 0.8e-9 off at 4096^2) */
+  constexpr bool TWO_SUMS = kLeanBulk<R> && 2 * SEG > 16;
+  R odd[NC];
+#pragma unroll
+  for (int k = 0; k < NC; k++) odd[k] = R(0.0);
   unsigned seen = 0u; /* phases of the lane's bulk cells (their phi extrema, folded at the end) */
 
   /* mu rows in a ring of kCellRing register slots, row r in slot (r - xa) mod kCellRing, so that no slot is
@@ -488,8 +495,8 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
             }
           }
           if (STATS) {
-            if (UNI || se) bulk_stats<N, NC>(st, ne, de);
-            if (UNI || so) bulk_stats<N, NC>(st, no, dn);
+            if (UNI || se) bulk_stats<N, NC>(st, st + 3 * N + 2 * NC, ne, de);
+            if (UNI || so) bulk_stats<N, NC>(st, TWO_SUMS ? odd : st + 3 * N + 2 * NC, no, dn);
           }
         };
         R ne[NC], no[NC], de[NC], dn[NC];
@@ -551,8 +558,13 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
     __builtin_amdgcn_s_waitcnt(0x0f70);
     rows(std::true_type{}, TileMasks<N>{});
     if (STATS) {
-      if (!inner) stats_init<N, NC>(st);
-      else seen = 1u << tb;
+      if (!inner) {
+        stats_init<N, NC>(st);
+#pragma unroll
+        for (int k = 0; k < NC; k++) odd[k] = R(0.0);
+      } else {
+        seen = 1u << tb;
+      }
     }
   } else {
 #pragma unroll
@@ -598,10 +610,9 @@ __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, 
   }
   if constexpr (STATS) {
     bulk_seen_fold<N>(st, seen);
-    stats_partials<N, NC, true>(st, partials, pstride, w, nwaves, lane);
+    stats_partials<N, NC, true>(st, partials, pstride, w, nwaves, lane, TWO_SUMS ? odd : nullptr);
   }
 }
-
 
 /* The halo of the new state: each halo cell takes the value of its proxy, as write_images scatters it
  * (apply_boundary_conditions as a gather). Halo row X = hx[k] has the proxy row sx[f][k] when that is an interior row and

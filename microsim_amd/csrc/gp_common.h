@@ -193,9 +193,9 @@ __device__ __forceinline__ float max_val(float a, float b) {
 /* The statistics of a wavefront's lanes (layout of stats_init: extrema of phi and mu first, then the sums), reduced:
  * put(i, value) is called once for every statistic i, by one lane each. Extrema reduce in the statistics' own precision
  * (exact; a minimum as the maximum of the negated values), sums in FP64. PHI_SUMS_ZERO: the squared phi increments are
- * +0 on every lane, and so are their sums. */
+ * +0 on every lane, and so are their sums. more: unless NULL, second sums of the lane's squared mu increments. */
 template <int N, int NC, bool PHI_SUMS_ZERO, int NSA, typename R, class F>
-__device__ __forceinline__ void stats_reduce(const R (&st)[NSA], int lane, F put) {
+__device__ __forceinline__ void stats_reduce(const R (&st)[NSA], int lane, F put, const R *more = nullptr) {
   constexpr int ME = 2 * N + 2 * NC, S0 = PHI_SUMS_ZERO ? 3 * N + 2 * NC : ME, MS = NSA - S0;
   constexpr int QE = (ME + 3) / 4, QS = (MS + 3) / 4;
   const auto is_min = [](int i) { return (i >= N && i < 2 * N) || i >= 2 * N + NC; };
@@ -205,6 +205,10 @@ __device__ __forceinline__ void stats_reduce(const R (&st)[NSA], int lane, F put
   for (int i = 0; i < ME; i++) e[i] = is_min(i) ? -st[i] : st[i];
 #pragma unroll
   for (int i = 0; i < MS; i++) v[i] = (double)st[S0 + i];
+  if (more) {
+#pragma unroll
+    for (int k = 0; k < NC; k++) v[3 * N + 2 * NC - S0 + k] += (double)more[k];
+  }
   wave_reduce(e, te, [](R a, R b) { return max_val(a, b); });
   wave_reduce(v, ts, [](double a, double b) { return a + b; });
   /* lane q of a row stores its j = q value, so that each group leaves in one store */

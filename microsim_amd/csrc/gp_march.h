@@ -201,12 +201,12 @@ __device__ __forceinline__ void stats_add(R (&st)[NSA], const R *pn, const R *dp
 /* wavefront reduction of the per-lane statistics into partials[i * pstride + w] (statistic-major, FP64) */
 template <int N, int NC, bool PHI_SUMS_ZERO = false, int NSA, typename R>
 __device__ __forceinline__ void stats_partials(R (&st)[NSA], double *__restrict__ partials, int64_t pstride,
-                                               int w, int nwaves, int lane) {
+                                               int w, int nwaves, int lane, const R *more = nullptr) {
   /* PHI_SUMS_ZERO: the kernel updates bulk cells only, whose squared phi increments are +0 on every lane */
   if constexpr (NSA > 1) /* (kernels without statistics hold one slot and do not come here) */
     stats_reduce<N, NC, PHI_SUMS_ZERO>(st, lane, [&](int i, double r) {
       if (w < nwaves) partials[(int64_t)i * pstride + w] = r;
-    });
+    }, more);
 }
 
 /* Tiles: wavefront w of a step kernel handles tile w = (strip w % nstrips, segment w / nstrips), i.e. the 60
