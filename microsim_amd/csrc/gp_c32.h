@@ -2,7 +2,7 @@
  * gp_c32.h -- kernels of the compensated FP32 mode (GP_FP32C).
  *
  * State: every mu component is an FP32 plane (hi) plus an int8 plane (q), the value being
- * c32_decode(hi, q) = hi + q ulp32(hi) / 128; every phi component is a pair of FP32 planes (hi, lo), the value being
+ * c32_decode(hi, q) = hi - q ulp32(hi) / 128; every phi component is a pair of FP32 planes (hi, lo), the value being
  * df_decode(hi, lo) = hi + lo (gp_model.h). The step is the cell-classified one of gp_cells.h:
  *   k_cbulk<..., C = true>  bulk cells: the FP32 closed-form increment of mu (from the hi parts), added to the
  *                           decoded value and re-encoded (the increments are not rounded away); phi stays e_b

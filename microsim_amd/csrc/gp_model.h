@@ -974,7 +974,7 @@ GP_HD void mu_update(const Model<R> &m, const V &v, bool smooth, const R *dph, c
 
 /* ------------------------------------------------------------------ compensated FP32 storage (GP_FP32C)
  * mu: a value v is stored as hi = fl32(v) (round to nearest) and an 8-bit signed extension q counting units of
- * ulp32(hi) / 128: v ~= hi + q * 2^(E - 157), E the biased exponent of hi (ulp32(hi) = 2^(E - 150) for a normal
+ * ulp32(hi) / 128 from v to hi: v ~= hi - q * 2^(E - 157), E the biased exponent of hi (ulp32(hi) = 2^(E - 150) for a normal
  * hi). |v - hi| <= ulp32(hi) / 2 gives |q| <= 64. Zero, subnormal and non-finite hi carry q = 0. The pair holds
  * about 31 significant bits, relative to v.
  * phi: the model forms 1 - phi (h, dh/dphi, the anti-trapping s(phi)), which near phi = 1 needs absolute precision
@@ -1011,18 +1011,19 @@ GP_HD double pow2d(int k) {
   return d;
 #endif
 }
-/* Branch-free: q is 0 where hi has no extension, and adds a zero there. The products are by powers of two, hence exact,
- * and the fused forms round once, as the separate sum would. */
+/* Branch-free: where hi has no extension, the sum adds (+0) (-2^k) = -0, which keeps hi and the sign of a zero (q counts
+ * from v to hi for this: the other way round, it would add +0 and turn -0 into +0). The products are by powers of two,
+ * hence exact, and the fused forms round once, as the separate sum would. */
 GP_HD double c32_decode(float hi, int8_t q) {
   const int E = (int)((f32_bits(hi) >> 23) & 0xffu);
-  return __builtin_fma((double)q, pow2d(E - 157), (double)hi);
+  return __builtin_fma((double)q, -pow2d(E - 157), (double)hi);
 }
 GP_HD void c32_encode(double v, float &hi, int8_t &q) {
   hi = (float)v;
   const int E = (int)((f32_bits(hi) >> 23) & 0xffu);
-  /* the count of units, |v - hi| <= ulp32(hi) / 2 and so within +-64, rounded to nearest even by the sum with
+  /* the count of units, |hi - v| <= ulp32(hi) / 2 and so within +-64, rounded to nearest even by the sum with
    * 1.5 2^52, whose low bits then hold the integer */
-  const double s = __builtin_fma(v - (double)hi, pow2d(157 - E), 6755399441055744.0);
+  const double s = __builtin_fma((double)hi - v, pow2d(157 - E), 6755399441055744.0);
   q = (unsigned)(E - 1) < 254u ? (int8_t)f64_low(s) : (int8_t)0;
 }
 GP_HD double df_decode(float hi, float lo) { return (double)hi + (double)lo; }
