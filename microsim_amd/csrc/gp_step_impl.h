@@ -191,10 +191,15 @@ __global__ __launch_bounds__(kBX *kBY) void k_invariants(const Model<R> *__restr
       }
 #pragma unroll
       for (int k = 0; k < NC; k++) mv[k] = mu[k * fs + c];
-      bool on[N]; /* wave-uniform: the phase is not zero on some lane's stencil */
+      /* wave-uniform: the phase is not zero on some lane's stencil, or a mu is not finite or so large that its terms may
+       * overflow (0 times them is not 0: the sums of such a state are those over all phases) */
+      bool on[N], big = false;
+#pragma unroll
+      for (int k = 0; k < NC; k++) big = big || !(fabs(mv[k]) < R(sizeof(R) < 8 ? 1e9 : 1e100));
 #pragma unroll
       for (int a = 0; a < N; a++) {
-        on[a] = __any(!(ph[a] == R(0.0) && dn[a] == R(0.0) && up[a] == R(0.0) && rt[a] == R(0.0) && lf[a] == R(0.0)));
+        const bool zero = ph[a] == R(0.0) && dn[a] == R(0.0) && up[a] == R(0.0) && rt[a] == R(0.0) && lf[a] == R(0.0);
+        on[a] = __any(big || !zero);
       }
       R e = R(0.0);
 #pragma unroll
