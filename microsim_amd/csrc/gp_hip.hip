@@ -883,7 +883,11 @@ int gp_adjoint_backward(gp_handle *h, const double *gphi_T, const double *gmu_T,
       ok = hipMemcpyAsync(A->model64, &m, sizeof m, hipMemcpyHostToDevice, h->stream) == hipSuccess &&
            hipStreamSynchronize(h->stream) == hipSuccess;
     }
-    if (!ok) return gp_fail(h, GP_E_OOM, "adjoint: buffers do not fit in device memory");
+    if (!ok) {
+      w.reset(); /* a further call starts over */
+      A->g[0] = nullptr;
+      return gp_fail(h, GP_E_OOM, "adjoint: buffers do not fit in device memory");
+    }
   }
   int rc;
   if ((rc = rows_to_device(h, PACK_F64, A->g[1], nullptr, nullptr, nullptr, gphi_T, h->N))) return rc;

@@ -20,6 +20,7 @@
 #include <utility>
 #include <vector>
 
+#include "gp_arena.h"
 #include "gp_common.h"
 #include "gp_frame.h"
 #include "gp_hip.h"
@@ -46,7 +47,6 @@ constexpr int kAdjBlocks = GP_ADJ_BLOCKS;   /* grid of the adjoint's reverse-mod
 }  // namespace
 
 struct GpOps;
-class Arena;
 
 struct gp_handle {
   gp_params p;
@@ -107,7 +107,7 @@ struct gp_handle {
   bool pow2;
   int profiling;            /* 0 off, GP_PROFILE_LAUNCHES: events around every launch, GP_PROFILE_CALLS: around
                                every gp_step / gp_smooth call */
-  class Arena *mem;         /* the device buffers above, but those allocated on first use */
+  Arena *mem;               /* the device buffers above, but those allocated on first use */
   struct Adjoint *adj;      /* checkpoints and buffers of the adjoint (gp_adjoint_forward / _backward) */
   const struct GpOps *ops;  /* kernels instantiated for this handle's phases, components and precision */
   std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> prof;
@@ -172,38 +172,6 @@ inline size_t dphi_esize(const gp_handle *h) { return h->precision == GP_FP32 ? 
 /* Device buffers of the adjoint: checkpoints every `every` steps, the recomputed states of one segment, the
  * state adjoints of two consecutive steps, the delta-phi adjoint, the parameter gradient and the cell lists of the
  * reverse-mode stages. */
-/* Device memory cut into pieces of 256-byte alignment: take() the sizes, allocate once, then read the pieces. (One
- * hipMalloc and hipFree per buffer made up a quarter of a short gradient: 45 calls of 35 and 116 us.) */
-class Arena {
- public:
-  ~Arena() {
-    if (base_) (void)hipFree(base_);
-  }
-  /* reserve room for a buffer whose address goes to *p when the arena is allocated */
-  template <typename T>
-  void take(T **p, size_t bytes) {
-    *p = nullptr;
-    pieces_.push_back({(void **)p, size_});
-    size_ += (bytes + 255) & ~(size_t)255;
-  }
-  bool allocate() {
-    if (!base_ && size_ && hipMalloc(&base_, size_) != hipSuccess) {
-      base_ = nullptr;
-      return false;
-    }
-    for (auto &q : pieces_) *q.first = (char *)base_ + q.second;
-    pieces_.clear();
-    return true;
-  }
-  void *base() const { return base_; }
-  size_t size() const { return size_; }
-
- private:
-  std::vector<std::pair<void **, size_t>> pieces_;
-  void *base_ = nullptr;
-  size_t size_ = 0;
-};
-
 struct Adjoint {
   Arena ckpts, work; /* the checkpoints; everything below but scan */
   int64_t nsteps = 0, every = 0;

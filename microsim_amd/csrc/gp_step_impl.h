@@ -679,6 +679,7 @@ static int adj_widen_any(gp_handle *h) {
 static int c32_wide_buffer(gp_handle *h, int i) {
   if (!h->wide[i] && hipMalloc((void **)&h->wide[i], state_elems(h) * sizeof(double)) != hipSuccess) {
     h->wide[i] = nullptr;
+    (void)hipGetLastError(); /* reported here: the next launch's check must not find it */
     return gp_fail(h, GP_E_OOM, "FP64 state copy does not fit in device memory");
   }
   return GP_OK;
