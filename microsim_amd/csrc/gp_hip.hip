@@ -18,6 +18,7 @@
  * (phases, mu fields) in gp_step_impl.h, instantiated once per supported pair by gp_ops.hip.
  * Reference routines replaced: see include/gp_hip.h.
  */
+#include <memory>
 #include <mutex>
 
 #include "gp_internal.h"
@@ -832,9 +833,11 @@ int gp_adjoint_forward(gp_handle *h, int64_t nsteps, int64_t every) {
     return gp_fail(h, GP_E_ARG, "the adjoint covers isothermal runs in a fixed frame");
   if (!h->use_march) return gp_fail(h, GP_E_ARG, "the adjoint records single-pass steps (GP_PATH=twopass is set)");
   if (h->fs > 0x7fffffff) return gp_fail(h, GP_E_ARG, "the adjoint indexes cells with 32 bits: grid too large");
+  /* the handle takes the recording over when it is whole: after a failure there is none, and a backward sweep is refused
+   * (its checkpoints would be null or unwritten) */
   delete h->adj;
-  h->adj = new Adjoint();
-  Adjoint *A = h->adj;
+  h->adj = nullptr;
+  std::unique_ptr<Adjoint> A(new Adjoint());
   if (every <= 0) every = (int64_t)ceil(sqrt((double)(nsteps > 0 ? nsteps : 1)));
   A->nsteps = nsteps;
   A->every = every;
@@ -848,6 +851,7 @@ int gp_adjoint_forward(gp_handle *h, int64_t nsteps, int64_t every) {
     if (!rc) rc = gp_step(h, std::min(every, nsteps - k * every), nullptr);
     if (rc) return rc;
   }
+  h->adj = A.release();
   return GP_OK;
 }
 

@@ -1,0 +1,57 @@
+"""The adjoint after a call that failed: every later call is refused or gives what a fresh handle gives."""
+import os
+import tempfile
+
+import numpy as np
+import pytest
+
+from microsim_amd import _abi, configs, host
+from microsim_amd.solver import GPError, GPSolver
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(mx, my):
+    inp, _, _ = configs.config_ternary(max(mx, my), 0, seed=1234)
+    inp.mesh_x, inp.mesh_y = mx, my
+    fills = [configs.Fill("cylinder", 0, (mx // 2, 9, 5.0)), configs.Fill("cylinder", 1, (mx // 3, my - 14, 6.0))]
+    with tempfile.TemporaryDirectory() as d:
+        configs.write_case(d, inp, fills)
+        return host.load_case(os.path.join(d, "Input.in"), os.path.join(d, "Filling.in"))
+
+
+def _weights(case):
+    rng = np.random.default_rng(3)
+    return rng.standard_normal(case.phi.shape), rng.standard_normal(case.mu.shape)
+
+
+def _same(a, b):
+    """Gradients of one trajectory: sums in the order of atomic additions."""
+    for x, y in zip(a, b):
+        assert np.abs(x - y).max() <= 1e-11 * np.abs(y).max()
+
+
+def test_no_sweep_over_checkpoints_that_do_not_fit():
+    """4096 checkpoints of 2048^2 are more than the card holds: the recording fails, there is none afterwards (the earlier
+    one is gone as well), and a sweep is refused before it launches anything."""
+    case = _case(2048, 2048)
+    w = _weights(case)
+    with GPSolver(case.params) as s:
+        s.upload(case.phi, case.mu)
+        for before in (0, 2):
+            if before:
+                s.adjoint_forward(before, 1)
+            print("[gpu] recording that does not fit, after", before, "steps", flush=True)
+            with pytest.raises(GPError) as e:
+                s.adjoint_forward(4096, 1)
+            assert e.value.code == _abi.GP_E_OOM
+            with pytest.raises(GPError) as e:
+                s.adjoint_backward(*w)
+            assert e.value.code == _abi.GP_E_ARG
+        s.upload(case.phi, case.mu)
+        s.adjoint_forward(3, 2)
+        got = s.adjoint_backward(*w)
+    with GPSolver(case.params) as s:
+        s.upload(case.phi, case.mu)
+        s.adjoint_forward(3, 2)
+        _same(got, s.adjoint_backward(*w))
