@@ -841,7 +841,7 @@ int gp_adjoint_forward(gp_handle *h, int64_t nsteps, int64_t every) {
   if (every <= 0) every = (int64_t)ceil(sqrt((double)(nsteps > 0 ? nsteps : 1)));
   A->nsteps = nsteps;
   A->every = every;
-  const int64_t nck = (nsteps + every - 1) / every;
+  const int64_t nck = nsteps / every + (nsteps % every != 0);
   A->ckpt.resize((size_t)nck);
   for (double *&b : A->ckpt) A->ckpts.take(&b, state_bytes(h));
   if (!A->ckpts.allocate())

@@ -55,3 +55,15 @@ def test_no_sweep_over_checkpoints_that_do_not_fit():
         s.upload(case.phi, case.mu)
         s.adjoint_forward(3, 2)
         _same(got, s.adjoint_backward(*w))
+
+
+def test_one_checkpoint_of_the_largest_interval():
+    case = _case(40, 36)
+    w, got = _weights(case), []
+    for every in (3, (1 << 63) - 1):
+        print("[gpu] checkpoint interval", every, flush=True)
+        with GPSolver(case.params) as s:
+            s.upload(case.phi, case.mu)
+            s.adjoint_forward(3, every)
+            got.append(s.adjoint_backward(*w))
+    _same(*got)
