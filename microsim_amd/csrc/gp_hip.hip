@@ -842,10 +842,17 @@ int gp_adjoint_forward(gp_handle *h, int64_t nsteps, int64_t every) {
   A->nsteps = nsteps;
   A->every = every;
   const int64_t nck = nsteps / every + (nsteps % every != 0);
-  A->ckpt.resize((size_t)nck);
-  for (double *&b : A->ckpt) A->ckpts.take(&b, state_bytes(h));
-  if (!A->ckpts.allocate())
-    return gp_fail(h, GP_E_OOM, "adjoint: %lld checkpoints do not fit in device memory", (long long)nck);
+  /* a count that no device could hold is refused before the host lists its buffers (it would run out of memory first, or
+   * their sizes out of 64 bits) */
+  size_t free_bytes = 0, device_bytes = 0;
+  HIPCHK(h, hipMemGetInfo(&free_bytes, &device_bytes));
+  bool fits = (uint64_t)nck <= device_bytes / state_bytes(h);
+  if (fits) {
+    A->ckpt.resize((size_t)nck);
+    for (double *&b : A->ckpt) A->ckpts.take(&b, state_bytes(h));
+    fits = A->ckpts.allocate();
+  }
+  if (!fits) return gp_fail(h, GP_E_OOM, "adjoint: %lld checkpoints do not fit in device memory", (long long)nck);
   for (int64_t k = 0; k < nck; k++) {
     int rc = state_save(h, A->ckpt[(size_t)k]);
     if (!rc) rc = gp_step(h, std::min(every, nsteps - k * every), nullptr);

@@ -67,3 +67,16 @@ def test_one_checkpoint_of_the_largest_interval():
             s.adjoint_forward(3, every)
             got.append(s.adjoint_backward(*w))
     _same(*got)
+
+
+@pytest.mark.parametrize("nsteps", [1 << 40, (1 << 62) + 1])
+def test_recording_of_more_checkpoints_than_the_host_could_list(nsteps):
+    case = _case(40, 36)
+    with GPSolver(case.params) as s:
+        s.upload(case.phi, case.mu)
+        print("[gpu] recording", nsteps, "checkpoints", flush=True)
+        with pytest.raises(GPError) as e:
+            s.adjoint_forward(nsteps, 1)
+        assert e.value.code == _abi.GP_E_OOM
+        phi, mu = s.download()
+        assert np.array_equal(phi, case.phi) and np.array_equal(mu, case.mu)
