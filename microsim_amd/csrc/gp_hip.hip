@@ -257,7 +257,7 @@ struct StateBinding {
   gp_handle *h;
   void *phi[2], *mu[2];
   int8_t *lo[2];
-  bool direct;
+  bool direct, bound = false;
   explicit StateBinding(gp_handle *hh) : h(hh), direct(hh->use_cells) {
     for (int b = 0; b < 2; b++) {
       phi[b] = h->phi[b];
@@ -277,16 +277,21 @@ struct StateBinding {
   }
   void bind(int b, double *state) {
     const size_t es = esize(h), pb = (size_t)h->N * h->fs * es, mb = (size_t)h->NC * h->fs * es;
+    bound = true;
     h->phi[b] = state;
     h->mu[b] = (char *)state + pb;
     if (h->precision == GP_FP32C) h->lo[b] = (int8_t *)state + pb + mb;
   }
+  /* the handle's own buffers again: the codes and flags of the bound states say nothing of them */
   void release() {
+    if (!bound) return;
+    bound = false;
     for (int b = 0; b < 2; b++) {
       h->phi[b] = phi[b];
       h->mu[b] = mu[b];
       h->lo[b] = lo[b];
     }
+    h->codes_valid = h->flags_valid = h->prev_valid = false;
   }
   ~StateBinding() { release(); }
 };

@@ -80,3 +80,35 @@ def test_recording_of_more_checkpoints_than_the_host_could_list(nsteps):
         assert e.value.code == _abi.GP_E_OOM
         phi, mu = s.download()
         assert np.array_equal(phi, case.phi) and np.array_equal(mu, case.mu)
+
+
+@pytest.mark.parametrize("precision", [_abi.GP_FP64, _abi.GP_FP32C])
+@pytest.mark.parametrize("nsteps", [3, 4, 5])
+def test_steps_after_a_sweep_that_failed(precision, nsteps, monkeypatch):
+    """A sweep that ends in the middle of a segment leaves the handle with one of its own two states, the last of the
+    trajectory or the one before, and steps from there as an undisturbed run does (the cell classes are those of the state
+    that it holds, not those of the segment)."""
+    case = _case(60, 52)
+    wphi, wmu = _weights(case)
+    wmu[0, 30, 20] = np.nan
+    with GPSolver(case.params, precision) as s:
+        s.upload(case.phi, case.mu)
+        s.adjoint_forward(nsteps, nsteps)
+        monkeypatch.setenv("GP_ADJOINT_CHECK", "1000")
+        print("[gpu] sweep that fails,", nsteps, "steps, precision", precision, flush=True)
+        with pytest.raises(GPError) as e:
+            s.adjoint_backward(wphi, wmu)
+        assert e.value.code == _abi.GP_E_NAN
+        held = s.download()
+        s.step(7)
+        got = s.download()
+    equal = lambda u, v: np.array_equal(u[0], v[0]) and np.array_equal(u[1], v[1])
+    for n in (nsteps - 1, nsteps):
+        with GPSolver(case.params, precision) as s:
+            s.upload(case.phi, case.mu)
+            s.step(n)
+            if equal(held, s.download()):
+                s.step(7)
+                assert equal(got, s.download())
+                return
+    raise AssertionError("the state is none of the trajectory's last two")
