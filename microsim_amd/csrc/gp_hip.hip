@@ -258,22 +258,12 @@ struct StateBinding {
   void *phi[2], *mu[2];
   int8_t *lo[2];
   bool direct, bound = false;
-  explicit StateBinding(gp_handle *hh) : h(hh), direct(hh->use_cells) {
+  explicit StateBinding(gp_handle *hh) : h(hh), direct(hh->use_cells && hh->halo_whole) {
     for (int b = 0; b < 2; b++) {
       phi[b] = h->phi[b];
       mu[b] = h->mu[b];
       lo[b] = h->lo[b];
     }
-    const Maps &m = h->maps;
-    for (int f = 0; f < 2; f++)
-      for (int k = 0; k < 6; k++) {
-        int bx = 0, by = 0; /* earlier images of the same row or column: a step writes two (halo_source) */
-        for (int j = 0; j < k; j++) {
-          bx += m.sx[f][j] == m.sx[f][k];
-          by += m.sy[f][j] == m.sy[f][k];
-        }
-        if (bx >= 2 || by >= 2) direct = false;
-      }
   }
   void bind(int b, double *state) {
     const size_t es = esize(h), pb = (size_t)h->N * h->fs * es, mb = (size_t)h->NC * h->fs * es;
@@ -486,6 +476,16 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
     h->maps.hx[k] = (int32_t)hx[k];
     h->maps.hy[k] = (int32_t)hy[k];
   }
+  h->halo_whole = true;
+  for (int f = 0; f < 2; f++)
+    for (int k = 0; k < 6; k++) {
+      int bx = 0, by = 0; /* earlier images of the same row or column: a step writes two (halo_source) */
+      for (int j = 0; j < k; j++) {
+        bx += h->maps.sx[f][j] == h->maps.sx[f][k];
+        by += h->maps.sy[f][j] == h->maps.sy[f][k];
+      }
+      if (bx >= 2 || by >= 2) h->halo_whole = false;
+    }
   if (hipGetDevice(&h->device) != hipSuccess) {
     delete h;
     return gp_fail(nullptr, GP_E_NODEV, "hipGetDevice failed");

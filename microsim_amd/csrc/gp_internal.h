@@ -104,6 +104,7 @@ struct gp_handle {
   bool use_cells;           /* single-pass update by cell class (k_cbulk + k_ilist, default) or by march tiles */
   bool prev_valid;          /* the other buffer holds the state before the last step */
   gpk::Maps maps;
+  bool halo_whole;          /* a step writes every halo cell (else some keep what an upload left there, in each buffer) */
   bool pow2;
   int profiling;            /* 0 off, GP_PROFILE_LAUNCHES: events around every launch, GP_PROFILE_CALLS: around
                                every gp_step / gp_smooth call */

@@ -427,8 +427,12 @@ static int launch_step_p(gp_handle *h, int mode) {
     int8_t *codes_o = h->codes[1 - h->ccur];
     const bool stats = mode == MODE_MARCH_STATS;
     if (!h->codes_valid) {
-      hipLaunchKernelGGL((k_codes<N, R>), dim3((unsigned)((h->ry + 63) / 64), (unsigned)((h->rx + 3) / 4)), dim3(256),
-                         0, h->stream, phi, h->codes[h->ccur], h->fs, h->ps, h->rx, h->ry);
+      /* of the current state, and of the other buffer where it has halo cells that no step writes */
+      const dim3 g((unsigned)((h->ry + 63) / 64), (unsigned)((h->rx + 3) / 4));
+      hipLaunchKernelGGL((k_codes<N, R>), g, dim3(256), 0, h->stream, phi, h->codes[h->ccur], h->fs, h->ps, h->rx, h->ry);
+      if (!h->halo_whole)
+        hipLaunchKernelGGL((k_codes<N, R>), g, dim3(256), 0, h->stream, (const R *)h->phi[1 - h->cur], codes_o, h->fs,
+                           h->ps, h->rx, h->ry);
     }
     if (!h->use_cells) {
       /* delta-phi of the candidate cells, tiles of 64 y-cells by kDTileRows rows over x, y in [2, mesh+3] */
@@ -762,9 +766,14 @@ static int launch_step_c(gp_handle *h, int mode) {
   const int8_t *codes = h->codes[h->ccur];
   int8_t *codes_o = h->codes[1 - h->ccur];
   const bool stats = mode == MODE_MARCH_STATS;
-  if (!h->codes_valid)
-    hipLaunchKernelGGL((k_c32_codes<N>), dim3((unsigned)((h->ry + 63) / 64), (unsigned)((h->rx + 3) / 4)), dim3(256),
-                       0, h->stream, phi, plo, h->codes[h->ccur], fs, h->ps, h->rx, h->ry);
+  if (!h->codes_valid) {
+    /* (as in launch_step_p) */
+    const dim3 g((unsigned)((h->ry + 63) / 64), (unsigned)((h->rx + 3) / 4));
+    hipLaunchKernelGGL((k_c32_codes<N>), g, dim3(256), 0, h->stream, phi, plo, h->codes[h->ccur], fs, h->ps, h->rx, h->ry);
+    if (!h->halo_whole)
+      hipLaunchKernelGGL((k_c32_codes<N>), g, dim3(256), 0, h->stream, (const float *)phi_o, (const float *)plo_o, codes_o,
+                         fs, h->ps, h->rx, h->ry);
+  }
   if (!h->lgrid_d) {
     h->lgrid_d = list_grid(h, k_dlist_c<N, NC, P2>);
     h->lgrid_i = list_grid(h, k_ilist_c<N, NC, P2, true>);
