@@ -42,22 +42,6 @@ __device__ __forceinline__ void theta_flush(const double *th, int nth, double *g
     }
 }
 
-/* ---------------------------------------------------------------- stage Q of bulk cells, in closed form
- *
- * A "bulk" cell c of stage Q has phi_b(c) exactly 1 for some phase (mu_update takes its bulk branch, with the
- * first such b) and no solid-phase delta-phi on itself or its four neighbours (each anti-trapping current of
- * its faces returns +0 before any arithmetic, so carries no derivative). Its stage Q is then
- *   phi_new = phi + dphi,   mu_new = Mu_b(c_b(mu) + dt divflux),
- *   divflux_k = sum over faces f (neighbour e, spacing d_f) of sum_l M_f[k][l] (mu_l(e) - mu_l(c)) / d_f^2,
- *   M_f = (M(c) + M(e)) / 2,   M(x)[k][l] = sum_a sum_q DC[a][k][l][q] phi_a(x),
- * and its transpose is formed here in closed form (exact derivatives, rounded differently from the dual
- * evaluation). With cbar_k(c) = sum_j gmu'_j dMu_j/dc_k and Fbar(c) = dt cbar(c) (zero for other cells), the
- * adjoint of a cell n gathers, over its faces f with neighbour e:
- *   gmu_l(n)  += sum_k (Fbar_k(e) - Fbar_k(n)) M_f[k][l] / d_f^2
- *   gphi_a(n) += sum_k (Fbar_k(n) - Fbar_k(e)) / 2 sum_l DCs[a][k][l] (mu_l(e) - mu_l(n)) / d_f^2
- * plus, when n itself is bulk, gmu_l(n) += sum_k cbar_k(n) cmu_b[k][l], gphi(n) += gphi'(n), gdphi(n) = gphi'(n),
- * and the liquid diffusivities' gradient sum_k Fbar_k(n) sum_f (phi_L(n) + phi_L(e)) / 2 sum_l cmu_L[k][l]
- * (mu_l(e) - mu_l(n)) / d_f^2 (DCs[a][k][l] = sum_q DC[a][k][l][q] = dM/dphi_a). */
 /* Append a block's cells with `flag` set to list (count: entries so far), ROWS per thread: one atomic per block of 256
  * threads. With one per wavefront the grid passes waited for the several thousand that met in one counter (k_adj_codes,
  * which holds 1024 cells in a block, 1024^2 ternary 39 -> 20 us). */
@@ -91,8 +75,26 @@ __device__ __forceinline__ void block_append(const bool (&flag)[ROWS], const int
 
 constexpr int kCodeRows = 16; /* rows of 64 cells of a block of the grid passes that list cells */
 
-/* The bulk phase of a cell in stage Q (or -1), from the byte planes of the evaluation state: the pure-phase code (a cell that is not pure falls back to
- * phi) and the candidate flags (delta-phi is read only at candidates; it is +0 at every other cell). */
+/* ---------------------------------------------------------------- stage Q of bulk cells, in closed form
+ *
+ * A "bulk" cell c of stage Q has phi_b(c) exactly 1 for some phase (mu_update takes its bulk branch, with the
+ * first such b) and no solid-phase delta-phi on itself or its four neighbours (each anti-trapping current of
+ * its faces returns +0 before any arithmetic, so carries no derivative). Its stage Q is then
+ *   phi_new = phi + dphi,   mu_new = Mu_b(c_b(mu) + dt divflux),
+ *   divflux_k = sum over faces f (neighbour e, spacing d_f) of sum_l M_f[k][l] (mu_l(e) - mu_l(c)) / d_f^2,
+ *   M_f = (M(c) + M(e)) / 2,   M(x)[k][l] = sum_a sum_q DC[a][k][l][q] phi_a(x),
+ * and its transpose is formed here in closed form (exact derivatives, rounded differently from the dual
+ * evaluation). With cbar_k(c) = sum_j gmu'_j dMu_j/dc_k and Fbar(c) = dt cbar(c) (zero for other cells), the
+ * adjoint of a cell n gathers, over its faces f with neighbour e:
+ *   gmu_l(n)  += sum_k (Fbar_k(e) - Fbar_k(n)) M_f[k][l] / d_f^2
+ *   gphi_a(n) += sum_k (Fbar_k(n) - Fbar_k(e)) / 2 sum_l DCs[a][k][l] (mu_l(e) - mu_l(n)) / d_f^2
+ * plus, when n itself is bulk, gmu_l(n) += sum_k cbar_k(n) cmu_b[k][l], gphi(n) += gphi'(n), gdphi(n) = gphi'(n),
+ * and the liquid diffusivities' gradient sum_k Fbar_k(n) sum_f (phi_L(n) + phi_L(e)) / 2 sum_l cmu_L[k][l]
+ * (mu_l(e) - mu_l(n)) / d_f^2 (DCs[a][k][l] = sum_q DC[a][k][l][q] = dM/dphi_a). */
+
+/* The bulk phase of a cell in stage Q (or -1), from the byte planes of the evaluation state: the pure-phase code (a cell
+ * that is not pure falls back to phi) and the candidate flags (delta-phi is read only at candidates; it is +0 at every
+ * other cell). */
 template <int N, int NC>
 __device__ __forceinline__ int bulk_q_codes(const double *phi, const double *dphi, const int8_t *pcode,
                                             const int8_t *cand, int64_t c, int64_t fs, int64_t ps) {

@@ -37,7 +37,7 @@ __device__ __forceinline__ void write_images(R *__restrict__ base, int ncomp, co
     }
 }
 
-/* Wavefront reductions of a double over the 64 lanes, returned to every lane. DPP steps keep the data in the
+/* Wavefront sums over the 64 lanes, returned to every lane. DPP steps keep the data in the
  * VALU (no LDS round trips): quad_perm [1,0,3,2] and [2,3,0,1], row_half_mirror and row_mirror reduce each
  * 16-lane row; row_bcast:15 (rows 1, 3) and row_bcast:31 (rows 2, 3) combine the rows, leaving the result in
  * lane 63. Lanes that a masked step does not write receive the operation's identity. */
@@ -57,14 +57,6 @@ __device__ __forceinline__ double lane63(double v) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 template <int CTRL, int ROWMASK>
-__device__ __forceinline__ float mov(float v, float identity) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(__float_as_int(identity), __float_as_int(v), CTRL, ROWMASK, 0xf, false));
-}
-__device__ __forceinline__ float lane63(float v) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-template <int CTRL, int ROWMASK>
 __device__ __forceinline__ int mov(int v, int identity) {
   return __builtin_amdgcn_update_dpp(identity, v, CTRL, ROWMASK, 0xf, false);
 }
@@ -81,24 +73,11 @@ __device__ __forceinline__ T reduce(T v, T identity, Op op) {
 }
 }  // namespace dpp
 
-__device__ __forceinline__ double wave_max(double v) {
-  return dpp::reduce<double>(v, -INFINITY, [](double a, double b) { return fmax(a, b); });
-}
-__device__ __forceinline__ double wave_min(double v) {
-  return dpp::reduce<double>(v, INFINITY, [](double a, double b) { return fmin(a, b); });
-}
 __device__ __forceinline__ double wave_sum(double v) {
   return dpp::reduce<double>(v, 0.0, [](double a, double b) { return a + b; });
 }
 __device__ __forceinline__ int wave_sum(int v) {
   return dpp::reduce<int>(v, 0, [](int a, int b) { return a + b; });
-}
-/* extrema are exact in any precision: FP32 values take the single-register form */
-__device__ __forceinline__ float wave_max(float v) {
-  return dpp::reduce<float>(v, -INFINITY, [](float a, float b) { return fmaxf(a, b); });
-}
-__device__ __forceinline__ float wave_min(float v) {
-  return dpp::reduce<float>(v, INFINITY, [](float a, float b) { return fminf(a, b); });
 }
 
 /* Many wavefront reductions at once. Reduced one by one, M values take M times six steps of two registers; here the

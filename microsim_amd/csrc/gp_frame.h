@@ -27,7 +27,6 @@ namespace gpk {
 
 /* what k_thermo needs of the parameters (FP64, passed by value) */
 struct ThermoParams {
-  int32_t N, NC;
   int32_t hy[6], srcT[6]; /* halo columns and the columns their T copies (itself when that side copies nothing) */
   double Teq;
   double Beq[P][NCM], dBbdT[P][NCM], A[P][NCM][NCM];

@@ -596,8 +596,6 @@ int gp_create(const gp_params *params, int precision, gp_handle **out) {
   if (params->tempgrady) {
     /* the row coefficients' parameters (gp_frame.h k_thermo) */
     ThermoParams &tp = h->tp;
-    tp.N = h->N;
-    tp.NC = h->NC;
     tp.Teq = params->Teq;
     for (int k = 0; k < 6; k++) {
       tp.hy[k] = h->maps.hy[k];

@@ -497,7 +497,8 @@ GP_HD void project_simplex_vjp(const double *phi, const double *divphi, const do
 
 /* ---------------------------------------------------------------- stage P: phi_delta transposed */
 /* gout[N]: the adjoint of the (projected) delta-phi of the centre cell. Adds its transposed Jacobian to acc: phi on
- * the 3x3 stencil, mu at the centre (acc.m(k, 0, 0)), theta. Non-smoothing steps only. */
+ * the 3x3 stencil, mu at the centre (acc.m(k, 0, 0)), theta. Non-smoothing steps only. All ordered pairs: the device runs
+ * the form by present pairs below, which the host checks compare with this one. */
 template <int N, int NC, class V>
 GP_HD void phi_delta_vjp(const Model<double> &m, const V &v, const double *gout, RevAcc<N, NC> &acc) {
   double phi[N], mu[NC > 0 ? NC : 1], divphi[N], lambda[N], out[N];

@@ -15,7 +15,6 @@ namespace gpk {
 
 /* ------------------------------------------------------------------------------------------------ kernels */
 
-/* TG: non-isothermal, th holds the coefficients of every allocated row (gp_frame.h) */
 /* Grid of a list-driven kernel (a grid-stride loop over a list, 256-thread blocks): the blocks the device holds at
  * once, its occupancy times the compute units, at most kListBlocks (the bound the statistics partials are sized
  * for). One batch of resident wavefronts: none waits for a slot while others finish their share of the list. */
@@ -29,6 +28,7 @@ static int list_grid(const gp_handle *h, K kernel) {
   return (int)(g < kListBlocks ? g : kListBlocks);
 }
 
+/* TG: non-isothermal, th holds the coefficients of every allocated row (gp_frame.h) */
 template <int N, int NC, typename R, bool SMOOTH, bool P2, bool TG = false>
 __global__ __launch_bounds__(kBX *kBY) void k_phi(const Model<R> *__restrict__ mp, const R *__restrict__ phi,
                                                   const R *__restrict__ mu, R *__restrict__ dphi, int64_t fs,
