@@ -131,7 +131,11 @@ typedef struct gp_params {
 
 /* Diagnostics. max/min are cumulative from the last gp_upload with the reference's initial values
  * (phi_max 1, phi_min 0, mu_max = mu_min = 1, GPs/solverloop/serialinfo_xy.h:52-59); sums are over interior
- * cells of the last step. solute/energy are evaluated on the state after the last step. */
+ * cells of the last step. solute/energy are evaluated on the state after the last step.
+ * Known defect: on a grid whose mesh_x is not a multiple of four, the default step adds the increments of up to three
+ * invented rows past mesh_x + 2 to rel_change_mu (and their values to mu_max, mu_min and nonfinite) wherever the last
+ * rows of a 60-cell strip are of one phase. Where mu varies along x there, rel_change_mu comes out too large (by 4% on
+ * a 2047 x 1801 run); the state, phi's figures and grids with mesh_x a multiple of four are not touched. */
 typedef struct gp_stats {
   double phi_max[GP_MAXP], phi_min[GP_MAXP];
   double mu_max[GP_MAXNC], mu_min[GP_MAXNC];
@@ -202,8 +206,8 @@ int gp_get_frame(gp_handle *h, int64_t *shift_offset, double *T_rows);
  *   out      device array of NC + 1 doubles: solute[0..NC-1], then energy
  *   stream   hipStream_t to enqueue on, or NULL for the handle's stream
  * The per-block sums go to a device array the library holds for the life of the process, one per GPU, of
- * GP_NOALLOC_SCRATCH_DOUBLES doubles: a grid needs (NC + 1) * ceil(mesh_y/64) * ceil(mesh_x/4) of them (8192^2 with
- * NC = 2 fits), larger grids are rejected with GP_E_ARG. Every call on one GPU shares that array: calls that overlap
+ * GP_NOALLOC_SCRATCH_DOUBLES doubles: a grid may need up to (NC + 1) * ceil(mesh_y/64) * ceil(mesh_x/4) of them (8192^2
+ * with NC = 2 fits), and one with a larger bound is rejected with GP_E_ARG. Every call on one GPU shares that array: calls that overlap
  * in time on one GPU (other streams or handles) race and must be ordered by the caller. The handle's device must be
  * current. */
 #define GP_NOALLOC_SCRATCH_DOUBLES (1 << 20)

@@ -31,8 +31,14 @@ constexpr int kCellOut = 124;  /* output cells of a k_cbulk strip: 64 lanes x 2 
 constexpr int kCellSegMax = 16; /* longest x-segment of k_cbulk (instantiated for 16 and kCellSegMin rows) */
 constexpr int kCellSegMin = 4;
 /* Tiles from which k_cbulk takes the long segments: about one wavefront per SIMD. Below it the rows of a tile in turn are
- * the step's critical path (1024^2 FP64, 576 long tiles: 39 us long, 28 us short); above it the short segments' doubled
- * prologue costs more than it hides (2047 x 1801 FP32, 1920 long tiles: 33 us long, 45 us short). */
+ * the step's critical path; above it the short segments' doubled prologue costs more than it hides. Measured with
+ * statistics, ternary n^2, short / long segments in us (long tiles):
+ *            1024 (576)    1280 (880)    1408 (1056)   1600 (1300)   2048 (2176)   2560 (3360)
+ *   FP32     18.5 / 23.3   24.2 / 24.9   27.3 / 27.2   32.5 / 29.2   41.7 / 35.4   59.4 / 45.3
+ *   FP32C    20.3 / 27.7   26.9 / 29.4   30.5 / 33.1   33.6 / 35.5   43.9 / 43.4   61.9 / 58.0
+ *   FP64     24.1 / 36.2   31.9 / 37.4   32.8 / 41.7   37.9 / 46.5   48.6 / 62.3   68.3 / 83.9
+ * The line is FP32's. FP32C's would lie at about 2000 tiles, and FP64 (161-175 registers with long segments, 140-158 with
+ * short ones) does not reach its own by 2560^2. */
 constexpr int kCellFill = 1024;
 constexpr int kPadOut = 60, kPadSeg = 16; /* tiles of the statistics' padding rows (pad_stats) */
 
@@ -252,11 +258,12 @@ __device__ __forceinline__ TileMasks<N> tile_masks(const unsigned (&cv)[ROWS]) {
   return t;
 }
 
-/* The statistics of the padding rows. The reported extrema and sums of squared increments of mu include, on a grid whose
- * rows are not a multiple of four, up to three rows past mesh+2 for the tiles of kPadOut cells by kPadSeg rows at the
- * grid's end whose cells and neighbours are all of one phase: the updates of row mesh+3 with itself as the row above
- * (and, after the first, below). These terms belong to no cell; they are kept so that the reported figures stay what
- * they were. One wavefront per strip s; returns its partials through st. */
+/* The statistics of the padding rows: a known defect that is kept. The reported extrema and sums of squared increments of
+ * mu include, on a grid whose rows are not a multiple of four, up to three rows past mesh+2 for the tiles of kPadOut cells
+ * by kPadSeg rows at the grid's end whose cells and neighbours are all of one phase: the updates of row mesh+3 with itself
+ * as the row above (and, after the first, below). They came from a step whose uniform tiles ran their padding rows into
+ * the statistics, belong to no cell and can make rel_change_mu a few percent too large (gp_stats); without them the
+ * figure of every such run would change. One wavefront per strip s; returns its partials through st. */
 template <int N, int NC, typename R, bool P2, bool C, int NSA>
 __device__ __forceinline__ void pad_stats(const Model<R> &m, const R *__restrict__ mu, const int8_t *__restrict__ mlo,
                                           const int8_t *__restrict__ codes, int s, int64_t fs, int64_t ps, int64_t mx,
@@ -305,9 +312,10 @@ __device__ __forceinline__ void pad_stats(const Model<R> &m, const R *__restrict
 
 /* Two cells per lane and no LDS: a wavefront has 512 B (FP32) or 1 KiB (FP64) per load in flight, neighbouring lanes meet by
  * one DPP move per two cells, and a strip re-reads 4 of 128 columns where one cell per lane re-reads 4 of 64. Bound by
- * VALU issue and memory together: 4096^2 compensated, 1.2% of the cells at interfaces, 122 us (137 with one cell
- * per lane, codes in LDS) for 411 MB of traffic; FP32 2047 x 1801 33 us (45). On small grids it is one tile's latency:
- * 48 x 40 ternary FP64 13 us with 4-row segments (39 with 16-row ones and the cell-by-cell test), 200^2 binary 12 (30). */
+ * VALU issue and memory together: 4096^2 compensated with statistics 118 us a step over a run (137 with one cell per
+ * lane, codes in LDS), about 480 MB; FP32 2047 x 1801 30 us (45). FP64 at that size gains nothing: 190 us (193), although
+ * it moves 9% less (670 MB): 175 registers leave two wavefronts per SIMD. On small grids it is one tile's latency:
+ * 48 x 40 ternary FP64 13 us with 4-row segments (39 with 16-row ones and the cell-by-cell test), 200^2 binary 9 (30). */
 template <int N, int NC, typename R, bool P2, bool STATS, int SEG, bool C = false>
 __global__ __launch_bounds__(256) void k_cbulk(const Model<R> *__restrict__ mp, const R *__restrict__ mu, const int8_t *__restrict__ codes_in,
              R *__restrict__ phi_o, R *__restrict__ mu_o, int8_t *__restrict__ codes_out,

@@ -8,12 +8,14 @@
  *   dphi (N planes) holds delta-phi when it is asked for.
  * A time step (default, gp_cells.h) classifies cells by the phase codes of the current state: k_cbulk updates the
  * bulk cells (streaming mu; phi stays e_b) and lists the interface cells and the delta-phi candidates (its blocks
- * past the tiles add the candidates of the boundary ring); k_dlist evaluates delta-phi of the listed candidates and k_ilist the
- * general update of the listed interface cells, both with full wavefronts; k_stats folds the statistics when they
- * are asked for. Every kernel writes the halo images of the boundary cells it updates.
+ * past the tiles add the candidates of the boundary ring); k_dlist_step (k_dlist_c in the compensated mode) evaluates
+ * delta-phi of the listed candidates, copies the halo cells whose proxy is a bulk cell, lists the others and folds the
+ * statistics of the step before; k_ilist (k_ilist_c) runs the general update of the listed interface cells and of the
+ * listed halo cells' proxies; k_stats folds the last step of a run with statistics.
  * GP_PATH=march selects the tiled march (gp_march.h: k_dphi, then k_march near an interface and k_bulk on deep
  * tiles); GP_PATH=twopass the two-pass form (k_phi: delta-phi on x,y in [2, mesh+3]; k_mu: currents and update
- * on the interior), which also runs the smoothing steps and recomputes delta-phi for gp_download.
+ * on the interior), which also runs the smoothing steps and recomputes delta-phi for gp_download. The kernels of both
+ * write the halo images of the boundary cells they update.
  * This file holds the C ABI and the host-side handling; the kernels and their launch sequences are templates over
  * (phases, mu fields) in gp_step_impl.h, instantiated once per supported pair by gp_ops.hip.
  * Reference routines replaced: see include/gp_hip.h.
@@ -764,7 +766,8 @@ int gp_get_frame(gp_handle *h, int64_t *shift_offset, double *T_rows) {
 int gp_invariants_noalloc(gp_handle *h, const void *phi, const void *mu, double *out, void *stream) {
   if (!h || !phi || !mu || !out) return h ? gp_fail(h, GP_E_ARG, "null argument") : GP_E_ARG;
   const int64_t mx = h->p.mesh_x, my = h->p.mesh_y;
-  /* the block grid of k_invariants (one block per 64 y-cells by 4 x-rows of the interior) and its block sums */
+  /* the block sums of k_invariants with one row a thread (64 y-cells by 4 x-rows a block); larger grids take several rows
+   * and fewer blocks (invariant_rows), but the bound is the same for every grid */
   const int64_t nblocks = ((my + 63) / 64) * ((mx + 3) / 4);
   const int64_t need = (int64_t)(h->NC + 1) * nblocks;
   if (need > (int64_t)GP_NOALLOC_SCRATCH_DOUBLES)

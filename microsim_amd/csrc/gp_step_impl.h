@@ -156,10 +156,12 @@ __global__ __launch_bounds__(kStatThreads) void k_stats_thermo(const double *__r
  *   energy = [ sum_a h_a psi_a(mu) + eps sum_{a<b} Gamma_ab ac(q_ab)^2 |q_ab|^2 + w(phi) / eps ] dx dy,
  * with q_ab from the centred gradients. Cells are evaluated in the state's precision and accumulated in FP64:
  * a block sum per quantity into partials[i * nblocks + block], folded by k_fold_sum. */
-/* Bound by VALU issue before (one row a thread: every cell's energy terms of all phases and pairs, and three wavefront
- * reductions per 64 cells: 4096^2 ternary FP64 229 us, 2.9 TB/s). A thread now walks `rows` rows, keeping the rows above and
- * below in registers (3 loads of phi per cell instead of 5) and reducing once, and a wavefront skips the phases that are
- * zero on all its five-point stencils, whose terms are zeros: 165 us with the fold. */
+/* A thread walks `rows` rows, keeping the rows above and below in registers (3 loads of phi per cell instead of 5) and
+ * reducing once, and a wavefront skips the phases that are zero on all its five-point stencils, whose terms are zeros.
+ * 4096^2 ternary FP64: 229 us with one row a thread and every phase (VALU issue: energy terms of all phases and pairs,
+ * three reductions per 64 cells), 165 us now. It is bound by memory now: it reads 1.03 GB, at 95% of a large copy's rate,
+ * where the state is 0.67 GB (0.88 GB with one row a thread: the rows that neighbouring blocks share are further apart,
+ * in time and between the XCDs' L2s). */
 template <int N, int NC, typename R>
 __global__ __launch_bounds__(kBX *kBY) void k_invariants(const Model<R> *__restrict__ mp, const R *__restrict__ phi,
                                                          const R *__restrict__ mu, double *__restrict__ partials,
@@ -277,8 +279,10 @@ static __global__ __launch_bounds__(kStatThreads) void k_fold_sum(const double *
   if (threadIdx.x == 0) out[blockIdx.x] = red[0];
 }
 
-/* rows per thread of k_invariants: as many as leave eight wavefronts a SIMD, at most eight (512 x 480 FP64: 8.5 us with one
- * row, 14 with eight; 2048^2 FP32: 38.8 with one, 28.9 with eight) */
+/* rows per thread of k_invariants: as many as leave eight wavefronts a SIMD, at most eight. One, two, four and eight rows,
+ * FP64 us (FP32 alike): 512 x 480 8.1, 8.3, 10.4, 14.8; 1024^2 17.3, 16.6, 16.3, 21.2; 1448^2 29.0, 26.2, 28.4, 28.3;
+ * 2048^2 49.3, 40.9, 46.2, 46.4; 2896^2 113, 93, 90, 88; 4096^2 219, 185, 175, 166. The rule takes 1, 2, 4, 8, 8, 8: within
+ * 13% of the best on each. */
 static int invariant_rows(int64_t mx, int64_t my) {
   const int64_t waves = (my + kBX - 1) / kBX * mx;
   return (int)std::max<int64_t>(1, std::min<int64_t>(8, waves / 8192));
